@@ -48,6 +48,7 @@ struct samp_args {
     int diag;                  // chain on the diagonal (sigma, sigma): p ~ rho(sigma, sigma), both sides flipped
     uint32_t tag;              // random stream: counter word 3 = {0 start, 1 proposal} + 16 tag
     int lpc;                   // lanes per chain (power of two)
+    int rep;                   // FP64: copies of the group in a wave (power of two, lpc rep <= 64), 1 in packed launches
     int restart;               // draw a fresh uniform configuration per chain
     int compat_stale_last_slice;
     uint64_t seed;
@@ -59,7 +60,7 @@ struct samp_args {
     uint32_t* chain_acc;       // chains: accepted proposals per chain, added to (nullable)
     int waves;                 // waves per workgroup, 1, 2 or 4 (0: 4)
 };
-int nq_sampler_lanes_per_chain(const ndm_dims& d);
+int nq_sampler_lanes_per_chain(const ndm_dims& d, bool fp64);
 hipError_t nq_launch_metropolis(const samp_args& a, bool fp64, hipStream_t st);
 
 // ---- S build (k_sbuild.hip)

@@ -1287,7 +1287,7 @@ static nqh_status run_sampler(nqh_ctx* c) {
     a.burn = a.restart ? c->burn : 0;
     a.stored = compat ? c->chain_len - 1 : c->chain_len;
     a.compat_stale_last_slice = compat ? 1 : 0;
-    a.lpc = is_rbm(c) ? 1 : nq_sampler_lanes_per_chain(c->d);
+    a.lpc = is_rbm(c) ? 1 : nq_sampler_lanes_per_chain(c->d, fp64_net(c));
     a.seed = c->seed;
     a.iter = c->iter;
     a.chain_state = P<uint64_t>(c->chain_state);
@@ -2381,7 +2381,8 @@ nq_pk_member pk_describe(nqh_ctx* c, double eps, int kind, double lr) {
     a.burn = a.restart ? c->burn : 0;
     a.stored = compat ? c->chain_len - 1 : c->chain_len;
     a.compat_stale_last_slice = compat ? 1 : 0;
-    a.lpc = nq_sampler_lanes_per_chain(d);
+    a.lpc = nq_sampler_lanes_per_chain(d, fp64_net(c));
+    a.rep = 1;
     a.seed = c->seed;
     a.iter = c->iter;
     a.iter_dev = P<uint32_t>(c->iter_dev);
@@ -3061,7 +3062,7 @@ nqh_status nqh_observable(nqh_ctx* c, const nqh_optable* op, int64_t chains, int
     a.restart = 1;
     a.diag = 1;
     a.tag = 1;
-    a.lpc = is_rbm(c) ? 1 : nq_sampler_lanes_per_chain(c->d);
+    a.lpc = is_rbm(c) ? 1 : nq_sampler_lanes_per_chain(c->d, fp64_net(c));
     a.seed = c->seed;
     a.iter = c->iter;
     a.chain_state = P<uint64_t>(c->obs_state);
