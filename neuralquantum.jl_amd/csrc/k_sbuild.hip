@@ -5,14 +5,18 @@
 // B = [Im Pi | Im mu]; S in P order is A^T A embedded at [0, nA) plus B^T B
 // embedded at [nlam, np) (the lambda-mu block is identically zero).
 //
-// FP64 / FP32 (k_gram): each workgroup computes one 64x64 upper-triangular
-// tile of a Gram block; the 4 waves own 32x32 quadrants of 2x2 MFMA 16x16
-// tiles.  Columns are centred (Y - mean) while staging through LDS, which is
-// what the reference's O - Obar does (BaseIterativeSampler.jl:19-26).
+// FP64 / FP32 (k_gram_part): each workgroup computes one 64x64 upper-triangular
+// tile of a Gram block over one chunk of the samples; the 4 waves own 32x32
+// quadrants of 2x2 MFMA 16x16 tiles.  Columns are centred (Y - mean) while
+// staging through LDS, which is what the reference's O - Obar does
+// (BaseIterativeSampler.jl:19-26).
 //   FP64: v_mfma_f64_16x16x4f64     FP32: v_mfma_f32_16x16x4f32
 // BF16 (k_center_t + k_gram_bf16_part + k_gram_finish): a centred, transposed
 // BF16 copy, then a split-K Gram of 128x128 tiles with
-// v_mfma_f32_16x16x32_bf16 (FP32 accumulation) and one pass that writes S.
+// v_mfma_f32_16x16x32_bf16 (FP32 accumulation).
+// In every precision k_gram_finish then sums the chunks and writes S.
+#include <algorithm>
+
 #include "nq_kernels.h"
 
 namespace {
@@ -23,7 +27,7 @@ typedef __bf16 bf8 __attribute__((ext_vector_type(8)));
 
 template <int MODE> struct gram_traits;
 template <> struct gram_traits<NQ_GRAM_F64> { typedef double st; typedef d4 acc; static constexpr int KC = 16; };
-template <> struct gram_traits<NQ_GRAM_F32> { typedef float st; typedef f4 acc; static constexpr int KC = 16; };
+template <> struct gram_traits<NQ_GRAM_F32> { typedef float st; typedef f4 acc; static constexpr int KC = 32; };
 
 __device__ __forceinline__ void tri_decode(int b, int* I, int* J) {
     int j = (int)((sqrtf(8.0f * (float)b + 1.0f) - 1.0f) * 0.5f);
@@ -33,21 +37,33 @@ __device__ __forceinline__ void tri_decode(int b, int* I, int* J) {
     *I = b - j * (j + 1) / 2;
 }
 
+// FP64 / FP32 tile `tile` (block A: Y columns [0, nA), TA tiles a side; then block B: the next nB)
+// over samples [split kchunk, (split + 1) kchunk): the accumulators, row-major 64 x 64, to `part`.
+// Bound by the matrix cores: 16 products of 64 (FP64) or 32 (FP32) cycles per wave and k-step against
+// 16 KB (8 KB) loaded per workgroup.  One workgroup per tile over all samples, one launch per block,
+// left the chip between a half and a seventh full (2 Ns n^2 / 2 flop in two launches of 351 tiles at
+// the 4x4 XYZ shapes, of 120 at 12 sites); the chunks fill it, and with chunk = workgroup mod 8 each
+// XCD's L2 holds one chunk's rows for all its tiles, so Y comes from HBM once.  Four workgroups per CU
+// (32 KB of LDS, 64 x 64 without padding: element (k, c) at column c ^ 16 (k mod 4), so that the four
+// sample rows of an operand read fall on different banks) hide the loads and the barrier.
 template <int MODE, typename YT>
-__device__ __forceinline__ void gram_body(const gram_args& a, int bx) {
+__device__ __forceinline__ void gram_part_body(const YT* Yall, int64_t Ns, int ldy, const double* mu, int nA, int TA,
+                                               int nB, int64_t kchunk, int tiles, void* partv, int tile, int split) {
     typedef typename gram_traits<MODE>::st ST;
     typedef typename gram_traits<MODE>::acc AT;
     constexpr int KC = gram_traits<MODE>::KC;
-    constexpr int PITCH = 65;                 // [k][64 + 1]: k-major, rows contiguous
-    constexpr int TILE = KC * PITCH;
+    constexpr int TILE = KC * 64;
     constexpr int NJ = KC / 4;                // sample rows staged per thread and k-step
     __shared__ ST As[2 * TILE];               // double-buffered: one barrier per k-step
     __shared__ ST Bs[2 * TILE];
 
+    const int tilesA = TA * (TA + 1) / 2;
+    const bool second = tile >= tilesA;
+    const int c0 = second ? nA : 0, n = second ? nB : nA;
     int I, J;
-    tri_decode(bx, &I, &J);
-    const int r0 = I * 64, q0 = J * 64;
-    const YT* Y = reinterpret_cast<const YT*>(a.Y);
+    tri_decode(second ? tile - tilesA : tile, &I, &J);
+    const int64_t kbeg = (int64_t)split * kchunk;
+    const int len = (int)((kbeg + kchunk < Ns ? kbeg + kchunk : Ns) - kbeg);
     const int tid = threadIdx.x;
     const int lane = tid & 63, wave = tid >> 6;
     const int wr = wave >> 1, wc = wave & 1;
@@ -56,84 +72,114 @@ __device__ __forceinline__ void gram_body(const gram_args& a, int bx) {
 #pragma unroll
     for (int m = 0; m < 2; ++m)
 #pragma unroll
-        for (int n = 0; n < 2; ++n)
+        for (int q = 0; q < 2; ++q)
 #pragma unroll
-            for (int v = 0; v < 4; ++v) acc[m][n][v] = 0;
+            for (int v = 0; v < 4; ++v) acc[m][q][v] = 0;
 
-    // this thread's staging column and its mean
-    const int lc = tid & 63;
-    const int ca = r0 + lc, cb = q0 + lc;
-    const bool va = ca < a.n, vb = cb < a.n;
-    const double mua = (va && a.mu) ? a.mu[a.c0 + ca] : 0.0;
-    const double mub = (vb && a.mu) ? a.mu[a.c0 + cb] : 0.0;
-    double ya[NJ], yb[NJ];
-    // unconditional loads from clamped addresses (one k-step ahead), centred
-    // and selected when stored
-    auto load = [&](int64_t k0) {
+    // this thread's staging columns and their means; columns past the block stand on column 0: they
+    // only reach accumulator rows and columns that nothing reads
+    const int lc = tid & 63, lr = tid >> 6;
+    const int xa = I * 64 + lc < n ? I * 64 + lc : 0, xb = J * 64 + lc < n ? J * 64 + lc : 0;
+    const double mua = mu ? mu[c0 + xa] : 0.0, mub = mu ? mu[c0 + xb] : 0.0;
+    // FP32 rows centred in FP32 by the mean as a sum of two floats: as exact as the difference taken in
+    // FP64 and rounded, without two conversions per element
+    const float mha = (float)mua, mla = (float)(mua - mha), mhb = (float)mub, mlb = (float)(mub - mhb);
+    auto centre = [](YT y, double m, float mh, float ml) -> ST {
+        if constexpr (MODE == NQ_GRAM_F32 && sizeof(YT) == 4) return ((float)y - mh) - ml;
+        else return (ST)((double)y - m);
+    };
+    const YT* pa = Yall + (kbeg + lr) * (int64_t)ldy + c0 + xa;
+    const YT* pb = Yall + (kbeg + lr) * (int64_t)ldy + c0 + xb;
+    YT ya[NJ], yb[NJ];
+    const int sc = lc ^ (16 * lr);            // lr = sample row mod 4
+    // whole k-steps of KC samples, loaded one step ahead of their staging
+    auto load = [&](int step) {
 #pragma unroll
         for (int j = 0; j < NJ; ++j) {
-            const int64_t s = k0 + (tid >> 6) + 4 * j;
-            const YT* row = Y + (s < a.Ns ? s : a.Ns - 1) * (int64_t)a.ldy + a.c0;
-            ya[j] = (double)row[va ? ca : 0];
-            yb[j] = (double)row[vb ? cb : 0];
+            const int64_t o = (int64_t)(step * KC + 4 * j) * ldy;
+            ya[j] = pa[o];
+            yb[j] = pb[o];
         }
     };
-    auto store = [&](int buf, int64_t k0) {
+    auto store = [&](int buf) {
 #pragma unroll
         for (int j = 0; j < NJ; ++j) {
-            const int kk = (tid >> 6) + 4 * j;
-            const int64_t s = k0 + kk;
-            As[buf * TILE + kk * PITCH + lc] = (ST)((s < a.Ns && va) ? ya[j] - mua : 0.0);
-            Bs[buf * TILE + kk * PITCH + lc] = (ST)((s < a.Ns && vb) ? yb[j] - mub : 0.0);
+            As[buf * TILE + (lr + 4 * j) * 64 + sc] = centre(ya[j], mua, mha, mla);
+            Bs[buf * TILE + (lr + 4 * j) * 64 + sc] = centre(yb[j], mub, mhb, mlb);
         }
     };
-    const int64_t nsteps = (a.Ns + KC - 1) / KC;
-    load(0);
-    store(0, 0);
-    if (nsteps > 1) load(KC);
-    __syncthreads();
     const int li = lane & 15, lk = lane >> 4;
-    for (int64_t i = 0; i < nsteps; ++i) {
-        if (i + 1 < nsteps) store((int)((i + 1) & 1), (i + 1) * KC);
-        if (i + 2 < nsteps) load((i + 2) * KC);
-        const ST* A = As + (i & 1) * TILE;
-        const ST* B = Bs + (i & 1) * TILE;
+    int fa[2], fb[2];                         // operand offsets of this lane within four sample rows
+#pragma unroll
+    for (int m = 0; m < 2; ++m) {
+        fa[m] = lk * 64 + ((wr * 32 + m * 16 + li) ^ (16 * lk));
+        fb[m] = lk * 64 + ((wc * 32 + m * 16 + li) ^ (16 * lk));
+    }
+    auto multiply = [&](int buf) {
 #pragma unroll
         for (int k = 0; k < KC; k += 4) {
             ST av[2], bv[2];
 #pragma unroll
-            for (int m = 0; m < 2; ++m) av[m] = A[(k + lk) * PITCH + wr * 32 + m * 16 + li];
+            for (int m = 0; m < 2; ++m) av[m] = As[buf * TILE + k * 64 + fa[m]];
 #pragma unroll
-            for (int n = 0; n < 2; ++n) bv[n] = B[(k + lk) * PITCH + wc * 32 + n * 16 + li];
+            for (int q = 0; q < 2; ++q) bv[q] = Bs[buf * TILE + k * 64 + fb[q]];
 #pragma unroll
             for (int m = 0; m < 2; ++m)
 #pragma unroll
-                for (int n = 0; n < 2; ++n) {
+                for (int q = 0; q < 2; ++q) {
                     if constexpr (MODE == NQ_GRAM_F64)
-                        acc[m][n] = __builtin_amdgcn_mfma_f64_16x16x4f64(av[m], bv[n], acc[m][n], 0, 0, 0);
+                        acc[m][q] = __builtin_amdgcn_mfma_f64_16x16x4f64(av[m], bv[q], acc[m][q], 0, 0, 0);
                     else
-                        acc[m][n] = __builtin_amdgcn_mfma_f32_16x16x4f32(av[m], bv[n], acc[m][n], 0, 0, 0);
+                        acc[m][q] = __builtin_amdgcn_mfma_f32_16x16x4f32(av[m], bv[q], acc[m][q], 0, 0, 0);
                 }
         }
+    };
+    // the last, partial k-step first (zeros past its samples), then the whole ones
+    const int nsteps = len / KC, rest = len - nsteps * KC;
+    if (rest > 0) {
+#pragma unroll
+        for (int j = 0; j < NJ; ++j) {
+            const int r = lr + 4 * j;
+            const bool in = r < rest;
+            const int64_t o = in ? (int64_t)(nsteps * KC + 4 * j) * ldy : -(int64_t)lr * ldy;
+            As[TILE + r * 64 + sc] = in ? centre(pa[o], mua, mha, mla) : ST(0);
+            Bs[TILE + r * 64 + sc] = in ? centre(pb[o], mub, mhb, mlb) : ST(0);
+        }
+    }
+    if (nsteps > 0) {
+        load(0);
+        store(0);
+        load(nsteps > 1 ? 1 : 0);
+    }
+    __syncthreads();
+    if (rest > 0) {
+        multiply(1);
         __syncthreads();
     }
+    // step i in buffer i & 1; two per round so that the buffers are immediate offsets
+    int i = 0;
+    for (; i + 2 <= nsteps; i += 2) {
+        store(1);
+        load(i + 2 < nsteps ? i + 2 : nsteps - 1);
+        multiply(0);
+        __syncthreads();
+        store(0);
+        load(i + 3 < nsteps ? i + 3 : nsteps - 1);
+        multiply(1);
+        __syncthreads();
+    }
+    if (i < nsteps) multiply(0);
 
     // D[i][j] of a 16x16 tile, j = lane % 16:  f32: i = 4 (lane / 16) + v;  f64: i = lane / 16 + 4 v
-    const int lj = lane & 15, lg = lane >> 4;
+    ST* part = reinterpret_cast<ST*>(partv) + ((int64_t)split * tiles + tile) * (64 * 64);
 #pragma unroll
     for (int m = 0; m < 2; ++m)
 #pragma unroll
-        for (int n = 0; n < 2; ++n)
+        for (int q = 0; q < 2; ++q)
 #pragma unroll
             for (int v = 0; v < 4; ++v) {
-                const int ti = (MODE == NQ_GRAM_F64) ? lg + 4 * v : 4 * lg + v;
-                const int r = r0 + wr * 32 + m * 16 + ti;
-                const int c = q0 + wc * 32 + n * 16 + lj;
-                if (r < a.n && c < a.n) {
-                    const double val = a.scale * (double)acc[m][n][v];
-                    a.S[(int64_t)(a.o + r) + (int64_t)(a.o + c) * a.lds] += val;
-                    if (I != J) a.S[(int64_t)(a.o + c) + (int64_t)(a.o + r) * a.lds] += val;
-                }
+                const int ti = (MODE == NQ_GRAM_F64) ? lk + 4 * v : 4 * lk + v;
+                part[(wr * 32 + m * 16 + ti) * 64 + wc * 32 + q * 16 + li] = acc[m][q][v];
             }
 }
 
@@ -283,16 +329,18 @@ __device__ __forceinline__ void gram_bf16_part_body(const __bf16* Yt, int64_t ns
 // sum over the chunks of element (rr, cc) of the Gram block whose tiles start at toff
 // offset of element (rr, cc) of a Gram block in split 0 of the partials
 // (upper tiles only: the lower half is read transposed)
+template <int TS>
 __device__ __forceinline__ int gram_part_off(int toff, int rr, int cc) {
-    int I = rr >> 7, J = cc >> 7, x = rr & 127, y = cc & 127;
+    int I = rr / TS, J = cc / TS, x = rr % TS, y = cc % TS;
     if (I > J) {
         const int t0 = I; I = J; J = t0;
         const int t1 = x; x = y; y = t1;
     }
-    return (toff + J * (J + 1) / 2 + I) * (128 * 128) + x * 128 + y;
+    return (toff + J * (J + 1) / 2 + I) * (TS * TS) + x * TS + y;
 }
 
-__device__ __forceinline__ void gram_finish_body(const float* part, int splits, int tiles, int nA, int TA, int nB,
+template <typename PT, int TS>
+__device__ __forceinline__ void gram_finish_body(const PT* part, int splits, int tiles, int nA, int TA, int nB,
                                                  int offB, double scale, double* S, int np, int lds, int bx) {
     __shared__ double T[64][65];
     int bi, bj;
@@ -307,18 +355,18 @@ __device__ __forceinline__ void gram_finish_body(const float* part, int splits, 
     for (int m = 0; m < 16; ++m) {
         const int r = bi * 64 + x0 + 4 * m;
         const bool in = r < np && c < np;
-        oa[m] = (in && r < nA && c < nA) ? gram_part_off(0, r, c) : -1;
+        oa[m] = (in && r < nA && c < nA) ? gram_part_off<TS>(0, r, c) : -1;
         ob[m] = (in && nB > 0 && r >= offB && c >= offB && r - offB < nB && c - offB < nB)
-                    ? gram_part_off(tilesA, r - offB, c - offB)
+                    ? gram_part_off<TS>(tilesA, r - offB, c - offB)
                     : -1;
     }
-    const int64_t stride = (int64_t)tiles * (128 * 128);
+    const int64_t stride = (int64_t)tiles * (TS * TS);
     double sa[16], sb[16];
 #pragma unroll
     for (int m = 0; m < 16; ++m) sa[m] = sb[m] = 0.0;
     for (int sp = 0; sp < splits; ++sp) {
-        const float* p = part + sp * stride;
-        float la[16], lb[16];   // unconditional loads (offset 0 stands in), selected after
+        const PT* p = part + sp * stride;
+        PT la[16], lb[16];   // unconditional loads (offset 0 stands in), selected after
 #pragma unroll
         for (int m = 0; m < 16; ++m) {
             la[m] = p[oa[m] >= 0 ? oa[m] : 0];
@@ -394,9 +442,12 @@ __device__ __forceinline__ void colsum_finish_body(const double* part, int chunk
     if (g == 0 && c < R) mu[c] = ((red[0][x] + red[1][x]) + (red[2][x] + red[3][x])) * scale;
 }
 
+// workgroup b: chunk b mod splits of tile b / splits
 template <int MODE, typename YT>
-__global__ __launch_bounds__(256) void k_gram(gram_args a) {
-    gram_body<MODE, YT>(a, blockIdx.x);
+__global__ __launch_bounds__(256) void k_gram_part(const YT* Y, int64_t Ns, int ldy, const double* mu, int nA, int TA,
+                                                   int nB, int64_t kchunk, int tiles, int splits, void* part) {
+    gram_part_body<MODE, YT>(Y, Ns, ldy, mu, nA, TA, nB, kchunk, tiles, part, blockIdx.x / splits,
+                             blockIdx.x % splits);
 }
 
 template <typename YT>
@@ -410,9 +461,10 @@ __global__ __launch_bounds__(256) void k_gram_bf16_part(const __bf16* Yt, int64_
     gram_bf16_part_body(Yt, nsp, nA, TA, nB, kchunk, tiles, part, blockIdx.x, blockIdx.y);
 }
 
-__global__ __launch_bounds__(256) void k_gram_finish(const float* part, int splits, int tiles, int nA, int TA, int nB,
+template <typename PT, int TS>
+__global__ __launch_bounds__(256) void k_gram_finish(const PT* part, int splits, int tiles, int nA, int TA, int nB,
                                                      int offB, double scale, double* S, int np, int lds) {
-    gram_finish_body(part, splits, tiles, nA, TA, nB, offB, scale, S, np, lds, blockIdx.x);
+    gram_finish_body<PT, TS>(part, splits, tiles, nA, TA, nB, offB, scale, S, np, lds, blockIdx.x);
 }
 
 template <typename YT>
@@ -428,28 +480,12 @@ __global__ __launch_bounds__(256) void k_colsum_finish(const double* part, int c
 // ---- packed forms (block records and descriptors as in nq_pk_member)
 __device__ __forceinline__ const nq_pk_member& pk_member(const nq_pk_member* M, uint2 b) { return M[b.x & 0xffff]; }
 
-// the FP64 / FP32 Gram block `which` of a member (build_s: block A then B, adding into S)
-__host__ __device__ inline gram_args pk_gram_args(const nq_pk_member& m, int which) {
-    gram_args g{};
-    g.Y = m.Y;
-    g.y_fp64 = m.fp64;
-    g.Ns = m.Ns;
-    g.ldy = m.R;
-    g.mu = m.mu;
-    g.S = m.S;
-    g.lds = m.ldS;
-    g.scale = 1.0 / (double)m.Ns;
-    g.c0 = which == 0 ? 0 : m.nA;
-    g.n = which == 0 ? m.nA : m.nB;
-    g.o = which == 0 ? 0 : m.offB;
-    return g;
-}
-
 template <int MODE, typename YT>
-__global__ __launch_bounds__(256) void k_gram_pk(const nq_pk_member* M, const uint2* blk, int which) {
+__global__ __launch_bounds__(256) void k_gram_part_pk(const nq_pk_member* M, const uint2* blk) {
     const uint2 b = blk[blockIdx.x];
-    const gram_args a = pk_gram_args(pk_member(M, b), which);
-    gram_body<MODE, YT>(a, b.y & 0xffff);
+    const nq_pk_member& m = pk_member(M, b);
+    gram_part_body<MODE, YT>((const YT*)m.Y, m.Ns, m.R, m.mu, m.nA, m.TA, m.nB, m.kchunk, m.tiles, m.gpart,
+                             b.y & 0xffff, b.y >> 16);
 }
 
 template <typename YT>
@@ -475,36 +511,47 @@ __global__ __launch_bounds__(256) void k_center_t_pk(const nq_pk_member* M, cons
 __global__ __launch_bounds__(256) void k_gram_bf16_part_pk(const nq_pk_member* M, const uint2* blk) {
     const uint2 b = blk[blockIdx.x];
     const nq_pk_member& m = pk_member(M, b);
-    gram_bf16_part_body(m.Yt, m.nsp, m.nA, m.TA, m.nB, m.kchunk, m.tiles, m.gpart, b.y & 0xffff, b.y >> 16);
+    gram_bf16_part_body(m.Yt, m.nsp, m.nA, m.TA, m.nB, m.kchunk, m.tiles, (float*)m.gpart, b.y & 0xffff, b.y >> 16);
 }
 
+template <typename PT, int TS>
 __global__ __launch_bounds__(256) void k_gram_finish_pk(const nq_pk_member* M, const uint2* blk) {
     const uint2 b = blk[blockIdx.x];
     const nq_pk_member& m = pk_member(M, b);
-    gram_finish_body(m.gpart, m.splits, m.tiles, m.nA, m.TA, m.nB, m.offB, 1.0 / (double)m.Ns, m.S, m.np, m.ldS,
+    gram_finish_body<PT, TS>((const PT*)m.gpart, m.splits, m.tiles, m.nA, m.TA, m.nB, m.offB, 1.0 / (double)m.Ns, m.S, m.np, m.ldS,
                      b.y & 0xffff);
 }
 
-template <int MODE>
-hipError_t launch_mode(const gram_args& a, hipStream_t st) {
-    const int T = (a.n + 63) / 64;
-    const int blocks = T * (T + 1) / 2;
-    if (blocks == 0) return hipSuccess;
-    if (a.y_fp64)
-        hipLaunchKernelGGL((k_gram<MODE, double>), dim3(blocks), dim3(256), 0, st, a);
-    else
-        hipLaunchKernelGGL((k_gram<MODE, float>), dim3(blocks), dim3(256), 0, st, a);
+template <typename PT, int TS>
+hipError_t launch_finish(const void* part, const nq_gram_plan& g, int nA, int nB, int offB, double scale, double* S,
+                         int np, int lds, hipStream_t st) {
+    const int T = (np + 1 + 63) / 64;
+    hipLaunchKernelGGL((k_gram_finish<PT, TS>), dim3(T * (T + 1) / 2), dim3(256), 0, st, (const PT*)part, g.splits,
+                       g.tiles, nA, g.TA, nB, offB, scale, S, np, lds);
     return hipGetLastError();
+}
+
+template <int MODE, typename YT>
+void launch_part(const gram_args& a, const nq_gram_plan& g, hipStream_t st) {
+    hipLaunchKernelGGL((k_gram_part<MODE, YT>), dim3((unsigned)(g.tiles * g.splits)), dim3(256), 0, st,
+                       (const YT*)a.Y, a.Ns, a.ldy, a.mu, a.nA, g.TA, a.nB, g.kchunk, g.tiles, g.splits, a.part);
 }
 
 }  // namespace
 
 hipError_t nq_launch_gram(const gram_args& a, int mode, hipStream_t st) {
-    switch (mode) {
-        case NQ_GRAM_F64: return launch_mode<NQ_GRAM_F64>(a, st);
-        case NQ_GRAM_F32: return launch_mode<NQ_GRAM_F32>(a, st);
+    if (mode != NQ_GRAM_F64 && mode != NQ_GRAM_F32) return hipErrorInvalidValue;
+    const nq_gram_plan g = nq_plan_gram(mode, a.nA, a.nB, a.Ns, 0);
+    if (g.tiles > 0 && mode == NQ_GRAM_F64) {
+        if (a.y_fp64) launch_part<NQ_GRAM_F64, double>(a, g, st);
+        else launch_part<NQ_GRAM_F64, float>(a, g, st);
+    } else if (g.tiles > 0) {
+        if (a.y_fp64) launch_part<NQ_GRAM_F32, double>(a, g, st);
+        else launch_part<NQ_GRAM_F32, float>(a, g, st);
     }
-    return hipErrorInvalidValue;
+    if (mode == NQ_GRAM_F64)
+        return launch_finish<double, 64>(a.part, g, a.nA, a.nB, a.offB, a.scale, a.S, a.np, a.lds, st);
+    return launch_finish<float, 64>(a.part, g, a.nA, a.nB, a.offB, a.scale, a.S, a.np, a.lds, st);
 }
 
 hipError_t nq_launch_center_t(const void* Y, int y_fp64, int64_t Ns, int ldy, int c0, int n, const double* mu,
@@ -517,55 +564,50 @@ hipError_t nq_launch_center_t(const void* Y, int y_fp64, int64_t Ns, int ldy, in
     return hipGetLastError();
 }
 
-// split-K chunks of the BF16 Gram: max_splits when given (a tuned shape),
-// otherwise about three tiles in flight per CU, with the partial sums (64 KB
-// per tile and chunk) kept within twice the BF16 input so that small
-// problems (many of them sharing the device) do not turn into partial-sum
-// traffic; at most one chunk per 64 samples and 64 chunks
-int nq_gram_split_plan(int nA, int nB, int64_t nsp, int max_splits, int64_t* kchunk) {
-    const int TA = (nA + 127) / 128, TB = (nB + 127) / 128;
-    const int tiles = TA * (TA + 1) / 2 + TB * (TB + 1) / 2;
-    int s;
-    if (max_splits > 0) {
+// Tiles and sample chunks of a Gram.  BF16 (128 x 128 tiles): max_splits chunks when given (a tuned
+// shape), otherwise about three tiles in flight per CU.  FP64 / FP32 (64 x 64 tiles): a multiple of
+// eight chunks, one XCD each, at least three workgroups per CU.  The partial sums stay within twice
+// the input, so that small problems (many of them sharing the device) do not turn into partial-sum
+// traffic; at least 64 samples per chunk, at most 64 chunks.
+// One workgroup per tile over all samples, one launch per block -> chunks (time of both blocks):
+// FP64 4x4 XYZ (702 tiles, 16384 samples) 3.3 -> 2.4 ms beside the forces launch; 12 sites (240 tiles)
+// 4.1 -> 0.75 ms beside it; ket RBM of 16 sites (171 tiles, 8192 samples) alone 0.59 -> 0.24 ms, 49
+// TFLOP/s; FP32 12 sites 2.26 -> 0.41 ms; 6 sites (6 tiles, 2000 samples) 294 -> 12 us.  Twice and four
+// times the chunks changed none of these by more than 5 % and made the sum over them longer.
+nq_gram_plan nq_plan_gram(int mode, int nA, int nB, int64_t Ns, int max_splits) {
+    nq_gram_plan g{};
+    const bool bf16 = mode == NQ_GRAM_BF16;
+    const int ts = bf16 ? 128 : 64;
+    const int TB = (nB + ts - 1) / ts;
+    g.TA = (nA + ts - 1) / ts;
+    g.tiles = g.TA * (g.TA + 1) / 2 + TB * (TB + 1) / 2;
+    g.elt = mode == NQ_GRAM_F64 ? 8 : 4;
+    const int64_t ns = bf16 ? (Ns + 63) / 64 * 64 : Ns;   // the transposed copy is padded
+    int64_t s = 1;
+    if (bf16 && max_splits > 0) {
         s = max_splits;
-    } else {
-        s = tiles > 0 ? (3 * 256 + tiles - 1) / tiles : 1;
-        const int64_t in_bytes = 2 * nsp * (int64_t)(nA + nB);
-        const int64_t cap = tiles > 0 ? 2 * in_bytes / ((int64_t)tiles * 128 * 128 * 4) : 1;
-        if (cap < s) s = cap > 1 ? (int)cap : 1;
+    } else if (g.tiles > 0) {
+        s = bf16 ? (3 * 256 + g.tiles - 1) / g.tiles : (int64_t)8 * ((3 * 256 + 8 * g.tiles - 1) / (8 * g.tiles));
+        const int64_t in_bytes = (bf16 ? 2 : g.elt) * ns * (int64_t)(nA + nB);
+        s = std::min(s, 2 * in_bytes / ((int64_t)g.tiles * ts * ts * g.elt));
     }
-    const int maxs = nsp >= 64 ? (int)(nsp / 64) : 1;
-    s = s < maxs ? s : maxs;
-    s = s < 64 ? s : 64;
-    s = s > 1 ? s : 1;
-    int64_t kc = (nsp + s - 1) / s;
-    kc = (kc + 63) / 64 * 64;
-    if (kc < 64) kc = 64;
-    *kchunk = kc;
-    return (int)((nsp + kc - 1) / kc);
-}
-
-size_t nq_gram_split_part_floats(int nA, int nB, int64_t nsp, int max_splits) {
-    int64_t kc;
-    const int splits = nq_gram_split_plan(nA, nB, nsp, max_splits, &kc);
-    const int TA = (nA + 127) / 128, TB = (nB + 127) / 128;
-    const int tiles = TA * (TA + 1) / 2 + TB * (TB + 1) / 2;
-    return (size_t)splits * tiles * 128 * 128;
+    s = std::min<int64_t>(s, ns >= 64 ? ns / 64 : 1);
+    s = std::min<int64_t>(s, 64);
+    s = std::max<int64_t>(s, 1);
+    const int64_t unit = bf16 ? 64 : 32;
+    g.kchunk = std::max<int64_t>(((ns + s - 1) / s + unit - 1) / unit * unit, unit);
+    g.splits = (int)((ns + g.kchunk - 1) / g.kchunk);
+    g.part_bytes = (size_t)g.splits * g.tiles * ts * ts * g.elt;
+    return g;
 }
 
 hipError_t nq_launch_gram2_bf16(const __bf16* Yt, int64_t nsp, int nA, int nB, int offB, double scale, float* part,
                                 double* S, int np, int lds, int max_splits, hipStream_t st) {
-    int64_t kc;
-    const int splits = nq_gram_split_plan(nA, nB, nsp, max_splits, &kc);
-    const int TA = (nA + 127) / 128, TB = (nB + 127) / 128;
-    const int tiles = TA * (TA + 1) / 2 + TB * (TB + 1) / 2;
-    if (tiles > 0)
-        hipLaunchKernelGGL(k_gram_bf16_part, dim3(tiles, splits), dim3(256), 0, st, Yt, nsp, nA, TA, nB, kc, tiles,
-                           part);
-    const int TS = (np + 1 + 63) / 64;
-    hipLaunchKernelGGL(k_gram_finish, dim3(TS * (TS + 1) / 2), dim3(256), 0, st, part, splits, tiles, nA, TA, nB, offB,
-                       scale, S, np, lds);
-    return hipGetLastError();
+    const nq_gram_plan g = nq_plan_gram(NQ_GRAM_BF16, nA, nB, nsp, max_splits);
+    if (g.tiles > 0)
+        hipLaunchKernelGGL(k_gram_bf16_part, dim3(g.tiles, g.splits), dim3(256), 0, st, Yt, nsp, nA, g.TA, nB,
+                           g.kchunk, g.tiles, part);
+    return launch_finish<float, 128>(part, g, nA, nB, offB, scale, S, np, lds, st);
 }
 
 hipError_t nq_launch_colsum(const void* Y, int y_fp64, int64_t Ns, int R, double* part, int chunks,
@@ -584,17 +626,10 @@ hipError_t nq_launch_colsum_finish(const double* part, int chunks, int R, double
     return hipGetLastError();
 }
 
-void nq_gram_shape(int nA, int nB, int64_t nsp, int max_splits, int* TA, int* tiles, int* splits, int64_t* kchunk) {
-    *splits = nq_gram_split_plan(nA, nB, nsp, max_splits, kchunk);
-    *TA = (nA + 127) / 128;
-    const int TB = (nB + 127) / 128;
-    *tiles = *TA * (*TA + 1) / 2 + TB * (TB + 1) / 2;
-}
-
 hipError_t nq_pk_sbuild(const nq_pk_member* M, const nq_pk_launch& L, hipStream_t st) {
     if (L.nblk <= 0) return hipSuccess;
     const dim3 g((unsigned)L.nblk), b((unsigned)L.threads);
-    const bool f64 = L.variant != 0;
+    const bool f64 = L.variant != 0;   // column sums and centring
     switch (L.kernel) {
         case NQ_PK_COLSUM:
             if (f64) hipLaunchKernelGGL((k_colsum_pk<double>), g, b, 0, st, M, L.blk);
@@ -605,24 +640,26 @@ hipError_t nq_pk_sbuild(const nq_pk_member* M, const nq_pk_launch& L, hipStream_
             if (f64) hipLaunchKernelGGL((k_center_t_pk<double>), g, b, 0, st, M, L.blk);
             else hipLaunchKernelGGL((k_center_t_pk<float>), g, b, 0, st, M, L.blk);
             break;
-        case NQ_PK_GRAM_PART: hipLaunchKernelGGL(k_gram_bf16_part_pk, g, b, 0, st, M, L.blk); break;
-        case NQ_PK_GRAM_FIN: hipLaunchKernelGGL(k_gram_finish_pk, g, b, 0, st, M, L.blk); break;
-        case NQ_PK_GRAM:
-            // variant: S-build mode | FP64 rows << 1
-            switch (L.variant) {
-                case 0: hipLaunchKernelGGL((k_gram_pk<NQ_GRAM_F64, float>), g, b, 0, st, M, L.blk, L.param); break;
-                case 1: hipLaunchKernelGGL((k_gram_pk<NQ_GRAM_F32, float>), g, b, 0, st, M, L.blk, L.param); break;
-                case 2: hipLaunchKernelGGL((k_gram_pk<NQ_GRAM_F64, double>), g, b, 0, st, M, L.blk, L.param); break;
-                case 3: hipLaunchKernelGGL((k_gram_pk<NQ_GRAM_F32, double>), g, b, 0, st, M, L.blk, L.param); break;
-                default: return hipErrorInvalidValue;
+        case NQ_PK_GRAM_PART:
+            // variant: S-build mode | FP64 rows << 2
+            switch (L.variant & 3) {
+                case NQ_GRAM_F64:
+                    if (L.variant & 4) hipLaunchKernelGGL((k_gram_part_pk<NQ_GRAM_F64, double>), g, b, 0, st, M, L.blk);
+                    else hipLaunchKernelGGL((k_gram_part_pk<NQ_GRAM_F64, float>), g, b, 0, st, M, L.blk);
+                    break;
+                case NQ_GRAM_F32:
+                    if (L.variant & 4) hipLaunchKernelGGL((k_gram_part_pk<NQ_GRAM_F32, double>), g, b, 0, st, M, L.blk);
+                    else hipLaunchKernelGGL((k_gram_part_pk<NQ_GRAM_F32, float>), g, b, 0, st, M, L.blk);
+                    break;
+                default: hipLaunchKernelGGL(k_gram_bf16_part_pk, g, b, 0, st, M, L.blk);
             }
+            break;
+        case NQ_PK_GRAM_FIN:
+            if (L.variant == NQ_GRAM_F64) hipLaunchKernelGGL((k_gram_finish_pk<double, 64>), g, b, 0, st, M, L.blk);
+            else if (L.variant == NQ_GRAM_F32) hipLaunchKernelGGL((k_gram_finish_pk<float, 64>), g, b, 0, st, M, L.blk);
+            else hipLaunchKernelGGL((k_gram_finish_pk<float, 128>), g, b, 0, st, M, L.blk);
             break;
         default: return hipErrorInvalidValue;
     }
     return hipGetLastError();
-}
-
-int nq_pk_gram_blocks(const nq_pk_member& m, int which) {
-    const int T = (pk_gram_args(m, which).n + 63) / 64;
-    return T * (T + 1) / 2;
 }

@@ -1437,13 +1437,6 @@ __global__ __launch_bounds__(256) void k_prep_pk(const nq_pk_member* M, const ui
     }
 }
 
-__global__ __launch_bounds__(256) void k_sfill_pk(const nq_pk_member* M, const uint2* blk) {
-    const uint2 b = blk[blockIdx.x];
-    const nq_pk_member& m = pk_m(M, b);
-    const int64_t i = (int64_t)pk_x(b) * blockDim.x + threadIdx.x;
-    if (i < (int64_t)m.ldS * m.ldS) m.S[i] = 0.0;
-}
-
 template <typename T>
 __global__ __launch_bounds__(1024) void k_stats_pk(const nq_pk_member* M, const uint2* blk) {
     const nq_pk_member& m = pk_m(M, blk[blockIdx.x]);
@@ -1782,28 +1775,19 @@ hipError_t nq_pk_plan(const nq_pk_member& m, int kernel, int param, nq_pk_shape*
             o->gy = NQ_FORCE_GROUPS;
             break;
         case NQ_PK_FORCE_FIN: o->gx = (int)nblk(m.np, 256); break;
-        case NQ_PK_SFILL:
-            if (m.s_mode >= 0) o->gx = (int)nblk((int64_t)m.ldS * m.ldS, 256);
-            break;
-        case NQ_PK_GRAM:
-            if (m.s_mode >= 0) {
-                o->variant = m.s_mode | (m.fp64 << 1);
-                o->gx = nq_pk_gram_blocks(m, param);
-            }
-            break;
         case NQ_PK_CENTER:
-            if (m.s_mode >= 0) break;
+            if (m.s_mode != NQ_GRAM_BF16) break;
             o->variant = m.fp64;
             o->gx = (m.R + 63) / 64;
             o->gy = (int)((m.nsp + 63) / 64);
             break;
         case NQ_PK_GRAM_PART:
-            if (m.s_mode >= 0) break;
+            o->variant = m.s_mode | (m.s_mode != NQ_GRAM_BF16 && m.fp64 ? 4 : 0);
             o->gx = m.tiles;
             o->gy = m.splits;
             break;
         case NQ_PK_GRAM_FIN: {
-            if (m.s_mode >= 0) break;
+            o->variant = m.s_mode;
             const int TS = (m.np + 1 + 63) / 64;
             o->gx = TS * (TS + 1) / 2;
             break;
@@ -1867,7 +1851,6 @@ hipError_t nq_pk_solve(const nq_pk_member* M, const nq_pk_launch& L, hipStream_t
             break;
         case NQ_PK_FORCE_PART: hipLaunchKernelGGL(k_force_part_pk, g, b, 0, st, M, L.blk); break;
         case NQ_PK_FORCE_FIN: hipLaunchKernelGGL(k_force_finish_pk, g, b, 0, st, M, L.blk); break;
-        case NQ_PK_SFILL: hipLaunchKernelGGL(k_sfill_pk, g, b, 0, st, M, L.blk); break;
         case NQ_PK_SPLIT_COPY: hipLaunchKernelGGL(k_split_copy_pk, g, b, 0, st, M, L.blk); break;
         case NQ_PK_CHOL_STEP: hipLaunchKernelGGL(k_chol_step_pk, g, b, 0, st, M, L.blk, phase, j); break;
         case NQ_PK_SCHUR: hipLaunchKernelGGL(k_split_schur_pk, g, b, 0, st, M, L.blk); break;
@@ -1894,8 +1877,7 @@ hipError_t nq_pk_run(const nq_pk_member* M, const nq_pk_launch& L, hipStream_t s
         case NQ_PK_COLSUM_FIN:
         case NQ_PK_CENTER:
         case NQ_PK_GRAM_PART:
-        case NQ_PK_GRAM_FIN:
-        case NQ_PK_GRAM: return nq_pk_sbuild(M, L, st);
+        case NQ_PK_GRAM_FIN: return nq_pk_sbuild(M, L, st);
         default: return nq_pk_solve(M, L, st);
     }
 }

@@ -65,18 +65,27 @@ int nq_sampler_lanes_per_chain(const ndm_dims& d);
 hipError_t nq_launch_metropolis(const samp_args& a, hipStream_t st);
 
 // ---- S build (k_sbuild.hip)
-enum { NQ_GRAM_F64 = 0, NQ_GRAM_F32 = 1 };
-// S[o + r, o + c] += scale * sum_s (Y[s, c0 + r] - mu[c0 + r]) (Y[s, c0 + c] - mu[c0 + c])
-// for r, c < n; S is column-major with leading dimension lds.  Y is Ns x ldy of
-// type double (y_fp64) or float.
+enum { NQ_GRAM_F64 = 0, NQ_GRAM_F32 = 1, NQ_GRAM_BF16 = 2 };
+// tiles (TA a side in block A), sample chunks of kchunk samples, element size and bytes of the
+// partial sums of a Gram of block A = nA columns and block B = nB; max_splits: BF16 chunks (0: chosen)
+struct nq_gram_plan {
+    int TA, tiles, splits, elt;
+    int64_t kchunk;
+    size_t part_bytes;
+};
+nq_gram_plan nq_plan_gram(int mode, int nA, int nB, int64_t Ns, int max_splits);
+// FP64 / FP32 S build: block A = Y columns [0, nA), block B = the next nB (Y: Ns x ldy of double
+// (y_fp64) or float), centred by mu (nullable), written as nq_launch_gram2_bf16 writes S; part:
+// nq_plan_gram's part_bytes
 struct gram_args {
     const void* Y;
     int y_fp64;
     int64_t Ns;
-    int ldy, c0, n;
-    const double* mu;          // column means (length >= c0 + n), nullable
+    int ldy, nA, nB, offB;
+    const double* mu;
+    void* part;
     double* S;
-    int lds, o;
+    int np, lds;
     double scale;
 };
 hipError_t nq_launch_gram(const gram_args& a, int mode, hipStream_t st);
@@ -88,10 +97,8 @@ hipError_t nq_launch_center_t(const void* Y, int y_fp64, int64_t Ns, int ldy, in
 // split-K BF16 Gram of up to two column blocks of Yt (block A: rows [0, nA),
 // block B: rows [nA, nA + nB)) written into all of the (np + 1)^2 matrix S:
 // scale * A^T A at [0, nA) plus scale * B^T B at [offB, offB + nB), zeros
-// elsewhere (row and column np included); `part` holds
-// nq_gram_split_part_floats(nA, nB, nsp, max_splits) floats of partial sums;
-// max_splits: split-K chunks (0: chosen from the shape)
-size_t nq_gram_split_part_floats(int nA, int nB, int64_t nsp, int max_splits);
+// elsewhere (row and column np included); `part` holds nq_plan_gram's
+// part_bytes of partial sums; max_splits: split-K chunks (0: chosen from the shape)
 hipError_t nq_launch_gram2_bf16(const __bf16* Yt, int64_t nsp, int nA, int nB, int offB, double scale, float* part,
                                 double* S, int np, int lds, int max_splits, hipStream_t st);
 
@@ -342,12 +349,11 @@ struct nq_pk_member {
     double* Fpart;             // force_grid x np force partials
     double* fpart2;            // NQ_FORCE_GROUPS x np
     double* F;
-    int s_mode;                // S build: NQ_GRAM_F64 / NQ_GRAM_F32 (fill + two k_gram), -1: BF16 split-K
-    // BF16 S build
+    int s_mode;                // S build: NQ_GRAM_F64, NQ_GRAM_F32 or NQ_GRAM_BF16
     __bf16* Yt;
     int64_t nsp, kchunk;
     int nA, nB, offB, TA, tiles, splits, ldS;
-    float* gpart;
+    void* gpart;
     double* S;
     // split Cholesky solve (nq_split_factor, nq_split_substitute)
     double* A2;
@@ -383,8 +389,6 @@ enum {
     NQ_PK_CENTER,
     NQ_PK_GRAM_PART,
     NQ_PK_GRAM_FIN,
-    NQ_PK_SFILL,         // S = 0 before the FP64 / FP32 Gram blocks
-    NQ_PK_GRAM,          // param: Gram block (0: A, 1: B)
     NQ_PK_SPLIT_COPY,
     NQ_PK_CHOL_STEP,     // param: phase << 16 | panel number within the phase
     NQ_PK_SCHUR,
@@ -432,5 +436,3 @@ hipError_t nq_pk_sbuild(const nq_pk_member* M, const nq_pk_launch& L, hipStream_
 hipError_t nq_pk_solve(const nq_pk_member* M, const nq_pk_launch& L, hipStream_t st);
 int nq_est_variant(const est_args& a, bool fp64, int* threads, size_t* lds);
 int nq_sampler_variant(const samp_args& a, int* threads, size_t* lds, int* grid);
-void nq_gram_shape(int nA, int nB, int64_t nsp, int max_splits, int* TA, int* tiles, int* splits, int64_t* kchunk);
-int nq_pk_gram_blocks(const nq_pk_member& m, int which);

@@ -302,6 +302,16 @@ void gram_blocks(const nqh_ctx* c, int* nA, int* nB, int* offB) {
     }
 }
 
+int gram_mode(const nqh_ctx* c) {
+    return c->s_prec == NQH_PREC_BF16 ? NQ_GRAM_BF16 : (c->s_prec == NQH_PREC_FP64 ? NQ_GRAM_F64 : NQ_GRAM_F32);
+}
+
+nq_gram_plan gram_plan_of(const nqh_ctx* c, int64_t Ns) {
+    int nA, nB, offB;
+    gram_blocks(c, &nA, &nB, &offB);
+    return nq_plan_gram(gram_mode(c), nA, nB, Ns, c->tune_splits);
+}
+
 // the NDM's S has a zero lambda-mu block: factor it through the split
 bool use_split(const nqh_ctx* c) {
     return !is_rbm(c) && c->d.nlam > 0 && c->d.nlam == c->d.nmu && c->d.npi > 0;
@@ -358,13 +368,10 @@ nqh_status ensure_samples(nqh_ctx* c, int64_t Ns) {
     if ((s = ensure(c, c->tmp, sizeof(double) * nsys(c)))) return s;
     if ((s = ensure(c, c->winv, sizeof(double) * nq_cholesky_winv_doubles(nsys(c))))) return s;
     if ((s = ensure(c, c->info, sizeof(int) * 4))) return s;
-    if (c->s_prec == NQH_PREC_BF16 && c->solver == NQH_SOLVER_CHOLESKY) {
+    if (c->solver == NQH_SOLVER_CHOLESKY) {
         const int64_t nsp = (Ns + 63) / 64 * 64;
-        if ((s = ensure(c, c->Yt, sizeof(uint16_t) * (size_t)ycols(c) * nsp))) return s;
-        int nA, nB, offB;
-        gram_blocks(c, &nA, &nB, &offB);
-        if ((s = ensure(c, c->gpart, sizeof(float) * nq_gram_split_part_floats(nA, nB, nsp, c->tune_splits))))
-            return s;
+        if (c->s_prec == NQH_PREC_BF16 && (s = ensure(c, c->Yt, sizeof(uint16_t) * (size_t)ycols(c) * nsp))) return s;
+        if ((s = ensure(c, c->gpart, gram_plan_of(c, Ns).part_bytes))) return s;
     }
     if ((s = ensure(c, c->flag, sizeof(int) * 4))) return s;
     return NQH_OK;
@@ -458,6 +465,23 @@ hipError_t launch_metropolis(nqh_ctx* c, const samp_args& a) {
     return nq_launch_rbm_metropolis(r, fp64_net(c), c->stream);
 }
 
+// the FP64 or FP32 S build from the O rows of Ns samples
+hipError_t launch_gram(nqh_ctx* c, int64_t Ns) {
+    gram_args g{};
+    g.Y = c->Y.p;
+    g.y_fp64 = fp64_net(c);
+    g.Ns = Ns;
+    g.ldy = ycols(c);
+    gram_blocks(c, &g.nA, &g.nB, &g.offB);
+    g.mu = P<double>(c->mu);
+    g.part = c->gpart.p;
+    g.S = P<double>(c->S);
+    g.np = nsys(c);
+    g.lds = g.np + 1;
+    g.scale = 1.0 / (double)Ns;
+    return nq_launch_gram(g, gram_mode(c), c->stream);
+}
+
 // RBMSplit: estimator, means, statistics, complex force, and the real
 // embedding [[A, -B], [B, A]] of the Hermitian S = A + i B
 nqh_status run_grad_pipeline_rbm(nqh_ctx* c, const uint64_t* keys_dev, int64_t chains, int64_t Lc) {
@@ -498,20 +522,7 @@ nqh_status run_grad_pipeline_rbm(nqh_ctx* c, const uint64_t* keys_dev, int64_t c
         HIPCHK(c, nq_launch_gram2_bf16(Yt, nsp, R, 0, 0, 1.0 / (double)Ns, P<float>(c->gpart), P<double>(c->S), n,
                                        ldS, c->tune_splits, c->stream));
     } else {
-        HIPCHK(c, nq_launch_fill(P<double>(c->S), (int64_t)ldS * ldS, 0.0, c->stream));
-        gram_args g{};
-        g.Y = c->Y.p;
-        g.y_fp64 = f64;
-        g.Ns = Ns;
-        g.ldy = R;
-        g.mu = P<double>(c->mu);
-        g.S = P<double>(c->S);
-        g.lds = ldS;
-        g.scale = 1.0 / (double)Ns;
-        g.c0 = 0;
-        g.n = R;
-        g.o = 0;
-        HIPCHK(c, nq_launch_gram(g, c->s_prec == NQH_PREC_FP64 ? NQ_GRAM_F64 : NQ_GRAM_F32, c->stream));
+        HIPCHK(c, launch_gram(c, Ns));
     }
     HIPCHK(c, nq_launch_embed_complex(P<double>(c->S), npc, ldS, c->stream));
     phase_end(c, PH_SBUILD);
@@ -611,25 +622,7 @@ static nqh_status build_s(nqh_ctx* c, int64_t Ns, bool f64) {
         c->solve_ok = false;
         return NQH_OK;
     }
-    HIPCHK(c, nq_launch_fill(P<double>(c->S), (int64_t)ldS * ldS, 0.0, c->stream));
-    const int mode = c->s_prec == NQH_PREC_FP64 ? NQ_GRAM_F64 : NQ_GRAM_F32;
-    gram_args g{};
-    g.Y = c->Y.p;
-    g.y_fp64 = f64;
-    g.Ns = Ns;
-    g.ldy = d.R;
-    g.mu = P<double>(c->mu);
-    g.S = P<double>(c->S);
-    g.lds = ldS;
-    g.scale = 1.0 / (double)Ns;
-    g.c0 = 0;
-    g.n = d.nlam + d.npi;
-    g.o = 0;
-    HIPCHK(c, nq_launch_gram(g, mode, c->stream));
-    g.c0 = d.nlam + d.npi;
-    g.n = d.npi + d.nmu;
-    g.o = d.nlam;
-    HIPCHK(c, nq_launch_gram(g, mode, c->stream));
+    HIPCHK(c, launch_gram(c, Ns));
     phase_end(c, PH_SBUILD);
     c->last_ns = Ns;
     c->grad_ready = true;
@@ -2427,12 +2420,16 @@ nq_pk_member pk_describe(nqh_ctx* c, double eps, int kind, double lr) {
     m.fpart2 = P<double>(c->fpart2);
     m.F = P<double>(c->F);
     // the S build (build_s): BF16 split-K, or FP64 / FP32 Gram blocks
-    m.s_mode = c->s_prec == NQH_PREC_BF16 ? -1 : (c->s_prec == NQH_PREC_FP64 ? NQ_GRAM_F64 : NQ_GRAM_F32);
+    m.s_mode = gram_mode(c);
     m.nsp = (Ns + 63) / 64 * 64;
     m.Yt = reinterpret_cast<__bf16*>(c->Yt.p);
     gram_blocks(c, &m.nA, &m.nB, &m.offB);
-    nq_gram_shape(m.nA, m.nB, m.nsp, c->tune_splits, &m.TA, &m.tiles, &m.splits, &m.kchunk);
-    m.gpart = P<float>(c->gpart);
+    const nq_gram_plan gp = gram_plan_of(c, Ns);
+    m.TA = gp.TA;
+    m.tiles = gp.tiles;
+    m.splits = gp.splits;
+    m.kchunk = gp.kchunk;
+    m.gpart = c->gpart.p;
     m.S = P<double>(c->S);
     m.ldS = d.np + 1;
     // the split solve (precondition_async) and the update
@@ -2467,11 +2464,8 @@ std::vector<std::pair<int, int>> pk_sequence(const std::vector<nq_pk_member>& M)
     }
     std::vector<std::pair<int, int>> q;
     for (int k : {NQ_PK_PREP, NQ_PK_METROPOLIS, NQ_PK_EST_WALK, NQ_PK_EST_FORCE, NQ_PK_COLSUM, NQ_PK_COLSUM_FIN,
-                  NQ_PK_STATS, NQ_PK_FORCE_PART, NQ_PK_FORCE_FIN, NQ_PK_CENTER, NQ_PK_GRAM_PART, NQ_PK_GRAM_FIN,
-                  NQ_PK_SFILL})
+                  NQ_PK_STATS, NQ_PK_FORCE_PART, NQ_PK_FORCE_FIN, NQ_PK_CENTER, NQ_PK_GRAM_PART, NQ_PK_GRAM_FIN})
         q.push_back({k, 0});
-    q.push_back({NQ_PK_GRAM, 0});
-    q.push_back({NQ_PK_GRAM, 1});
     q.push_back({NQ_PK_SPLIT_COPY, 0});
     for (int j = 0; j < pa; ++j) q.push_back({NQ_PK_CHOL_STEP, j});
     q.push_back({NQ_PK_SCHUR, 0});

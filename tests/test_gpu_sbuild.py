@@ -39,3 +39,29 @@ def test_bf16_gram_matches_cpu_gram_of_rounded_rows(gpu_ok, ref, N, alpha, chain
     assert rel_err(S, S_cpu) < 2e-5
     assert np.array_equal(S, S.T)                 # mirrored exactly
     ctx.close()
+
+
+# samples: fewer than a k-step of the FP64 (16) and FP32 (32) tiles, one past it, several chunks with
+# a ragged last k-step; nA = 15, 78, 210 columns (one tile of 64, ragged, several)
+@pytest.mark.parametrize("sprec", [_lib.PREC_FP64, _lib.PREC_FP32])
+@pytest.mark.parametrize("N,alpha,chains,Lc", [(2, 1, 2, 2), (5, 1, 3, 5), (5, 1, 11, 3), (8, 1, 2, 8), (8, 1, 125, 16),
+                                               (4, 3, 77, 9)])
+def test_gram_chunks_match_cpu_gram(gpu_ok, sprec, N, alpha, chains, Lc):
+    """The FP64 and FP32 Gram of the FP64 network's rows against the CPU Gram
+    of the same rows in FP64: rounding of the sums only (FP64: 1e-12; FP32:
+    the centred rows rounded to 24 bits, 2 x 6e-8 per product, and sums of at
+    most 2000 addends in FP32, below 1e-5 of the largest element)."""
+    flat, _, _ = ising(N)
+    ctx = Context(0, 1)
+    ctx.set_problem(flat)
+    ctx.set_ndm(N, alpha * N, alpha * N)
+    ctx.set_params(params(ctx.np_, seed=31, sigma=0.2))
+    ctx.set_precision(_lib.PREC_FP64, sprec)
+    keys = random_keys(N, chains * Lc, seed=32)
+    _, O = ctx.logpsi_grad(keys)
+    _, S, _, _ = ctx.grad_from_samples(keys, chains, Lc)
+    Oc = O - O.mean(axis=0)
+    S_cpu = (Oc.real.T @ Oc.real + Oc.imag.T @ Oc.imag) / len(keys)
+    assert rel_err(S, S_cpu) < (1e-12 if sprec == _lib.PREC_FP64 else 1e-5)
+    assert np.array_equal(S, S.T)
+    ctx.close()
