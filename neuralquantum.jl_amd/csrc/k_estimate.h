@@ -18,8 +18,10 @@
 // connection flipping k sites costs k FMAs per unit.
 //
 // Three kinds of launch (template parameter KIND):
-//   EK_WALK   log rho, O rows, and pass 1 over the connections: softplus
-//             (or logcosh) of the changed angles + one wave reduction -> W_c
+//   EK_WALK   log rho, O rows, and pass 1 over the connections: FP64 by
+//             products of the units' factors, FP32 (and FP64 weights outside
+//             their range) by softplus (or logcosh) of the changed angles +
+//             one wave reduction -> W_c
 //             = mel_c exp(log rho_c - log rho_s), L_loc = sum_c W_c; with
 //             rec_mode 1 it writes per sample the changed connections (W_c,
 //             flip masks), their count and the unchanged connections' mel sum.
@@ -79,6 +81,104 @@ __device__ __forceinline__ int p2ref(int k, const ndm_dims& d) {
 // after the reduction
 template <typename T> constexpr int est_batch() { return sizeof(T) == 8 ? 4 : 8; }
 
+// ---- FP64 connections by products (the walk; the forces below)
+// e^(dlog rho) of a connection is a product over the units, as in the sampler: with E = e^(K theta),
+// w = e^(K z) (K = 1 softplus, 2 logcosh, whose linear parts join the visible biases)
+//   |.|   = sqrt(prod over lambda units of (1 + E') / (1 + E)) |prod over Pi units of (1 + w') / (1 + w)|
+//   phase = (1/2) log(prod over mu units of (1 + E') / (1 + E)) (row side; minus, column side) + the
+//           phase of the complex Pi product
+// and E' = E e^(+-2 K w_i) per flipped site, from tables in LDS.  Per unit and connection that is one
+// product per flipped site, an addition and a product, in place of exp + log1p (real units) and exp +
+// sincos + log1p + atan2 (Pi units), about 360 instructions of the wave per connection; the square
+// root, logarithm, exponential and sincos that finish a connection are taken by one lane per
+// connection, 64 connections at a time.
+// Four connections per round, lane i + 16 k taking connection k and its units 16 t + i (lambda, mu and
+// Pi tiles of 16), then products over the 16 lanes.  Bound by FP64 issue at two waves per SIMD.
+// Before and now: 4x4 XYZ, 16384 samples 1.44 -> 0.34 ms; 12 sites, 16384 samples 0.66 -> 0.19;
+// the exact sum over 2^20 configurations of 10 sites 34.4 -> 7.7.
+// The ranges keep every partial product inside e^(+-700); a network whose weights leave them (or whose
+// tables do not fit in LDS beside the connections) takes the sums of f instead.
+constexpr double kEstRange = 600.0;
+
+// doubles: e^(2 K w) and e^(-2 K w) of (site, lambda or mu, unit); complex e^(+-K (u_la + i u_mu)) of
+// (site, Pi unit); the effective biases (la, mu) of a site; scratch of the ranges
+__host__ __device__ inline int ratio_bytes(const ndm_dims& d) {
+    return (8 * (4 * d.N * d.nh + 4 * d.N * d.na + 2 * d.N + d.N + 4) + 15) & ~15;
+}
+struct ratio_tables {
+    double *up, *dn;      // [(2 i + s) nh + h], s = 0 lambda, 1 mu
+    double2 *pup, *pdn;   // [i na + a]
+    double2* bias;        // [i]
+    double* range;        // max range of a real unit, of a Pi unit, then per site the sum over the units
+};
+__device__ __forceinline__ ratio_tables ratio_at(unsigned char* mem, const ndm_dims& d) {
+    ratio_tables t;
+    t.pup = reinterpret_cast<double2*>(mem);
+    t.pdn = t.pup + d.N * d.na;
+    t.bias = t.pdn + d.N * d.na;
+    t.up = reinterpret_cast<double*>(t.bias + d.N);
+    t.dn = t.up + 2 * d.N * d.nh;
+    t.range = t.dn + 2 * d.N * d.nh;
+    return t;
+}
+// fills the tables from the parameters gp (all threads; synchronises) and says whether the ranges hold:
+// th, tp: real and Pi units a lane multiplies, fmax: sites a connection flips
+template <int ACT>
+__device__ __forceinline__ bool ratio_fill(const ratio_tables& t, const double* gp, const ndm_dims& d, int th, int tp,
+                                           int fmax) {
+    constexpr double K = ACT == NQ_ACT_LOGCOSH ? 2.0 : 1.0;
+    const int N = d.N, nh = d.nh, na = d.na, units = 2 * nh + na;
+    for (int k = threadIdx.x; k < N + 4; k += blockDim.x) t.range[k] = 0.0;
+    for (int k = threadIdx.x; k < 2 * N * nh; k += blockDim.x) {
+        const int h = k % nh, is = k / nh, i = is >> 1;
+        const double e = exp(2.0 * K * gp[((is & 1) ? d.wmu : d.wla) + h + nh * i]);
+        t.up[k] = e;
+        t.dn[k] = 1.0 / e;
+    }
+    for (int k = threadIdx.x; k < N * na; k += blockDim.x) {
+        double s, c;
+        sincos(K * gp[d.umu + k], &s, &c);
+        const double e = exp(K * gp[d.ula + k]), r = 1.0 / e;
+        t.pup[k] = make_double2(e * c, e * s);
+        t.pdn[k] = make_double2(r * c, -r * s);
+    }
+    __syncthreads();
+    // unit u's weight at site i: lambda, mu, then the Pi units' real parts
+    auto weight = [&](int u, int i) {
+        return u < nh ? gp[d.wla + u + nh * i] : (u < 2 * nh ? gp[d.wmu + u - nh + nh * i] : gp[d.ula + u - 2 * nh + na * i]);
+    };
+    for (int u = threadIdx.x; u < units; u += blockDim.x) {
+        double m = fabs(u < nh ? gp[d.hla + u] : (u < 2 * nh ? gp[d.hmu + u - nh] : gp[d.dla + u - 2 * nh]));
+        for (int i = 0; i < N; ++i) m += fabs(weight(u, i));
+        atomicMax(reinterpret_cast<unsigned long long*>(t.range) + (u < 2 * nh ? 0 : 1),
+                  (unsigned long long)__double_as_longlong(K * m));
+    }
+    for (int k = threadIdx.x; k < N * 16; k += blockDim.x) {
+        const int i = k >> 4;
+        double m = 0.0;
+        for (int u = k & 15; u < units; u += 16) m += 2.0 * K * fabs(weight(u, i));
+        atomicAdd(t.range + 2 + i, m);
+    }
+    for (int i = threadIdx.x; i < N; i += blockDim.x) {
+        double bl = gp[d.bla + i], bm = gp[d.bmu + i];
+        if constexpr (ACT == NQ_ACT_LOGCOSH) {
+            for (int h = 0; h < nh; ++h) {
+                bl -= gp[d.wla + h + nh * i];
+                bm -= gp[d.wmu + h + nh * i];
+            }
+            for (int q = 0; q < na; ++q) {
+                bl -= gp[d.ula + q + na * i];
+                bm -= gp[d.umu + q + na * i];
+            }
+        }
+        t.bias[i] = make_double2(bl, bm);
+    }
+    __syncthreads();
+    bool ok = th * (t.range[0] + 0.7) <= kEstRange && tp * (t.range[1] + 0.7) <= 0.5 * kEstRange;
+    for (int i = 0; i < N; ++i) ok = ok && fmax * t.range[2 + i] <= kEstRange;
+    return ok;
+}
+
 // TAB_LDS: the connection table is staged in LDS (a compile-time choice, so
 // every table access is a known LDS or global access, never a flat one)
 // the block body; bx = the workgroup's number in its problem's grid of gx
@@ -94,7 +194,9 @@ __device__ __forceinline__ void estimate_body(const est_args& a, int bx, int gx)
     unsigned long long* sF = reinterpret_cast<unsigned long long*>(smem + a.lds_param_bytes);
     int* poison = reinterpret_cast<int*>(sF + 2 * d.np);
     const int fbytes = WALK ? 0 : fx_bytes(d.np);
-    cplx<T>* sW = reinterpret_cast<cplx<T>*>(smem + a.lds_param_bytes + fbytes);
+    constexpr bool RATIO = WALK && sizeof(T) == 8;
+    const int rbytes = RATIO && a.ratio ? ratio_bytes(d) : 0;
+    cplx<T>* sW = reinterpret_cast<cplx<T>*>(smem + a.lds_param_bytes + fbytes + rbytes);
     const int wpb0 = blockDim.x >> 6;
     uint2* sM = reinterpret_cast<uint2*>(sW + wpb0 * a.max_conn);          // flip masks of the cached connections
     unsigned char* sT = smem + ((reinterpret_cast<unsigned char*>(sM + wpb0 * a.max_conn) - smem + 15) & ~15);
@@ -106,6 +208,14 @@ __device__ __forceinline__ void estimate_body(const est_args& a, int bx, int gx)
         if (threadIdx.x == 0) *poison = 0;
     }
     __syncthreads();
+    bool products = false;   // the connections by products of the units' factors
+    const ratio_tables rt = ratio_at(smem + a.lds_param_bytes + fbytes, d);
+    if constexpr (RATIO) {
+        if (a.ratio) {
+            products = __builtin_amdgcn_readfirstlane(
+                           (int)ratio_fill<ACT>(rt, reinterpret_cast<const double*>(sp), d, 2 * RS, 2 * PS, tab.fmax)) != 0;
+        }
+    }
 
     const int lane0 = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -431,6 +541,163 @@ __device__ __forceinline__ void estimate_body(const est_args& a, int bx, int gx)
                         Lacc = cadd(Lacc, W);
                     }
                 }
+            } else if (RATIO && products) {
+              if constexpr (RATIO) {
+                constexpr double K = ACT == NQ_ACT_LOGCOSH ? 2.0 : 1.0;
+                constexpr int TH = 2 * RS, TP = 2 * PS;   // tiles of 16 lambda (mu) and Pi units
+                const int il = lane & 15, kg = lane >> 4;
+                double es[RS], ee[RS];
+#pragma unroll
+                for (int r = 0; r < RS; ++r) {
+                    es[r] = exp(K * th_s[r]);
+                    ee[r] = exp(K * th_e[r]);
+                }
+                // the sample's factors in the tile layout (0: no such unit) and the lane's products
+                double ls[TH], le[TH], ms_[TH], me_[TH];
+                cplx<double> w[TP];
+                double qls = 1.0, qle = 1.0, qms = 1.0, qme = 1.0;
+#pragma unroll
+                for (int t = 0; t < TH; ++t) {
+                    const int h = 16 * t + il, u = nh + h;
+                    const bool in = h < nh;
+                    ls[t] = __shfl(es[0], h & 63, 64);
+                    le[t] = __shfl(ee[0], h & 63, 64);
+                    ms_[t] = __shfl(es[0], u & 63, 64);
+                    me_[t] = __shfl(ee[0], u & 63, 64);
+                    if constexpr (RS > 1) {
+                        const double s1 = __shfl(es[1], u & 63, 64), e1 = __shfl(ee[1], u & 63, 64);
+                        ms_[t] = u >= 64 ? s1 : ms_[t];
+                        me_[t] = u >= 64 ? e1 : me_[t];
+                    }
+                    ls[t] = in ? ls[t] : 0.0;
+                    le[t] = in ? le[t] : 0.0;
+                    ms_[t] = in ? ms_[t] : 0.0;
+                    me_[t] = in ? me_[t] : 0.0;
+                    qls *= 1.0 + ls[t];
+                    qle *= 1.0 + le[t];
+                    qms *= 1.0 + ms_[t];
+                    qme *= 1.0 + me_[t];
+                }
+                const double ils = 1.0 / qls, ile = 1.0 / qle, ims = 1.0 / qms;
+                cplx<double> qp = cmk(1.0, 0.0);
+                {
+                    double sn, cs;
+                    sincos(K * pi_z[0].im, &sn, &cs);
+                    const double ex = exp(K * pi_z[0].re);
+#pragma unroll
+                    for (int t = 0; t < TP; ++t) {
+                        const int q = 16 * t + il;
+                        w[t] = cmk(__shfl(ex * cs, q & 63, 64), __shfl(ex * sn, q & 63, 64));
+                        if (q >= na) w[t] = cmk(0.0, 0.0);
+                        qp = cmul(qp, cmk(1.0 + w[t].re, w[t].im));
+                    }
+                }
+                const double ipn = 1.0 / (qp.re * qp.re + qp.im * qp.im);
+                const cplx<double> ipc = cmk(qp.re * ipn, -qp.im * ipn);
+                const int hb = il < nh ? il : 0, ab = il < na ? il : 0;   // tables of absent units: any entry (0 times it)
+                double kl = 1.0, km = 1.0;
+                cplx<double> kc = cmk(1.0, 0.0);
+                for (int c0 = 0, r = 0; c0 < ncc; c0 += 4, ++r) {
+                    uint32_t ms = 0u, me = 0u;
+                    if (c0 + kg < ncc) {
+                        const uint2 mm = mbuf[c0 + kg];
+                        ms = mm.x;
+                        me = mm.y;
+                    }
+                    double pl = 1.0, pm = 1.0;
+                    cplx<double> z[TP];
+#pragma unroll
+                    for (int t = 0; t < TP; ++t) z[t] = w[t];
+                    // one side's flips: the lambda and mu factors into fl, fm, the Pi units' into z
+                    auto side = [&](uint32_t m, uint32_t kk, double (&fl)[TH], double (&fm)[TH], double sgn) {
+                        for (; m; m &= m - 1) {
+                            const int i = __builtin_ctz(m);
+                            const bool down = ((kk >> i) & 1u) != 0;
+                            const double* tb = (down ? rt.dn : rt.up) + 2 * i * nh + hb;
+                            const double2* tc = (down ? rt.pdn : rt.pup) + i * na + ab;
+#pragma unroll
+                            for (int t = 0; t < TH; ++t)
+                                if (16 * t < nh) {
+                                    const int o = 16 * t + hb < nh ? 16 * t : 0;
+                                    fl[t] *= tb[o];
+                                    fm[t] *= tb[o + nh];
+                                }
+#pragma unroll
+                            for (int t = 0; t < TP; ++t)
+                                if (16 * t < na) {
+                                    const double2 f = tc[16 * t + ab < na ? 16 * t : 0];
+                                    z[t] = cmul(z[t], cmk(f.x, sgn * f.y));
+                                }
+                        }
+                    };
+                    if (ms) {
+                        double fl[TH], fm[TH], ql = ils, qm = ims;
+#pragma unroll
+                        for (int t = 0; t < TH; ++t) { fl[t] = ls[t]; fm[t] = ms_[t]; }
+                        side(ms, ks, fl, fm, 1.0);
+#pragma unroll
+                        for (int t = 0; t < TH; ++t)
+                            if (16 * t < nh) { ql *= 1.0 + fl[t]; qm *= 1.0 + fm[t]; }
+                        pl = ql;
+                        pm = qm;
+                    }
+                    if (me) {
+                        double fl[TH], fm[TH], ql = ile, qm = 1.0;
+#pragma unroll
+                        for (int t = 0; t < TH; ++t) { fl[t] = le[t]; fm[t] = me_[t]; }
+                        side(me, ke, fl, fm, -1.0);
+#pragma unroll
+                        for (int t = 0; t < TH; ++t)
+                            if (16 * t < nh) { ql *= 1.0 + fl[t]; qm *= 1.0 + fm[t]; }
+                        pl *= ql;
+                        pm *= qme / qm;
+                    }
+                    cplx<double> pc = ipc;
+#pragma unroll
+                    for (int t = 0; t < TP; ++t)
+                        if (16 * t < na) pc = cmul(pc, cmk(1.0 + z[t].re, z[t].im));
+                    // products over the connection's 16 lanes
+                    pl = group_product<16>(pl);
+                    pm = group_product<16>(pm);
+                    pc = cmul(pc, cmk(dpp_d<0xB1>(pc.re), dpp_d<0xB1>(pc.im)));
+                    pc = cmul(pc, cmk(dpp_d<0x4E>(pc.re), dpp_d<0x4E>(pc.im)));
+                    pc = cmul(pc, cmk(dpp_d<0x141>(pc.re), dpp_d<0x141>(pc.im)));
+                    pc = cmul(pc, cmk(dpp_d<0x140>(pc.re), dpp_d<0x140>(pc.im)));
+                    // lane i + 16 k keeps round i's connection k; after 16 rounds every lane finishes its own
+                    const bool mine = il == (r & 15);
+                    kl = mine ? pl : kl;
+                    km = mine ? pm : km;
+                    kc.re = mine ? pc.re : kc.re;
+                    kc.im = mine ? pc.im : kc.im;
+                    if ((r & 15) == 15 || c0 + 4 >= ncc) {
+                        const int c = 4 * ((r & ~15) + il) + kg;
+                        if (c < ncc) {
+                            const uint2 mm = mbuf[c];
+                            double dre = 0.0, dim = 0.5 * log(km);
+                            for (uint32_t m = mm.x; m; m &= m - 1) {
+                                const int i = __builtin_ctz(m);
+                                const double cc = 0.5 * cflip<double>(ks, i);
+                                const double2 b = rt.bias[i];
+                                dre += cc * b.x;
+                                dim += cc * b.y;
+                            }
+                            for (uint32_t m = mm.y; m; m &= m - 1) {
+                                const int i = __builtin_ctz(m);
+                                const double cc = 0.5 * cflip<double>(ke, i);
+                                const double2 b = rt.bias[i];
+                                dre += cc * b.x;
+                                dim -= cc * b.y;
+                            }
+                            double sn, cs;
+                            sincos(dim, &sn, &cs);
+                            const double er = sqrt(kl) * exp(dre);
+                            const cplx<double> W = cmul(cmul(wbuf[c], cmk(er * cs, er * sn)), kc);
+                            wbuf[c] = W;
+                            Lacc = cadd(Lacc, W);
+                        }
+                    }
+                }
+              }
             } else {
                 constexpr int EB = est_batch<T>(), LG = 32 / EB;   // LG lanes hold one connection's sums
                 // FP32 with one Pi unit per lane (na <= 32): two connections' Pi
@@ -1229,7 +1496,8 @@ inline int est_waves(const est_args& a, size_t elt) {
     if (a.G) return 1;
     if (a.waves == 4) return 4;
     if (a.waves == 8 && est_lds_bytes(a, elt, 8) <= 160 * 1024) return 8;
-    return est_lds_bytes(a, elt, 8) > 80 * 1024 ? 4 : 8;
+    // FP64 by products: its registers leave two waves per SIMD anyway, so one workgroup of 8 per CU
+    return est_lds_bytes(a, elt, 8) > (elt == 8 && a.ratio ? 160 : 80) * 1024 ? 4 : 8;
 }
 
 template <typename T, int NMAX, int RS, int PS, int ACT>

@@ -5,18 +5,28 @@
 hipError_t nq_launch_estimate_f32(const est_args& a, int grid, hipStream_t st);
 
 size_t est_lds_bytes(const est_args& a, size_t elt, int waves) {
-    // params | exact force accumulator | waves x (W cache + flip masks) | table (16-aligned);
+    // params | exact force accumulator | factor tables | waves x (W cache + flip masks) | table (16-aligned);
     // the FP32 forces launch stages its parameters in a padded layout of its own
     size_t pb = (size_t)a.lds_param_bytes;
     if (elt == 4 && a.rec_mode == 2 && !a.G)
         pb = std::max(pb, ((size_t)4 * nq_est::force_stage_floats(a.d) + 15) & ~(size_t)15);
     const size_t b = pb + ((a.Fpart || a.G) ? (size_t)fx_bytes(a.d.np) : 0) +
+                     (elt == 8 && a.ratio ? (size_t)nq_est::ratio_bytes(a.d) : 0) +
                      (size_t)waves * (size_t)a.max_conn * (2 * elt + 8);
     return ((b + 15) & ~(size_t)15) + (a.tab_lds ? (size_t)a.tab.bytes : 0);
 }
 
-hipError_t nq_launch_estimate(const est_args& a, bool fp64, int grid, hipStream_t st) {
+void nq_est_tables(est_args& a, bool fp64) {
+    a.ratio = 0;
+    if (!fp64 || a.G || a.rec_mode == 2 || !a.do_conn) return;
+    a.ratio = 1;
+    if (est_lds_bytes(a, 8, 4) > 160 * 1024) a.ratio = 0;
+}
+
+hipError_t nq_launch_estimate(const est_args& a0, bool fp64, int grid, hipStream_t st) {
+    est_args a = a0;
     if (a.d.N > 16) return hipErrorInvalidValue;
+    nq_est_tables(a, fp64);
     est_args b = a;
     if (b.rec_mode == 2) b.tab_lds = 0;
     if (est_lds_bytes(b, fp64 ? 8 : 4, b.G ? 1 : 4) > 160 * 1024) return hipErrorInvalidValue;
@@ -30,6 +40,7 @@ hipError_t nq_launch_estimate(const est_args& a, bool fp64, int grid, hipStream_
 int nq_est_variant(const est_args& a0, bool fp64, int* threads, size_t* lds) {
     est_args a = a0;
     if (a.d.N > 16 || a.G || (a.rec_mode != 1 && a.rec_mode != 2)) return -1;
+    nq_est_tables(a, fp64);
     if ((2 * a.d.nh + 63) / 64 > 1 || (2 * a.d.na + 63) / 64 > 1) return -1;
     const bool force = a.rec_mode == 2;
     if (force) a.tab_lds = 0;

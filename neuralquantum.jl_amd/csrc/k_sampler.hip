@@ -216,26 +216,6 @@ __device__ __forceinline__ void metropolis_body(const samp_args& a, int bx) {
 constexpr double kRatioRange = 600.0, kRatioBias = 60.0;
 constexpr int kRatioRefresh = 64;
 
-// product over aligned groups of W lanes, the same value in every lane of the group
-template <int W>
-__device__ __forceinline__ double group_product(double v) {
-    if constexpr (W >= 2) v *= dpp_d<0xB1>(v);
-    if constexpr (W >= 4) v *= dpp_d<0x4E>(v);
-    if constexpr (W >= 8) v *= dpp_d<0x141>(v);
-    if constexpr (W >= 16) v *= dpp_d<0x140>(v);
-    if constexpr (W >= 32) {
-        double a = v, b = v;
-        plswap<false>(a, b);
-        v = a * b;
-    }
-    if constexpr (W >= 64) {
-        double a = v, b = v;
-        plswap<true>(a, b);
-        v = a * b;
-    }
-    return v;
-}
-
 // LDS bytes of the tables: e^(+-2 K w) per (site, lambda unit), two complex factors per (site, Pi
 // unit), e^(+-2 b) per site
 __host__ __device__ inline size_t ratio_lds_bytes(const ndm_dims& d) {

@@ -381,6 +381,26 @@ __device__ __forceinline__ float dpp_t(float v) { return dpp_f<CTRL>(v); }
 template <int CTRL>
 __device__ __forceinline__ double dpp_t(double v) { return dpp_d<CTRL>(v); }
 
+// product over aligned groups of W lanes, the same value in every lane of the group
+template <int W>
+__device__ __forceinline__ double group_product(double v) {
+    if constexpr (W >= 2) v *= dpp_d<0xB1>(v);
+    if constexpr (W >= 4) v *= dpp_d<0x4E>(v);
+    if constexpr (W >= 8) v *= dpp_d<0x141>(v);
+    if constexpr (W >= 16) v *= dpp_d<0x140>(v);
+    if constexpr (W >= 32) {
+        double a = v, b = v;
+        plswap<false>(a, b);
+        v = a * b;
+    }
+    if constexpr (W >= 64) {
+        double a = v, b = v;
+        plswap<true>(a, b);
+        v = a * b;
+    }
+    return v;
+}
+
 // K = 8, 16 or 32 wave sums at once (a transposed reduction).  On return
 // lane L holds the sum over all 64 lanes of v[L / (64 / K)].  Each step pairs
 // lanes that differ in one lane bit and halves the values every lane holds:

@@ -33,7 +33,10 @@ struct est_args {
     int* cnum;                // Ns: changed connections per sample
     void* cwd;                // 2 Ns T: sum of the unchanged connections' mels
     int waves;                // waves per workgroup, 4 or 8 (0: 8 while the LDS allows two workgroups per CU)
+    int ratio;                // FP64 walk and forces: the factor tables fit in LDS (nq_est_tables)
 };
+// sets a.ratio for the launch a describes
+void nq_est_tables(est_args& a, bool fp64);
 size_t est_lds_bytes(const est_args& a, size_t elt, int waves);
 hipError_t nq_launch_estimate(const est_args& a, bool fp64, int grid, hipStream_t st);
 

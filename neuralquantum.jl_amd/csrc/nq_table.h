@@ -21,6 +21,7 @@ struct dev_table {
     // nsites_r << 16, row base of op_l, row base of op_r, 0, the sites of
     // op_l as bytes (2 words), those of op_r (2 words)
     const uint32_t* term_desc;
+    int fmax;                    // most sites one connection flips, both sides together
     int emax;                    // most connections one term yields (row entries, or their product)
 };
 

@@ -773,7 +773,13 @@ static nqh_status upload_table(nqh_ctx* c, const nqh_optable* t, bool ket_as_row
     const uint64_t lim = (N >= 64) ? ~0ull : ((1ull << N) - 1);
     for (int e = 0; e < t->n_entries; ++e)
         if (t->ent_flip[e] & ~lim) return fail(c, NQH_E_ARG, "flip mask beyond n_sites");
-    int maxc = 0, n_ket = 0, emax = 0;
+    int maxc = 0, n_ket = 0, emax = 0, fmax = 0;
+    auto maxflip = [&](int o) {
+        int m = 0;
+        for (int e = t->row_ent_off[t->op_row_off[o]]; e < t->row_ent_off[t->op_row_off[o + 1]]; ++e)
+            m = std::max(m, __builtin_popcountll(t->ent_flip[e]));
+        return m;
+    };
     for (int q = 0; q < t->n_terms; ++q) n_ket += t->term_kind[q] == 3;
     if (n_ket != 0 && n_ket != t->n_terms)
         return fail(c, NQH_E_ARG, "ket terms (kind 3) cannot be mixed with row/column terms");
@@ -795,6 +801,7 @@ static nqh_status upload_table(nqh_ctx* c, const nqh_optable* t, bool ket_as_row
         } else return fail(c, NQH_E_ARG, "bad term kind");
         maxc += e;
         emax = std::max(emax, e);
+        fmax = std::max(fmax, (k != 1 ? maxflip(ol) : 0) + (k == 1 || k == 2 ? maxflip(orr) : 0));
     }
     // one device allocation: int32 arrays, then doubles, floats, flips
     const size_t ni = (size_t)3 * t->n_terms + (t->n_ops + 1) + nsites_total + (t->n_ops + 1) + (t->n_rows + 1);
@@ -864,6 +871,7 @@ static nqh_status upload_table(nqh_ctx* c, const nqh_optable* t, bool ket_as_row
     tab.bytes = (int)host.size();
     tab.term_desc = reinterpret_cast<const uint32_t*>(base + bytes_tab);
     tab.emax = emax;
+    tab.fmax = fmax;
     *maxc_out = maxc;
     *nket_out = n_ket;
     return NQH_OK;
@@ -2398,10 +2406,12 @@ nq_pk_member pk_describe(nqh_ctx* c, double eps, int kind, double lr) {
     m.ew.rec_mode = 1;
     m.ew.lp = c->lp.p;
     m.ew.Y = c->Y.p;
+    nq_est_tables(m.ew, f64);
     m.ef = e;
     m.ef.rec_mode = 2;
     m.ef.tab_lds = 0;   // the records replace the walk
     m.ef.Fpart = P<double>(c->Fpart);
+    nq_est_tables(m.ef, f64);
     m.est_grid = c->est_grid;
     m.force_grid = force_grid_of(c, Ns);
     m.fp64 = f64 ? 1 : 0;

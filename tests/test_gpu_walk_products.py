@@ -1,0 +1,42 @@
+"""The FP64 walk by products of the units' factors against the oracle at the
+edges of its tiles (16 units), both activations, and where the weights leave
+the products' range (the sums of f): log rho, L_loc and, through the gradient,
+the recorded connections.  1e-10 relative, the bar of the FP64 path."""
+import numpy as np
+import pytest
+
+from _helpers import ising, params, random_keys, rel_err, xyz
+from nqhip import Context, _lib
+from oracle import nqref
+
+pytestmark = pytest.mark.gpu
+
+# (model, N, nh, na, sigma): one unit, full and ragged tiles, both unit rows (2 nh > 64), and a range
+# beyond e^(+-600) (sigma 4 at 64 units: a site's sum over the units is about 2 x 0.8 sigma (2 nh + na))
+SHAPES = [("ising", 2, 1, 1, 0.5), ("ising", 5, 15, 16, 0.3), ("ising", 5, 16, 17, 0.3), ("xyz", 4, 17, 15, 0.3),
+          ("xyz", 6, 32, 33, 0.2), ("ising", 4, 33, 31, 0.2), ("xyz", 6, 64, 64, 0.1), ("ising", 3, 64, 48, 4.0)]
+
+
+@pytest.mark.parametrize("act", [0, 1])
+@pytest.mark.parametrize("model,N,nh,na,sigma", SHAPES)
+def test_walk_matches_the_oracle(gpu_ok, act, model, N, nh, na, sigma):
+    ref = nqref.Ref(act=act)
+    flat, tab, _ = xyz(2, N // 2) if model == "xyz" else ising(N)
+    p = params(ref.ndm_np(N, nh, na), seed=nh + 3 * na, sigma=sigma)
+    ctx = Context(0, 1)
+    ctx.set_problem(flat)
+    ctx.set_ndm(N, nh, na, act)
+    ctx.set_params(p)
+    ctx.set_precision(_lib.PREC_FP64, _lib.PREC_FP64)
+    chains, length = 9, 5
+    keys = random_keys(N, chains * length, seed=7)
+    L = ctx.local_estimator(keys)
+    L_r, dL_r = ref.local_estimator(tab, nh, na, p, keys)
+    assert rel_err(L, L_r) < 1e-10
+    st, _, F, _ = ctx.grad_from_samples(keys, chains, length)
+    _, O_r = ref.logpsi_grad(N, nh, na, p, keys)
+    _, F_r, _, st_r = ref.grad_step(chains, length, O_r, L_r, dL_r)
+    assert rel_err(st, st_r) < 1e-10
+    if np.max(np.abs(F_r)) < 2.0 ** 30:   # the exact force sums take addends below 2^30 (NaN beyond, as sigma 4 is)
+        assert rel_err(F, F_r) < 1e-10
+    ctx.close()
