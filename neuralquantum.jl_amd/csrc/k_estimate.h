@@ -17,7 +17,7 @@
 // effective angles theta = h + W x of the sample live in registers; a
 // connection flipping k sites costs k FMAs per unit.
 //
-// Three kinds of launch (template parameter KIND):
+// Three kinds of launch (template parameter KIND, and the forces):
 //   EK_WALK   log rho, O rows, and pass 1 over the connections: FP64 by
 //             products of the units' factors, FP32 (and FP64 weights outside
 //             their range) by softplus (or logcosh) of the changed angles +
@@ -25,18 +25,12 @@
 //             = mel_c exp(log rho_c - log rho_s), L_loc = sum_c W_c; with
 //             rec_mode 1 it writes per sample the changed connections (W_c,
 //             flip masks), their count and the unchanged connections' mel sum.
-//   EK_FORCE  reads those records and L_loc and adds the force
-//             Re(V W_c O_k(c)), V = conj(L_loc)/Ns.  FP32 network: the
-//             products on the matrix cores (force_mma_body, k_force_mma,
-//             below).  FP64: per unit a dense part (x_s times a per-unit
-//             scalar) plus a sparse part on the flipped sites only (x_c =
-//             x_s + Delta_c); each lane sums its units' entries of one sample
-//             in registers (the flipped site indexes a register vector with a
-//             wave-uniform index: VGPR index mode), then adds them once per
-//             sample into the workgroup's force accumulator in LDS, held as
-//             exact 64-bit fixed-point integers (fx_add), so the sum is the
-//             same whatever order the waves arrive in.  The per-workgroup
-//             partials are then summed in a fixed order.
+//   forces    (force_mma_body, force64_body below) read those records and
+//             L_loc and add the force Re(V W_c O_k(c)), V = conj(L_loc)/Ns, by
+//             products on the matrix cores; a workgroup's sums are held as
+//             exact 64-bit fixed-point integers in LDS (fx_add), so they are
+//             the same whatever order the waves arrive in, and the
+//             per-workgroup partials are then summed in a fixed order.
 //   EK_GRAD   the parity mode: everything for one sample per wavefront and the
 //             per-sample dL_loc(s) written out (the force pass run with V = 1
 //             and V = -i for its real and imaginary parts).
@@ -47,7 +41,7 @@
 
 namespace nq_est {
 
-enum { EK_WALK = 0, EK_FORCE = 1, EK_GRAD = 2 };
+enum { EK_WALK = 0, EK_GRAD = 1 };
 
 template <typename T>
 __device__ __forceinline__ T xv(uint32_t bits, int i) { return ((bits >> i) & 1u) ? T(1) : T(-1); }
@@ -185,7 +179,7 @@ __device__ __forceinline__ bool ratio_fill(const ratio_tables& t, const double* 
 template <typename T, int NMAX, int RS, int PS, bool TAB_LDS, int KIND, int ACT>
 __device__ __forceinline__ void estimate_body(const est_args& a, int bx, int gx) {
     extern __shared__ __align__(16) unsigned char smem[];
-    constexpr bool WALK = KIND == EK_WALK, FORCE = KIND == EK_FORCE, GRAD = KIND == EK_GRAD;
+    constexpr bool WALK = KIND == EK_WALK, GRAD = KIND == EK_GRAD;
     using vN = T __attribute__((ext_vector_type(NMAX)));
     const ndm_dims d = a.d;
     const int N = d.N, nh = d.nh, na = d.na;
@@ -242,7 +236,7 @@ __device__ __forceinline__ void estimate_body(const est_args& a, int bx, int gx)
         const uint32_t ks = (uint32_t)key & pmask;
         const uint32_t ke = (uint32_t)(key >> N) & pmask;
 
-        // ---- effective angles of the sample (the forces need only f')
+        // ---- effective angles of the sample
         T th_s[RS], th_e[RS], f_s[RS], f_e[RS], a_s[RS], a_e[RS];
 #pragma unroll
         for (int r = 0; r < RS; ++r) {
@@ -262,13 +256,8 @@ __device__ __forceinline__ void estimate_body(const est_args& a, int bx, int gx)
                     }
                 }
                 th_s[r] = ts; th_e[r] = te;
-                if constexpr (FORCE) {
-                    a_s[r] = act_df<ACT>(ts);
-                    a_e[r] = act_df<ACT>(te);
-                } else {
-                    act_f_df<ACT>(ts, &f_s[r], &a_s[r]);
-                    act_f_df<ACT>(te, &f_e[r], &a_e[r]);
-                }
+                act_f_df<ACT>(ts, &f_s[r], &a_s[r]);
+                act_f_df<ACT>(te, &f_e[r], &a_e[r]);
             }
         }
         cplx<T> pi_z[PS], pi_f[PS], pi_p[PS];
@@ -288,12 +277,11 @@ __device__ __forceinline__ void estimate_body(const est_args& a, int bx, int gx)
                     }
                 }
                 pi_z[r] = cmk(zr, zi);
-                if constexpr (FORCE) pi_p[r] = cact_df<ACT>(pi_z[r]);
-                else cact_f_df<ACT>(pi_z[r], &pi_f[r], &pi_p[r]);
+                cact_f_df<ACT>(pi_z[r], &pi_f[r], &pi_p[r]);
             }
         }
 
-        if constexpr (!FORCE) {
+        {
             // ---- log rho(s) = Gamma_la + i Gamma_mu + Pi
             {
                 T re = T(0), im = T(0);
@@ -379,21 +367,7 @@ __device__ __forceinline__ void estimate_body(const est_args& a, int bx, int gx)
 
         int ncc;
         cplx<T> Wdiag, Lloc;
-        if constexpr (FORCE) {
-            // the connections of pass 1 from the walk launch
-            const int64_t rb = s * (int64_t)a.max_conn;
-            ncc = a.cnum[s];
-            const T* wd = reinterpret_cast<const T*>(a.cwd) + 2 * s;
-            const T* ll = reinterpret_cast<const T*>(a.Lloc) + 2 * s;
-            Wdiag = cmk(wd[0], wd[1]);
-            Lloc = cmk(ll[0], ll[1]);
-            const cplx<T>* rw = reinterpret_cast<const cplx<T>*>(a.crw) + rb;
-            for (int c = lane0; c < ncc; c += 64) {
-                wbuf[c] = rw[c];
-                mbuf[c] = a.crm[rb + c];
-            }
-            __builtin_amdgcn_wave_barrier();
-        } else {
+        {
             // ---- pass 1: W_c and L_loc.  The walk (terms spread over the
             // lanes) sums the unchanged connections (W = mel) per lane and
             // caches the changed ones (mel, flip masks) in LDS; those are then
@@ -849,16 +823,13 @@ __device__ __forceinline__ void estimate_body(const est_args& a, int bx, int gx)
                 }
             }
         }
-        if constexpr (!WALK) {
-            // ---- force pass: Re(V W_c O_k(c)) summed over the connections of
-            // this sample in registers, then added to the workgroup's exact
-            // accumulator once
+        if constexpr (GRAD) {
+            // ---- the parity mode's force pass: Re(V W_c O_k(c)) summed over the connections of
+            // this sample in registers, then through the exact accumulator
             constexpr bool PAIR_PI = PS == 1 && sizeof(T) == 4;
-            constexpr int NV = GRAD ? 2 : 1;
-            for (int vi = 0; vi < NV; ++vi) {
+            for (int vi = 0; vi < 2; ++vi) {
                 // Re(1 G) = Re G, Re(-i G) = Im G in the parity mode
-                const cplx<double> Vd = GRAD ? (vi == 0 ? cmk(1.0, 0.0) : cmk(0.0, -1.0))
-                                             : cmk((double)Lloc.re * a.invNs, -(double)Lloc.im * a.invNs);
+                const cplx<double> Vd = vi == 0 ? cmk(1.0, 0.0) : cmk(0.0, -1.0);
                 const cplx<T> V = cmk((T)Vd.re, (T)Vd.im);
                 // per unit: weights of the dense part (e_s, e_e, rho1, rho2) and the
                 // flipped-site shares (fw: w entries of the lambda / mu unit; fur,
@@ -1103,13 +1074,6 @@ __device__ __forceinline__ void estimate_body(const est_args& a, int bx, int gx)
                 }
             }
         }
-    }
-
-    if constexpr (FORCE) {
-        __syncthreads();
-        double* out = a.Fpart + (int64_t)bx * d.np;
-        const bool bad = *poison != 0;
-        for (int k = threadIdx.x; k < d.np; k += blockDim.x) out[k] = bad ? __builtin_nan("") : fx_value(sF, k);
     }
 }
 
@@ -1470,6 +1434,372 @@ __global__ __launch_bounds__(512, CLS < 2 ? 4 : 2) void k_force_mma_pk(const nq_
     force_mma_body<NMAX, CLS, ACT>(m.ef, (int)(b.y & 0xffff), m.force_grid);
 }
 
+// ---- the forces launch of the FP64 network: the same products on v_mfma_f64_16x16x4f64
+// f' at a connection's angles from the kept factors: E' = E e^(+-2 K w) per flipped site, f' =
+// E' / (1 + E') (softplus) or (E' - 1) / (E' + 1) (logcosh), the Pi units likewise in complex numbers;
+// from the angles themselves where the weights leave the range or the tables do not fit.  Per four
+// connections 12 products of 64 cycles against about 170 VALU instructions, on different pipes.  The
+// form it replaces, one unit per lane with the flipped site indexing a register vector and exp, sincos
+// and divides per unit, took 0.97 ms alone on the trained-chain 4x4 XYZ workload of 16384 samples and 2.2 ms beside the S
+// build; this one 0.36 both ways (12 sites: 0.6 -> 0.16).
+//   LDS: HW [N + 1][SW], PU [N][SP], PD [SP] as above in double, then up, dn [N][SW], pup, pdn [N][SP]
+typedef double d4v __attribute__((ext_vector_type(4)));
+
+// doubles of the staged parameters and of the factor tables
+__host__ __device__ inline int force64_stage_doubles(const ndm_dims& d, bool ratio) {
+    const int c = force_class(d) < 0 ? 2 : force_class(d);
+    const int sw = 32 << c, sp = 16 << c;
+    return sw * (d.N + 1) + sp * (2 * d.N + 1) + (ratio ? 2 * d.N * (sw + 2 * sp) : 0);
+}
+
+// 1 / x for normal x of moderate size: v_rcp_f64 and two Newton steps (1 ulp)
+__device__ __forceinline__ double rcp_newton(double x) {
+    double r = __builtin_amdgcn_rcp(x);
+    r = fma(fma(-x, r, 1.0), r, r);
+    return fma(fma(-x, r, 1.0), r, r);
+}
+
+template <int NMAX, int CLS, int ACT, bool RATIO>
+__device__ __forceinline__ void force64_samples(const est_args& a, int64_t gw, int64_t nw, const double* HW,
+                                                const double2* PU, const double* PD, const double* up,
+                                                const double* dn, const double2* pup, const double2* pdn,
+                                                cplx<double>* wbuf, uint2* mbuf, unsigned long long* sF, int* poison) {
+    constexpr int TW = 2 << CLS, TP = 1 << CLS, SW = 16 * TW, SP = 16 * TP, RS = (SW + 63) / 64;
+    constexpr double K = ACT == NQ_ACT_LOGCOSH ? 2.0 : 1.0;
+    const ndm_dims d = a.d;
+    const int N = d.N, nh = d.nh, na = d.na;
+    const int lane0 = threadIdx.x & 63;
+    const uint32_t pmask = (N >= 32) ? 0xffffffffu : ((1u << N) - 1u);
+    // f' of a real unit from its kept value (the factor e^(K x), or x), and of a Pi unit
+    auto df = [](double v) {
+        if constexpr (!RATIO) return act_df<ACT>(v);
+        else if constexpr (ACT == NQ_ACT_LOGCOSH) return (v - 1.0) * rcp_newton(v + 1.0);
+        else return v * rcp_newton(1.0 + v);
+    };
+    auto cdf = [](cplx<double> v) {
+        if constexpr (!RATIO) {
+            return cact_df<ACT>(v);
+        } else {
+            const double dr = 1.0 + v.re, den = rcp_newton(dr * dr + v.im * v.im);
+            if constexpr (ACT == NQ_ACT_LOGCOSH)
+                return cmk(((v.re - 1.0) * dr + v.im * v.im) * den, 2.0 * v.im * den);
+            else
+                return cmk((v.re * dr + v.im * v.im) * den, v.im * den);
+        }
+    };
+
+    d4v Fw[TW], Fr[TP], Fi[TP];
+    double hb[TW], db[TP], vbl = 0.0, vbm = 0.0;
+    const d4v zero = d4v{0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+    for (int t = 0; t < TW; ++t) { Fw[t] = zero; hb[t] = 0.0; }
+#pragma unroll
+    for (int t = 0; t < TP; ++t) { Fr[t] = Fi[t] = zero; db[t] = 0.0; }
+
+    int nacc = 0;
+    for (int64_t s = gw; s < a.Ns; s += nw) {
+        int lane = lane0;
+        asm volatile("" : "+v"(lane));   // as in the walk
+        const int il = lane & 15, kg = lane >> 4;
+        const uint64_t key = a.keys[s];
+        const uint32_t ks = (uint32_t)key & pmask;
+        const uint32_t ke = (uint32_t)(key >> N) & pmask;
+
+        // the sample's angles (factors), one unit per lane, then in the product layout
+        double ts1[RS], te1[RS];
+#pragma unroll
+        for (int r = 0; r < RS; ++r) {
+            const int u = lane + 64 * r;
+            double ts = 0.0, te = 0.0;
+            if (u < SW) {
+                ts = te = HW[u];
+#pragma unroll
+                for (int i = 0; i < NMAX; ++i) {
+                    if (i < N) {
+                        const double wi = HW[SW * (1 + i) + u];
+                        ts += wi * xv<double>(ks, i);
+                        te += wi * xv<double>(ke, i);
+                    }
+                }
+            }
+            ts1[r] = RATIO ? exp(K * ts) : ts;
+            te1[r] = RATIO ? exp(K * te) : te;
+        }
+        cplx<double> pz1 = cmk(0.0, 0.0);
+        if (lane < SP) {
+            double zr = PD[lane], zi = 0.0;
+#pragma unroll
+            for (int i = 0; i < NMAX; ++i) {
+                if (i < N) {
+                    const double xs = xv<double>(ks, i), xe = xv<double>(ke, i);
+                    const double2 uu = PU[SP * i + lane];
+                    zr += 0.5 * uu.x * (xs + xe);
+                    zi += 0.5 * uu.y * (xs - xe);
+                }
+            }
+            pz1 = cmk(zr, zi);
+            if constexpr (RATIO) {
+                double sn, cs;
+                sincos(K * zi, &sn, &cs);
+                const double e = exp(K * zr);
+                pz1 = cmk(e * cs, e * sn);
+            }
+        }
+        double ths[TW], the[TW];
+#pragma unroll
+        for (int t = 0; t < TW; ++t) {
+            const int src = 16 * (t & 3) + il, r = t >> 2;
+            ths[t] = __shfl(ts1[r], src, 64);
+            the[t] = __shfl(te1[r], src, 64);
+        }
+        cplx<double> pz[TP];
+#pragma unroll
+        for (int t = 0; t < TP; ++t) pz[t] = cmk(__shfl(pz1.re, 16 * t + il, 64), __shfl(pz1.im, 16 * t + il, 64));
+
+        if (a.do_conn) {
+            // the connections of pass 1 from the walk launch
+            const int64_t rb = s * (int64_t)a.max_conn;
+            const int ncc = a.cnum[s];
+            const double* wd = reinterpret_cast<const double*>(a.cwd) + 2 * s;
+            const double* ll = reinterpret_cast<const double*>(a.Lloc) + 2 * s;
+            const cplx<double> Wdiag = cmk(wd[0], wd[1]);
+            const cplx<double> V = cmk(ll[0] * a.invNs, -ll[1] * a.invNs);
+            const cplx<double>* rw = reinterpret_cast<const cplx<double>*>(a.crw) + rb;
+            for (int c = lane0; c < ncc; c += 64) {
+                wbuf[c] = rw[c];
+                mbuf[c] = a.crm[rb + c];
+            }
+            __builtin_amdgcn_wave_barrier();
+
+            // four connections per round; index ncc is the unchanged configurations
+            for (int c0 = 0; c0 <= ncc; c0 += 4) {
+                const int c = c0 + kg;
+                cplx<double> W = cmk(0.0, 0.0);
+                uint32_t ms = 0u, me = 0u;
+                if (c < ncc) {
+                    W = wbuf[c];
+                    const uint2 mm = mbuf[c];
+                    ms = mm.x;
+                    me = mm.y;
+                } else if (c == ncc) {
+                    W = Wdiag;
+                }
+                const cplx<double> VW = cmul(V, W);
+                double ts[TW], te[TW];
+                cplx<double> z[TP];
+#pragma unroll
+                for (int t = 0; t < TW; ++t) { ts[t] = ths[t]; te[t] = the[t]; }
+#pragma unroll
+                for (int t = 0; t < TP; ++t) z[t] = pz[t];
+                auto side = [&](uint32_t m, uint32_t kk, double (&v)[TW], double sgn) {
+                    for (; m; m &= m - 1) {
+                        const int i = __builtin_ctz(m);
+                        if constexpr (RATIO) {
+                            const bool down = ((kk >> i) & 1u) != 0;
+                            const double* tb = (down ? dn : up) + SW * i + il;
+                            const double2* tc = (down ? pdn : pup) + SP * i + il;
+#pragma unroll
+                            for (int t = 0; t < TW; ++t) v[t] *= tb[16 * t];
+#pragma unroll
+                            for (int t = 0; t < TP; ++t) {
+                                const double2 f = tc[16 * t];
+                                z[t] = cmul(z[t], cmk(f.x, sgn * f.y));
+                            }
+                        } else {
+                            const double cf = cflip<double>(kk, i), cc = 0.5 * cf;
+#pragma unroll
+                            for (int t = 0; t < TW; ++t) v[t] += cf * HW[SW * (1 + i) + 16 * t + il];
+#pragma unroll
+                            for (int t = 0; t < TP; ++t) {
+                                const double2 uu = PU[SP * i + 16 * t + il];
+                                z[t].re += cc * uu.x;
+                                z[t].im += sgn * cc * uu.y;
+                            }
+                        }
+                    }
+                };
+                side(ms, ks, ts, 1.0);
+                side(me, ke, te, -1.0);
+                const double gl = 0.5 * VW.re, gm = -0.5 * VW.im;
+                const bool sok = il < N;
+                const double Bs = sok ? xv<double>(ks ^ ms, il) : 0.0, Be = sok ? xv<double>(ke ^ me, il) : 0.0;
+#pragma unroll
+                for (int t = 0; t < TW; ++t) {
+                    const int u = 16 * t + il;
+                    const double gs = u < nh ? gl : (u < 2 * nh ? gm : 0.0);
+                    const double ge = u < nh ? gl : -gs;
+                    const double xa = gs * df(ts[t]), ya = ge * df(te[t]);
+                    hb[t] += xa + ya;
+                    Fw[t] = __builtin_amdgcn_mfma_f64_16x16x4f64(xa, Bs, Fw[t], 0, 0, 0);
+                    Fw[t] = __builtin_amdgcn_mfma_f64_16x16x4f64(ya, Be, Fw[t], 0, 0, 0);
+                }
+                const double Bp = 0.5 * (Bs + Be), Bm = 0.5 * (Bs - Be);
+#pragma unroll
+                for (int t = 0; t < TP; ++t) {
+                    const cplx<double> vp = cmul(VW, cdf(z[t]));
+                    const bool ok = 16 * t + il < na;
+                    const double ar = ok ? vp.re : 0.0, ai = ok ? -vp.im : 0.0;
+                    db[t] += ar;
+                    Fr[t] = __builtin_amdgcn_mfma_f64_16x16x4f64(ar, Bp, Fr[t], 0, 0, 0);
+                    Fi[t] = __builtin_amdgcn_mfma_f64_16x16x4f64(ai, Bm, Fi[t], 0, 0, 0);
+                }
+                vbl += VW.re * Bp;
+                vbm -= VW.im * Bm;
+            }
+        }
+
+        // every kForceFlush samples and after the wave's last one into the exact accumulator: product
+        // entry (row lane / 16 + 4 v, column lane % 16) of each tile, the bias sums over the four groups
+        if (++nacc == kForceFlush || s + nw >= a.Ns) {
+            nacc = 0;
+            const int PB_bla = 0, PB_hla = N, PB_wla = N + nh;
+            const int PB_d = d.nlam, PB_ula = d.nlam + na, PB_umu = d.nlam + na + na * N;
+            const int PB_bmu = d.nlam + d.npi, PB_hmu = PB_bmu + N, PB_wmu = PB_hmu + nh;
+#pragma unroll
+            for (int t = 0; t < TW; ++t) {
+                if (16 * t < 2 * nh) {
+#pragma unroll
+                    for (int v = 0; v < 4; ++v) {
+                        const int u = 16 * t + kg + 4 * v;
+                        if (u < 2 * nh && il < N)
+                            fx_add(sF, (u < nh ? PB_wla + u : PB_wmu + u - nh) + nh * il, Fw[t][v], poison);
+                    }
+                    double h = hb[t];
+                    h += __shfl_xor(h, 16, 64);
+                    h += __shfl_xor(h, 32, 64);
+                    const int u = 16 * t + il;
+                    if (kg == 0 && u < 2 * nh) fx_add(sF, u < nh ? PB_hla + u : PB_hmu + u - nh, h, poison);
+                }
+                Fw[t] = zero;
+                hb[t] = 0.0;
+            }
+#pragma unroll
+            for (int t = 0; t < TP; ++t) {
+                if (16 * t < na) {
+#pragma unroll
+                    for (int v = 0; v < 4; ++v) {
+                        const int au = 16 * t + kg + 4 * v;
+                        if (au < na && il < N) {
+                            fx_add(sF, PB_ula + au + na * il, Fr[t][v], poison);
+                            fx_add(sF, PB_umu + au + na * il, Fi[t][v], poison);
+                        }
+                    }
+                    double h = db[t];
+                    h += __shfl_xor(h, 16, 64);
+                    h += __shfl_xor(h, 32, 64);
+                    if (kg == 0 && 16 * t + il < na) fx_add(sF, PB_d + 16 * t + il, h, poison);
+                }
+                Fr[t] = Fi[t] = zero;
+                db[t] = 0.0;
+            }
+            double bl = vbl, bm = vbm;
+            bl += __shfl_xor(bl, 16, 64);
+            bl += __shfl_xor(bl, 32, 64);
+            bm += __shfl_xor(bm, 16, 64);
+            bm += __shfl_xor(bm, 32, 64);
+            if (kg == 0 && il < N) {
+                fx_add(sF, PB_bla + il, bl, poison);
+                fx_add(sF, PB_bmu + il, bm, poison);
+            }
+            vbl = vbm = 0.0;
+        }
+    }
+}
+
+template <int NMAX, int CLS, int ACT>
+__device__ __forceinline__ void force64_body(const est_args& a, int bx, int gx) {
+    static_assert(NMAX <= 16, "the sites fill one 16-column tile");
+    constexpr int SW = 32 << CLS, SP = 16 << CLS;
+    constexpr double K = ACT == NQ_ACT_LOGCOSH ? 2.0 : 1.0;
+    extern __shared__ __align__(16) unsigned char smem[];
+    const ndm_dims d = a.d;
+    const int N = d.N, nh = d.nh, na = d.na;
+    // the complex tables first: 16-byte entries
+    double2* PU = reinterpret_cast<double2*>(smem);
+    double2* pup = PU + SP * N;
+    double2* pdn = pup + (a.ratio ? SP * N : 0);
+    double* HW = reinterpret_cast<double*>(pdn + (a.ratio ? SP * N : 0));
+    double* PD = HW + SW * (N + 1);
+    double* up = PD + SP;
+    double* dn = up + (a.ratio ? SW * N : 0);
+    const int pbytes = (8 * force64_stage_doubles(d, a.ratio != 0) + 15) & ~15;
+    unsigned long long* sF = reinterpret_cast<unsigned long long*>(smem + pbytes);
+    int* poison = reinterpret_cast<int*>(sF + 2 * d.np);
+    int* out_of_range = poison + 1;   // the accumulator's last 16 bytes hold both
+    cplx<double>* sW = reinterpret_cast<cplx<double>*>(smem + pbytes + fx_bytes(d.np));
+    const int wpb = blockDim.x >> 6;
+    uint2* sM = reinterpret_cast<uint2*>(sW + wpb * a.max_conn);
+    const double* gp = reinterpret_cast<const double*>(a.p);
+    for (int k = threadIdx.x; k < SW * (N + 1); k += blockDim.x) {
+        const int r = k / SW, u = k - r * SW;
+        const int src = u < nh ? (r == 0 ? d.hla + u : d.wla + u + nh * (r - 1))
+                               : (r == 0 ? d.hmu + u - nh : d.wmu + u - nh + nh * (r - 1));
+        const double w = u < 2 * nh ? gp[src] : 0.0;
+        HW[k] = w;
+        if (a.ratio && r > 0) {
+            const double e = exp(2.0 * K * w);
+            up[k - SW] = e;
+            dn[k - SW] = 1.0 / e;
+        }
+    }
+    for (int k = threadIdx.x; k < SP * N; k += blockDim.x) {
+        const int i = k / SP, au = k - i * SP;
+        const bool ok = au < na;
+        const double ul = ok ? gp[d.ula + au + na * i] : 0.0, um = ok ? gp[d.umu + au + na * i] : 0.0;
+        PU[k] = make_double2(ul, um);
+        if (a.ratio) {
+            double sn, cs;
+            sincos(K * um, &sn, &cs);
+            const double e = exp(K * ul), r = 1.0 / e;
+            pup[k] = make_double2(e * cs, e * sn);
+            pdn[k] = make_double2(r * cs, -r * sn);
+        }
+    }
+    for (int k = threadIdx.x; k < SP; k += blockDim.x) PD[k] = k < na ? gp[d.dla + k] : 0.0;
+    for (int k = threadIdx.x; k < 2 * d.np; k += blockDim.x) sF[k] = 0ull;
+    if (threadIdx.x == 0) {
+        *poison = 0;
+        *out_of_range = 0;
+    }
+    __syncthreads();
+    // the largest |K theta| a unit reaches bounds its factors and |1 + w|^2
+    if (a.ratio) {
+        for (int u = threadIdx.x; u < SW + SP; u += blockDim.x) {
+            double m = fabs(u < SW ? HW[u] : PD[u - SW]);
+            for (int i = 0; i < N; ++i) m += fabs(u < SW ? HW[SW * (1 + i) + u] : PU[SP * i + u - SW].x);
+            if (!(K * m <= 0.5 * kEstRange)) atomicOr(out_of_range, 1);
+        }
+        __syncthreads();
+    }
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int64_t gw = (int64_t)bx * wpb + wave, nw = (int64_t)gx * wpb;
+    cplx<double>* wbuf = sW + wave * a.max_conn;
+    uint2* mbuf = sM + wave * a.max_conn;
+    const bool ratio = a.ratio && !__builtin_amdgcn_readfirstlane(*out_of_range);
+    if (ratio) force64_samples<NMAX, CLS, ACT, true>(a, gw, nw, HW, PU, PD, up, dn, pup, pdn, wbuf, mbuf, sF, poison);
+    else force64_samples<NMAX, CLS, ACT, false>(a, gw, nw, HW, PU, PD, up, dn, pup, pdn, wbuf, mbuf, sF, poison);
+
+    __syncthreads();
+    double* out = a.Fpart + (int64_t)bx * d.np;
+    const bool bad = *poison != 0;
+    for (int k = threadIdx.x; k < d.np; k += blockDim.x) out[k] = bad ? __builtin_nan("") : fx_value(sF, k);
+}
+
+// the FP64 forces launch of one tile class: one workgroup of 8 waves per CU, of 4 in class 2 (its
+// accumulators alone take 128 registers)
+#define NQ_F64_BOUNDS __launch_bounds__(CLS < 2 ? 512 : 256, CLS < 2 ? 2 : 1)
+template <int NMAX, int CLS, int ACT>
+__global__ NQ_F64_BOUNDS void k_force_mma64(est_args a) {
+    force64_body<NMAX, CLS, ACT>(a, blockIdx.x, gridDim.x);
+}
+template <int NMAX, int CLS, int ACT>
+__global__ NQ_F64_BOUNDS void k_force_mma64_pk(const nq_pk_member* M, const uint2* blk) {
+    const uint2 b = blk[blockIdx.x];
+    const nq_pk_member& m = M[b.x & 0xffff];
+    force64_body<NMAX, CLS, ACT>(m.ef, (int)(b.y & 0xffff), m.force_grid);
+}
+#undef NQ_F64_BOUNDS
+
 #define NQ_EST_BOUNDS __launch_bounds__(512, (sizeof(T) == 4 && RS == 1 && KIND != EK_GRAD) ? 4 : 2)
 
 template <typename T, int NMAX, int RS, int PS, bool TAB_LDS, int KIND, int ACT>
@@ -1477,14 +1807,13 @@ __global__ NQ_EST_BOUNDS void k_estimate(est_args a) {
     estimate_body<T, NMAX, RS, PS, TAB_LDS, KIND, ACT>(a, blockIdx.x, gridDim.x);
 }
 
-// packed: the members' walk (KIND = EK_WALK) or force launches in one grid
+// packed: the members' walk launches in one grid
 template <typename T, int NMAX, int RS, int PS, bool TAB_LDS, int KIND, int ACT>
 __global__ NQ_EST_BOUNDS void k_estimate_pk(const nq_pk_member* M, const uint2* blk) {
     const uint2 b = blk[blockIdx.x];
     const nq_pk_member& m = M[b.x & 0xffff];
-    const est_args a = KIND == EK_FORCE ? m.ef : m.ew;
-    estimate_body<T, NMAX, RS, PS, TAB_LDS, KIND, ACT>(a, (int)(b.y & 0xffff),
-                                                      KIND == EK_FORCE ? m.force_grid : m.est_grid);
+    const est_args a = m.ew;
+    estimate_body<T, NMAX, RS, PS, TAB_LDS, KIND, ACT>(a, (int)(b.y & 0xffff), m.est_grid);
 }
 #undef NQ_EST_BOUNDS
 
@@ -1495,35 +1824,36 @@ __global__ NQ_EST_BOUNDS void k_estimate_pk(const nq_pk_member* M, const uint2* 
 inline int est_waves(const est_args& a, size_t elt) {
     if (a.G) return 1;
     if (a.waves == 4) return 4;
+    if (elt == 8 && a.rec_mode == 2 && force_class(a.d) == 2) return 4;   // its launch bound
     if (a.waves == 8 && est_lds_bytes(a, elt, 8) <= 160 * 1024) return 8;
-    // FP64 by products: its registers leave two waves per SIMD anyway, so one workgroup of 8 per CU
-    return est_lds_bytes(a, elt, 8) > (elt == 8 && a.ratio ? 160 : 80) * 1024 ? 4 : 8;
+    // FP64 by products and the FP64 forces: their registers leave two waves per SIMD anyway, so one
+    // workgroup of 8 per CU
+    return est_lds_bytes(a, elt, 8) > (elt == 8 && (a.ratio || a.rec_mode == 2) ? 160 : 80) * 1024 ? 4 : 8;
 }
 
 template <typename T, int NMAX, int RS, int PS, int ACT>
 hipError_t launch_t(const est_args& a0, int grid, hipStream_t st) {
     est_args a = a0;
-    const int kind = a.G ? EK_GRAD : (a.rec_mode == 2 ? EK_FORCE : EK_WALK);
-    if (kind == EK_WALK && a.Fpart) return hipErrorInvalidValue;   // forces take a launch of their own
-    if (kind == EK_FORCE) a.tab_lds = 0;                             // the records replace the walk
+    const bool force = !a.G && a.rec_mode == 2;
+    if (!a.G && !force && a.Fpart) return hipErrorInvalidValue;   // forces take a launch of their own
+    if (force) a.tab_lds = 0;                                     // the records replace the walk
     const int wpb = est_waves(a, sizeof(T));
     const size_t lds = est_lds_bytes(a, sizeof(T), wpb);
-    if (kind == EK_FORCE) {
+    if (force) {
+        const int cls = force_class(a.d);
+        const dim3 g(grid), b(64 * wpb);
         if constexpr (sizeof(T) == 4) {
-            const int cls = force_class(a.d);
-            if (cls == 0)
-                hipLaunchKernelGGL((k_force_mma<NMAX, 0, ACT>), dim3(grid), dim3(64 * wpb), lds, st, a);
-            else if (cls == 1)
-                hipLaunchKernelGGL((k_force_mma<NMAX, 1, ACT>), dim3(grid), dim3(64 * wpb), lds, st, a);
-            else if (cls == 2)
-                hipLaunchKernelGGL((k_force_mma<NMAX, 2, ACT>), dim3(grid), dim3(64 * wpb), lds, st, a);
-            else
-                return hipErrorInvalidValue;
+            if (cls == 0) hipLaunchKernelGGL((k_force_mma<NMAX, 0, ACT>), g, b, lds, st, a);
+            else if (cls == 1) hipLaunchKernelGGL((k_force_mma<NMAX, 1, ACT>), g, b, lds, st, a);
+            else if (cls == 2) hipLaunchKernelGGL((k_force_mma<NMAX, 2, ACT>), g, b, lds, st, a);
+            else return hipErrorInvalidValue;
         } else {
-            hipLaunchKernelGGL((k_estimate<T, NMAX, RS, PS, false, EK_FORCE, ACT>), dim3(grid), dim3(64 * wpb), lds, st,
-                               a);
+            if (cls == 0) hipLaunchKernelGGL((k_force_mma64<NMAX, 0, ACT>), g, b, lds, st, a);
+            else if (cls == 1) hipLaunchKernelGGL((k_force_mma64<NMAX, 1, ACT>), g, b, lds, st, a);
+            else if (cls == 2) hipLaunchKernelGGL((k_force_mma64<NMAX, 2, ACT>), g, b, lds, st, a);
+            else return hipErrorInvalidValue;
         }
-    } else if (kind == EK_GRAD) {
+    } else if (a.G) {
         if (a.tab_lds)
             hipLaunchKernelGGL((k_estimate<T, NMAX, RS, PS, true, EK_GRAD, ACT>), dim3(grid), dim3(64), lds, st, a);
         else
@@ -1557,20 +1887,20 @@ hipError_t launch_prec(const est_args& a, int grid, hipStream_t st) {
 }
 
 // packed launches of one precision; variant bits: 0 force (else walk), 1 N > 8
-// (NMAX 16), 2 table in LDS, 3 logcosh, 5 tile class 0 of the FP32 forces
+// (NMAX 16), 2 table in LDS, 3 logcosh, 5 tile class 0 of the forces
 // (the walk and force kinds, one unit row and one Pi row per lane only)
 template <typename T, int NMAX, int ACT>
 hipError_t pk_launch_n(const nq_pk_member* M, const nq_pk_launch& L, hipStream_t st) {
     const dim3 g((unsigned)L.nblk), b((unsigned)L.threads);
     const bool force = (L.variant & 1) != 0, tl = (L.variant & 4) != 0;
     if (force) {
+        const bool c0 = (L.variant & 32) != 0;
         if constexpr (sizeof(T) == 4) {
-            if (L.variant & 32)
-                hipLaunchKernelGGL((k_force_mma_pk<NMAX, 0, ACT>), g, b, L.lds, st, M, L.blk);
-            else
-                hipLaunchKernelGGL((k_force_mma_pk<NMAX, 1, ACT>), g, b, L.lds, st, M, L.blk);
+            if (c0) hipLaunchKernelGGL((k_force_mma_pk<NMAX, 0, ACT>), g, b, L.lds, st, M, L.blk);
+            else hipLaunchKernelGGL((k_force_mma_pk<NMAX, 1, ACT>), g, b, L.lds, st, M, L.blk);
         } else {
-            hipLaunchKernelGGL((k_estimate_pk<T, NMAX, 1, 1, false, EK_FORCE, ACT>), g, b, L.lds, st, M, L.blk);
+            if (c0) hipLaunchKernelGGL((k_force_mma64_pk<NMAX, 0, ACT>), g, b, L.lds, st, M, L.blk);
+            else hipLaunchKernelGGL((k_force_mma64_pk<NMAX, 1, ACT>), g, b, L.lds, st, M, L.blk);
         }
     } else if (tl)
         hipLaunchKernelGGL((k_estimate_pk<T, NMAX, 1, 1, true, EK_WALK, ACT>), g, b, L.lds, st, M, L.blk);

@@ -10,15 +10,18 @@ size_t est_lds_bytes(const est_args& a, size_t elt, int waves) {
     size_t pb = (size_t)a.lds_param_bytes;
     if (elt == 4 && a.rec_mode == 2 && !a.G)
         pb = std::max(pb, ((size_t)4 * nq_est::force_stage_floats(a.d) + 15) & ~(size_t)15);
+    const bool f64_force = elt == 8 && a.rec_mode == 2 && !a.G;   // parameters and tables in its own layout
+    if (f64_force) pb = ((size_t)8 * nq_est::force64_stage_doubles(a.d, a.ratio != 0) + 15) & ~(size_t)15;
     const size_t b = pb + ((a.Fpart || a.G) ? (size_t)fx_bytes(a.d.np) : 0) +
-                     (elt == 8 && a.ratio ? (size_t)nq_est::ratio_bytes(a.d) : 0) +
+                     (elt == 8 && a.ratio && !f64_force ? (size_t)nq_est::ratio_bytes(a.d) : 0) +
                      (size_t)waves * (size_t)a.max_conn * (2 * elt + 8);
     return ((b + 15) & ~(size_t)15) + (a.tab_lds ? (size_t)a.tab.bytes : 0);
 }
 
 void nq_est_tables(est_args& a, bool fp64) {
     a.ratio = 0;
-    if (!fp64 || a.G || a.rec_mode == 2 || !a.do_conn) return;
+    if (!fp64 || a.G || !a.do_conn) return;
+    if (a.rec_mode == 2) a.tab_lds = 0;
     a.ratio = 1;
     if (est_lds_bytes(a, 8, 4) > 160 * 1024) a.ratio = 0;
 }
@@ -51,7 +54,7 @@ int nq_est_variant(const est_args& a0, bool fp64, int* threads, size_t* lds) {
     *lds = est_lds_bytes(a, elt, wpb);
     if (*lds > 160 * 1024) return -1;
     return (force ? 1 : 0) | (a.d.N > 8 ? 2 : 0) | (a.tab_lds ? 4 : 0) | (a.d.act == NQ_ACT_LOGCOSH ? 8 : 0) |
-           (fp64 ? 16 : 0) | (force && !fp64 && nq_est::force_class(a.d) == 0 ? 32 : 0);
+           (fp64 ? 16 : 0) | (force && nq_est::force_class(a.d) == 0 ? 32 : 0);
 }
 
 hipError_t nq_pk_estimate(const nq_pk_member* M, const nq_pk_launch& L, hipStream_t st) {

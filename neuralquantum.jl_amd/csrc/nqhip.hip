@@ -270,14 +270,13 @@ int est_grid_for(int64_t Ns, int spb = 0) {
 }
 
 // workgroups of the forces launch: from kSplitSamples samples on, where it
-// runs beside the S build, the FP32 network's matrix-core launch takes four
-// times the walk's samples per workgroup (staging, accumulator clear and
-// partial write amortised over more samples, fewer partials to sum, and more
-// of the GPU left to the S build); otherwise, and in FP64, the walk's grid.
-// A function of the batch alone, so that every path (graph, eager, profiled,
-// packed) sums the same partials
+// runs beside the S build, it takes four times the walk's samples per
+// workgroup (staging, accumulator clear and partial write amortised over more
+// samples, fewer partials to sum, and more of the GPU left to the S build);
+// otherwise the walk's grid.  A function of the batch alone, so that every
+// path (graph, eager, profiled, packed) sums the same partials
 int force_grid_of(const nqh_ctx* c, int64_t Ns) {
-    return (fp64_net(c) || Ns < kSplitSamples) ? c->est_grid : std::max(1, (c->est_grid + 3) / 4);
+    return Ns < kSplitSamples ? c->est_grid : std::max(1, (c->est_grid + 3) / 4);
 }
 
 // column-sum chunks of the NDM's O rows: 64 samples or more per chunk, at most kColChunks
