@@ -1170,9 +1170,25 @@ __device__ __forceinline__ void update_body(double* p64, float* p32, const doubl
     if (p32) p32[r] = (float)v;
 }
 
-__global__ void k_to_f32(const double* p64, float* p32, int64_t n) {
-    int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) p32[i] = (float)p64[i];
+// the parameters between pinned host memory and the device, one workgroup; `done` (pinned) takes the
+// transfer's number when all of it has been read (in) or written (out).  At the 17 KB of the 4x4 network
+// a copy through the runtime and the wait for it cost about 25 us in and 20 out; the caller of the first
+// does not wait (the next one does, for the staging buffer), that of the second polls `done`.
+__global__ __launch_bounds__(1024) void k_params_in(const double* host, double* p64, float* p32, int n, double* done,
+                                                    double seq) {
+    for (int k = threadIdx.x; k < n; k += blockDim.x) {
+        const double v = host[k];
+        p64[k] = v;
+        p32[k] = (float)v;
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) __hip_atomic_store(done, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+__global__ __launch_bounds__(1024) void k_params_out(const double* p64, double* host, int n, double* done, double seq) {
+    for (int k = threadIdx.x; k < n; k += blockDim.x) host[k] = p64[k];
+    __threadfence_system();
+    __syncthreads();
+    if (threadIdx.x == 0) __hip_atomic_store(done, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
 __device__ __forceinline__ void check_finite_body(const double* x, int64_t n, int* flag, int bx) {
@@ -1727,8 +1743,14 @@ hipError_t nq_launch_update(double* p64, float* p32, const double* delta, ndm_di
     return hipGetLastError();
 }
 
-hipError_t nq_launch_to_f32(const double* p64, float* p32, int64_t n, hipStream_t st) {
-    hipLaunchKernelGGL(k_to_f32, dim3(nblk(n, 256)), dim3(256), 0, st, p64, p32, n);
+hipError_t nq_launch_params_in(const double* host, double* p64, float* p32, int n, double* done, double seq,
+                               hipStream_t st) {
+    hipLaunchKernelGGL(k_params_in, dim3(1), dim3(1024), 0, st, host, p64, p32, n, done, seq);
+    return hipGetLastError();
+}
+
+hipError_t nq_launch_params_out(const double* p64, double* host, int n, double* done, double seq, hipStream_t st) {
+    hipLaunchKernelGGL(k_params_out, dim3(1), dim3(1024), 0, st, p64, host, n, done, seq);
     return hipGetLastError();
 }
 

@@ -222,7 +222,10 @@ hipError_t nq_split_tail(int nl, int npi, const double* x2, double* delta, int* 
                          const ndm_dims& d, double lr, const int* info, const double* stats, double* out,
                          hipStream_t st);
 // FP32 copy of the parameters
-hipError_t nq_launch_to_f32(const double* p64, float* p32, int64_t n, hipStream_t st);
+// parameters from / into pinned host memory; *done = seq when the transfer is complete
+hipError_t nq_launch_params_in(const double* host, double* p64, float* p32, int n, double* done, double seq,
+                               hipStream_t st);
+hipError_t nq_launch_params_out(const double* p64, double* host, int n, double* done, double seq, hipStream_t st);
 // NaN / Inf check: *flag |= 1 if any non-finite in x
 hipError_t nq_launch_check_finite(const double* x, int64_t n, int* flag, hipStream_t st);
 

@@ -3,6 +3,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <atomic>
 #include <cfloat>
 #include <chrono>
 #include <cmath>
@@ -50,6 +51,11 @@ struct nqh_ctx {
     ndm_dims d{};
     int rbm_N = 0, rbm_nh = 0, rbm_npc = 0;
     dbuf p64, p32;
+    // pinned staging of the parameters: [0] number of the last transfer completed, [1] unused, then the
+    // parameters; transfers are numbered, at most one is in flight
+    double* hpar = nullptr;
+    int hpar_cap = 0;
+    double hpar_seq = 0.0;
     int net_prec = NQH_PREC_FP64;
     int s_prec = NQH_PREC_FP64;
 
@@ -742,6 +748,7 @@ void nqh_destroy(nqh_ctx* c) {
     }
     (void)hipStreamDestroy(c->stream);
     if (c->hstat) (void)hipHostFree(c->hstat);
+    if (c->hpar) (void)hipHostFree(c->hpar);
     delete c;
 }
 
@@ -968,6 +975,42 @@ int64_t nqh_num_params(const nqh_ctx* c) { return (c && c->has_net) ? nsys(c) : 
 int64_t nqh_num_derivs(const nqh_ctx* c) { return (c && c->has_net) ? nderiv(c) : -1; }
 
 
+// the last parameter transfer is complete: a short spin on its number, then the stream's own wait
+// (which reports errors)
+static nqh_status param_wait(nqh_ctx* c) {
+    const volatile double* done = c->hpar;
+    const auto t0 = std::chrono::steady_clock::now();
+    while (*done != c->hpar_seq) {
+        if (std::chrono::steady_clock::now() - t0 > std::chrono::milliseconds(200)) {
+            HIPCHK(c, hipStreamSynchronize(c->stream));
+            break;
+        }
+        __builtin_ia32_pause();
+    }
+    std::atomic_thread_fence(std::memory_order_acquire);
+    return NQH_OK;
+}
+
+// the staging buffer, free of transfers in flight
+static nqh_status param_staging(nqh_ctx* c) {
+    const int n = nsys(c);
+    if (c->hpar) {
+        nqh_status s = param_wait(c);
+        if (s) return s;
+    }
+    if (c->hpar_cap >= n) return NQH_OK;
+    if (c->hpar) (void)hipHostFree(c->hpar);
+    c->hpar = nullptr;
+    c->hpar_cap = 0;
+    if (hipHostMalloc((void**)&c->hpar, sizeof(double) * (size_t)(n + 2), hipHostMallocCoherent) != hipSuccess) {
+        c->hpar = nullptr;
+        return fail(c, NQH_E_NOMEM, "hipHostMalloc of the parameter staging failed");
+    }
+    c->hpar_cap = n;
+    c->hpar[0] = c->hpar_seq;
+    return NQH_OK;
+}
+
 nqh_status nqh_set_params(nqh_ctx* c, const double* flat, int64_t np) {
     if (!c || !flat) return NQH_E_ARG;
     (void)hipSetDevice(c->device);
@@ -976,9 +1019,16 @@ nqh_status nqh_set_params(nqh_ctx* c, const double* flat, int64_t np) {
     if (np != nsys(c)) return fail(c, NQH_E_ARG, "parameter count mismatch");
     for (int64_t k = 0; k < np; ++k)
         if (!std::isfinite(flat[k])) return fail(c, NQH_E_NAN, "non-finite parameter");
-    HIPCHK(c, hipMemcpyAsync(c->p64.p, flat, sizeof(double) * np, hipMemcpyHostToDevice, c->stream));
-    HIPCHK(c, nq_launch_to_f32(P<double>(c->p64), P<float>(c->p32), np, c->stream));
-    HIPCHK(c, hipStreamSynchronize(c->stream));
+    // staged, so that `flat` is free at once, and read from there by a kernel on the context's stream
+    if ((s = param_staging(c))) return s;
+    std::memcpy(c->hpar + 2, flat, sizeof(double) * np);
+    c->hpar_seq += 1.0;
+    const hipError_t e = nq_launch_params_in(c->hpar + 2, P<double>(c->p64), P<float>(c->p32), (int)np, c->hpar,
+                                             c->hpar_seq, c->stream);
+    if (e != hipSuccess) {
+        c->hpar_seq -= 1.0;
+        return hip_fail(c, e, "nqh_set_params");
+    }
     return NQH_OK;
 }
 
@@ -989,8 +1039,15 @@ nqh_status nqh_get_params(const nqh_ctx* cc, double* flat, int64_t np) {
     nqh_status s = need_net(c);
     if (s) return s;
     if (np != nsys(c)) return fail(c, NQH_E_ARG, "parameter count mismatch");
-    HIPCHK(c, hipMemcpyAsync(flat, c->p64.p, sizeof(double) * np, hipMemcpyDeviceToHost, c->stream));
-    HIPCHK(c, hipStreamSynchronize(c->stream));
+    if ((s = param_staging(c))) return s;
+    c->hpar_seq += 1.0;
+    const hipError_t e = nq_launch_params_out(P<double>(c->p64), c->hpar + 2, (int)np, c->hpar, c->hpar_seq, c->stream);
+    if (e != hipSuccess) {
+        c->hpar_seq -= 1.0;
+        return hip_fail(c, e, "nqh_get_params");
+    }
+    if ((s = param_wait(c))) return s;
+    std::memcpy(flat, c->hpar + 2, sizeof(double) * np);
     return NQH_OK;
 }
 
