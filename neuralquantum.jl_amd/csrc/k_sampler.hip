@@ -7,18 +7,10 @@
 // proposal flips one uniformly chosen doubled site (LocalRule.jl:30-38) and is
 // rejected iff u - exp(log p' - log p) >= 0 (Metropolis.jl:148-154).
 //
-// The chains are walked in FP64 whatever precision the estimator runs in: by products of the
-// units' factors (metropolis_ratio_body), or by sums of f (metropolis_body) where the weights leave
-// their range.  An FP32 network's chains follow the FP64 parameters, with the 24-bit uniforms
-// (u24) they have always drawn: FP64 operations run at the FP32 rate here, so walking them in FP32
-// with exp, log and sin was the slower and the less exact way (4x4 XYZ, 4096 persistent chains
-// 113 us per launch before, 89 now; 1024 of 12 sites, 400 proposals, 278 -> 165).
-//
-// Mapping of both: a group of `lpc` lanes (power of two) runs one chain, 64/lpc chains
+// Mapping: a group of `lpc` lanes (power of two) runs one chain, 64/lpc chains
 // per wavefront.  Lane g of a group owns lambda units h = g + lpc r (both
 // sides) and Pi units a = g + lpc r; only the lambda and Pi blocks enter
-// Re log rho, the mu block does not.
-// metropolis_body: the effective angles stay in registers;
+// Re log rho, the mu block does not.  The effective angles stay in registers;
 // a proposal costs one FMA + one f (softplus or logcosh, the NDM's activation)
 // per lambda unit of the flipped side and one complex update + Re f per Pi
 // unit, then a group reduction.
@@ -34,16 +26,17 @@
 
 namespace {
 
-__device__ __forceinline__ double xv(uint32_t bits, int i) { return ((bits >> i) & 1u) ? 1.0 : -1.0; }
+template <typename T>
+__device__ __forceinline__ T xv(uint32_t bits, int i) { return ((bits >> i) & 1u) ? T(1) : T(-1); }
 
 // the block body; bx = the workgroup's number in its problem's grid
-template <int US, int ACT>
+template <typename T, int US, int ACT>
 __device__ __forceinline__ void metropolis_body(const samp_args& a, int bx) {
     extern __shared__ __align__(16) unsigned char smem[];
     const ndm_dims d = a.d;
     const int N = d.N, nh = d.nh, na = d.na;
-    double* sp = reinterpret_cast<double*>(smem);
-    const double* gp = reinterpret_cast<const double*>(a.p);
+    T* sp = reinterpret_cast<T*>(smem);
+    const T* gp = reinterpret_cast<const T*>(a.p);
     for (int k = threadIdx.x; k < d.np; k += blockDim.x) sp[k] = gp[k];
     __syncthreads();
 
@@ -58,7 +51,7 @@ __device__ __forceinline__ void metropolis_body(const samp_args& a, int bx) {
     const uint32_t pmask = (N >= 32) ? 0xffffffffu : ((1u << N) - 1u);
     const uint32_t k0 = (uint32_t)a.seed, k1 = (uint32_t)(a.seed >> 32);
     const uint32_t iter = a.iter_dev ? *a.iter_dev : a.iter;
-    const double half = 0.5;
+    const T half = T(0.5);
 
     const bool diag = a.diag != 0;
     const uint32_t ctr3 = 16u * a.tag;
@@ -78,8 +71,8 @@ __device__ __forceinline__ void metropolis_body(const samp_args& a, int bx) {
         }
     }
 
-    double th_s[US], th_e[US], f_s[US], f_e[US], fpi[US];
-    cplx<double> z[US];
+    T th_s[US], th_e[US], f_s[US], f_e[US], fpi[US];
+    cplx<T> z[US];
     uint64_t acc = 0;
     uint32_t t = a.t0;
     uint32_t rx0 = 0, rx1 = 0, rx2 = 0;   // this lane's pre-drawn proposal
@@ -91,22 +84,22 @@ __device__ __forceinline__ void metropolis_body(const samp_args& a, int bx) {
 #pragma unroll
         for (int r = 0; r < US; ++r) {
             const int h = g + lpc * r;
-            th_s[r] = th_e[r] = f_s[r] = f_e[r] = fpi[r] = 0.0;
-            z[r] = cmk(0.0, 0.0);
+            th_s[r] = th_e[r] = f_s[r] = f_e[r] = fpi[r] = T(0);
+            z[r] = cmk(T(0), T(0));
             if (h < nh) {
-                double ts = sp[d.hla + h], te = ts;
+                T ts = sp[d.hla + h], te = ts;
                 for (int i = 0; i < N; ++i) {
-                    const double w = sp[d.wla + h + nh * i];
-                    ts += w * xv(ks, i);
-                    te += w * xv(ke, i);
+                    const T w = sp[d.wla + h + nh * i];
+                    ts += w * xv<T>(ks, i);
+                    te += w * xv<T>(ke, i);
                 }
                 th_s[r] = ts; th_e[r] = te;
                 f_s[r] = act_f<ACT>(ts); f_e[r] = act_f<ACT>(te);
             }
             if (h < na) {
-                double zr = sp[d.dla + h], zi = 0.0;
+                T zr = sp[d.dla + h], zi = T(0);
                 for (int i = 0; i < N; ++i) {
-                    const double xs = xv(ks, i), xe = xv(ke, i);
+                    const T xs = xv<T>(ks, i), xe = xv<T>(ke, i);
                     zr += half * sp[d.ula + h + na * i] * (xs + xe);
                     zi += half * sp[d.umu + h + na * i] * (xs - xe);
                 }
@@ -128,18 +121,18 @@ __device__ __forceinline__ void metropolis_body(const samp_args& a, int bx) {
             const bool col = site >= N;
             const int j = col ? site - N : site;
             const uint32_t bits = col ? (uint32_t)(key >> N) : (uint32_t)key;
-            const double c = ((bits >> j) & 1u) ? -2.0 : 2.0;
+            const T c = ((bits >> j) & 1u) ? T(-2) : T(2);
 
-            double delta = 0.0;
-            double nth[US], nf[US], nfpi[US];
-            cplx<double> nz[US];
+            T delta = T(0);
+            T nth[US], nf[US], nfpi[US];
+            cplx<T> nz[US];
 #pragma unroll
             for (int r = 0; r < US; ++r) {
                 const int h = g + lpc * r;
-                nth[r] = nf[r] = nfpi[r] = 0.0;
+                nth[r] = nf[r] = nfpi[r] = T(0);
                 nz[r] = z[r];
                 if (h < nh) {
-                    const double th = col ? th_e[r] : th_s[r];
+                    const T th = col ? th_e[r] : th_s[r];
                     nth[r] = th + c * sp[d.wla + h + nh * j];
                     nf[r] = act_f<ACT>(nth[r]);
                     delta += nf[r] - (col ? f_e[r] : f_s[r]);
@@ -150,19 +143,25 @@ __device__ __forceinline__ void metropolis_body(const samp_args& a, int bx) {
                         nfpi[r] = cact_re<ACT>(nz[r]);
                         delta += nfpi[r] - fpi[r];
                     } else {
-                        const double cu = c * half;
+                        const T cu = c * half;
                         nz[r].re += cu * sp[d.ula + h + na * j];
                         nz[r].im += (col ? -cu : cu) * sp[d.umu + h + na * j];
                         nfpi[r] = cact_re<ACT>(nz[r]);
-                        delta += 2.0 * (nfpi[r] - fpi[r]);
+                        delta += T(2) * (nfpi[r] - fpi[r]);
                     }
                 }
             }
             delta = group_total(delta, lpc);
             delta += c * sp[d.bla + j];
 
-            const double u = a.u24 ? (double)u01_24(x1) : u01_53(x1, x2);
-            const bool accept = !(u - exp(delta) >= 0.0);
+            bool accept;
+            if constexpr (sizeof(T) == 8) {
+                const double u = u01_53(x1, x2);
+                accept = !(u - exp((double)delta) >= 0.0);
+            } else {
+                const float u = u01_24(x1);
+                accept = !(u - expf((float)delta) >= 0.0f);
+            }
             if (accept && live) {
                 key ^= diag ? ((1ull << site) | (1ull << (site + N))) : (1ull << site);
                 ++acc;
@@ -192,7 +191,7 @@ __device__ __forceinline__ void metropolis_body(const samp_args& a, int bx) {
     }
 }
 
-// ---- the same chains without a transcendental function per proposal
+// ---- FP64: the same chains without a transcendental function per proposal
 // Over the units the acceptance ratio e^(dlog p) is a ratio of products:
 //   softplus  e^f(x) = 1 + e^x,  e^(2 Re f(z)) = |1 + e^z|^2
 //   logcosh   e^f(x) = e^-x (1 + e^2x) / 2,  e^(2 Re f(z)) = e^(-2 Re z) |1 + e^2z|^2 / 4
@@ -245,11 +244,6 @@ __device__ __forceinline__ bool metropolis_ratio_body(const samp_args& a, int bx
     const int gw = lane & (width - 1);
     const int gbase = lane - gw;
 
-    // the weights into the tables' places (coalesced), then the sums below read LDS
-    for (int k = threadIdx.x; k < N * nh; k += blockDim.x) tl[k].x = gp[d.wla + k];
-    for (int k = threadIdx.x; k < N * na; k += blockDim.x) tp[k] = make_double2(gp[d.ula + k], gp[d.umu + k]);
-    __syncthreads();
-
     // this lane's units: the centring constants, the factors with every site at -1 (e0, and w0,
     // which is real there), and the range of the group's products
     int hu[US], au[US];
@@ -259,21 +253,30 @@ __device__ __forceinline__ bool metropolis_ratio_body(const samp_args& a, int bx
         const int u = g + lpc * r;
         hu[r] = u < nh ? u : -1;
         au[r] = u < na ? u : -1;
-        const int h = u < nh ? u : 0, q = u < na ? u : 0;
-        double tw = gp[d.hla + h], tu = gp[d.dla + q], mw = fabs(tw), mu = fabs(tu);
-#pragma unroll 4
-        for (int i = 0; i < N; ++i) {
-            const double w = tl[i * nh + h].x, ul = tp[i * na + q].x;
-            tw -= w;
-            mw += fabs(w);
-            tu -= ul;
-            mu += fabs(ul);
+        kl[r] = kp[r] = 1.0;
+        e0[r] = w0[r] = 0.0;
+        if (hu[r] >= 0) {
+            double t = gp[d.hla + u], m = fabs(t);
+            for (int i = 0; i < N; ++i) {
+                const double w = gp[d.wla + u + nh * i];
+                t -= w;
+                m += fabs(w);
+            }
+            kl[r] = exp(-0.5 * K * m);
+            e0[r] = exp(K * t - 0.5 * K * m);
+            range += 0.5 * K * m + 0.7;
         }
-        kl[r] = hu[r] >= 0 ? exp(-0.5 * K * mw) : 1.0;
-        kp[r] = au[r] >= 0 ? exp(-0.5 * K * mu) : 1.0;
-        e0[r] = hu[r] >= 0 ? exp(K * (tw - 0.5 * mw)) : 0.0;
-        w0[r] = au[r] >= 0 ? exp(K * (tu - 0.5 * mu)) : 0.0;
-        range += (hu[r] >= 0 ? 0.5 * K * mw + 0.7 : 0.0) + (au[r] >= 0 ? K * mu + 1.4 : 0.0);
+        if (au[r] >= 0) {
+            double t = gp[d.dla + u], m = fabs(t);
+            for (int i = 0; i < N; ++i) {
+                const double w = gp[d.ula + u + na * i];
+                t -= w;
+                m += fabs(w);
+            }
+            kp[r] = exp(-0.5 * K * m);
+            w0[r] = exp(K * t - 0.5 * K * m);
+            range += K * m + 1.4;
+        }
     }
     range = group_total(range, lpc);
     // the flipped site's bias factor: the visible bias, for logcosh less the units' linear parts
@@ -284,29 +287,26 @@ __device__ __forceinline__ bool metropolis_ratio_body(const samp_args& a, int bx
             double lin = 0.0;
 #pragma unroll
             for (int r = 0; r < US; ++r) {
-                if (hu[r] >= 0) lin += tl[j * nh + hu[r]].x;
-                if (au[r] >= 0) lin += tp[j * na + au[r]].x;
+                if (hu[r] >= 0) lin += gp[d.wla + hu[r] + nh * j];
+                if (au[r] >= 0) lin += gp[d.ula + au[r] + na * j];
             }
             b -= group_total(lin, lpc);
         }
         ok = ok && 2.0 * fabs(b) <= kRatioBias;
-        if (threadIdx.x == j) {
-            const double e = exp(2.0 * b);
-            tb[j] = make_double2(e, 1.0 / e);
-        }
+        if (threadIdx.x == 0) tb[j] = make_double2(exp(2.0 * b), exp(-2.0 * b));
     }
     if (!__builtin_amdgcn_readfirstlane((int)ok)) return false;   // the same sums in every group
-    __syncthreads();
     for (int k = threadIdx.x; k < N * nh; k += blockDim.x) {
-        const double e = exp(2.0 * K * tl[k].x);
-        tl[k] = make_double2(e, 1.0 / e);
+        const double w = 2.0 * K * gp[d.wla + k];
+        tl[k] = make_double2(exp(w), exp(-w));
     }
     for (int k = threadIdx.x; k < N * na; k += blockDim.x) {
         // a flip of one side to v moves z by v (u_la +- i u_mu); on the diagonal both sides flip
-        const double2 v = tp[k];
-        double s = 0.0, c = 1.0;
-        if (!diag) sincos(K * v.y, &s, &c);
-        const double ep = exp((diag ? 2.0 : 1.0) * K * v.x), em = 1.0 / ep;
+        const double ul = (diag ? 2.0 : 1.0) * K * gp[d.ula + k];
+        const double um = diag ? 0.0 : K * gp[d.umu + k];
+        double s, c;
+        sincos(um, &s, &c);
+        const double ep = exp(ul), em = exp(-ul);
         tp[k] = make_double2(ep * c, ep * s);
         tm[k] = make_double2(em * c, -em * s);
     }
@@ -350,7 +350,7 @@ __device__ __forceinline__ bool metropolis_ratio_body(const samp_args& a, int bx
         if (slot == 0) {
             const philox_out o = philox4x32_10(a.t0 + q + (uint32_t)gw, iter, (uint32_t)chain, ctr3 + 1u, k0, k1);
             dsite = (int)(((uint64_t)o.x[0] * (uint64_t)nsite) >> 32);
-            du = a.u24 ? (double)u01_24(o.x[1]) : u01_53(o.x[1], o.x[2]);
+            du = u01_53(o.x[1], o.x[2]);
         }
         site = __shfl(dsite, gbase + slot, 64);
         u = __shfl(du, gbase + slot, 64);
@@ -481,30 +481,38 @@ __device__ __forceinline__ bool metropolis_ratio_body(const samp_args& a, int bx
     return true;
 }
 
-// by products where the weights' range allows it, else by sums of f
-template <int LPC, int US, int ACT, bool DIAG>
-__device__ __forceinline__ void metropolis_any(const samp_args& a, int bx) {
-    if (metropolis_ratio_body<LPC, US, ACT, DIAG>(a, bx)) return;
+template <int US, int ACT>
+__global__ __launch_bounds__(256) void k_metropolis(samp_args a) {
+    metropolis_body<float, US, ACT>(a, blockIdx.x);
+}
+
+// FP64 chains: by products where the weights' range allows it, else by sums of f
+template <int LPC, int US, int ACT>
+__device__ __forceinline__ void metropolis_f64(const samp_args& a, int bx) {
+    if (a.diag ? metropolis_ratio_body<LPC, US, ACT, true>(a, bx) : metropolis_ratio_body<LPC, US, ACT, false>(a, bx)) return;
     __syncthreads();
     samp_args w = a;
     w.lpc = LPC * a.rep;   // the chain's lanes as one group
-    metropolis_body<US, ACT>(w, bx);
+    metropolis_body<double, US, ACT>(w, bx);
 }
-template <int LPC, int US, int ACT, bool DIAG>
-__global__ __launch_bounds__(256) void k_metropolis(samp_args a) {
-    metropolis_any<LPC, US, ACT, DIAG>(a, blockIdx.x);
+template <int LPC, int US, int ACT>
+__global__ __launch_bounds__(256) void k_metropolis_f64(samp_args a) {
+    metropolis_f64<LPC, US, ACT>(a, blockIdx.x);
 }
 
 // packed: the members' sampler launches in one grid (block records as in nq_pk_member)
-// (one launch for every group width, so that members of different sizes run side by side)
-template <int ACT>
+template <typename T, int ACT>
 __global__ __launch_bounds__(256) void k_metropolis_pk(const nq_pk_member* M, const uint2* blk) {
     const uint2 b = blk[blockIdx.x];
     const samp_args a = M[b.x & 0xffff].sa;
     const int bx = (int)(b.y & 0xffff);
-    if (a.lpc == 8) metropolis_any<8, 1, ACT, false>(a, bx);
-    else if (a.lpc == 16) metropolis_any<16, 1, ACT, false>(a, bx);
-    else metropolis_any<32, 1, ACT, false>(a, bx);
+    if constexpr (sizeof(T) == 8) {
+        if (a.lpc == 8) metropolis_f64<8, 1, ACT>(a, bx);
+        else if (a.lpc == 16) metropolis_f64<16, 1, ACT>(a, bx);
+        else metropolis_f64<32, 1, ACT>(a, bx);
+    } else {
+        metropolis_body<T, 1, ACT>(a, bx);
+    }
 }
 
 constexpr int kSampWaves = 4;   // wavefronts per workgroup (default)
@@ -518,79 +526,94 @@ int64_t samp_grid(const samp_args& a) {
     return (waves + samp_waves(a) - 1) / samp_waves(a);
 }
 
-// dynamic LDS: the product tables, or the parameters in their place
-size_t samp_lds(const ndm_dims& d) { return std::max(sizeof(double) * (size_t)d.np, ratio_lds_bytes(d)); }
+// dynamic LDS: the parameters, or in FP64 the product tables in their place
+size_t samp_lds(const ndm_dims& d, bool fp64) {
+    const size_t par = (fp64 ? sizeof(double) : sizeof(float)) * (size_t)d.np;
+    return fp64 ? std::max(par, ratio_lds_bytes(d)) : par;
+}
+
+template <int US>
+hipError_t launch_f32(const samp_args& a, hipStream_t st) {
+    const dim3 grid((unsigned)samp_grid(a)), blk(64 * samp_waves(a));
+    const size_t lds = samp_lds(a.d, false);
+    if (a.d.act == NQ_ACT_LOGCOSH)
+        hipLaunchKernelGGL((k_metropolis<US, NQ_ACT_LOGCOSH>), grid, blk, lds, st, a);
+    else
+        hipLaunchKernelGGL((k_metropolis<US, NQ_ACT_SOFTPLUS>), grid, blk, lds, st, a);
+    return hipGetLastError();
+}
 
 template <int LPC, int US>
-hipError_t launch_t(const samp_args& a, hipStream_t st) {
+hipError_t launch_f64(const samp_args& a, hipStream_t st) {
     const dim3 grid((unsigned)samp_grid(a)), blk(64 * samp_waves(a));
-    const size_t lds = samp_lds(a.d);
-    const bool lc = a.d.act == NQ_ACT_LOGCOSH;
-    if (a.diag && lc)
-        hipLaunchKernelGGL((k_metropolis<LPC, US, NQ_ACT_LOGCOSH, true>), grid, blk, lds, st, a);
-    else if (a.diag)
-        hipLaunchKernelGGL((k_metropolis<LPC, US, NQ_ACT_SOFTPLUS, true>), grid, blk, lds, st, a);
-    else if (lc)
-        hipLaunchKernelGGL((k_metropolis<LPC, US, NQ_ACT_LOGCOSH, false>), grid, blk, lds, st, a);
+    const size_t lds = samp_lds(a.d, true);
+    if (a.d.act == NQ_ACT_LOGCOSH)
+        hipLaunchKernelGGL((k_metropolis_f64<LPC, US, NQ_ACT_LOGCOSH>), grid, blk, lds, st, a);
     else
-        hipLaunchKernelGGL((k_metropolis<LPC, US, NQ_ACT_SOFTPLUS, false>), grid, blk, lds, st, a);
+        hipLaunchKernelGGL((k_metropolis_f64<LPC, US, NQ_ACT_SOFTPLUS>), grid, blk, lds, st, a);
     return hipGetLastError();
 }
 
 }  // namespace
 
-// one unit of each kind per lane (the group width is a template argument: 8 lanes or more)
-int nq_sampler_lanes_per_chain(const ndm_dims& d) {
+// one unit of each kind per lane; at least 8 lanes in FP64 (its group width is a template argument)
+int nq_sampler_lanes_per_chain(const ndm_dims& d, bool fp64) {
     const int m = d.nh > d.na ? d.nh : d.na;
-    int l = 8;
+    int l = fp64 ? 8 : 1;
     while (l < m && l < 64) l <<= 1;
     return l;
 }
 
-hipError_t nq_launch_metropolis(const samp_args& a0, hipStream_t st) {
+hipError_t nq_launch_metropolis(const samp_args& a0, bool fp64, hipStream_t st) {
     samp_args a = a0;
     const int m = a.d.nh > a.d.na ? a.d.nh : a.d.na;
     a.rep = 1;
-    // while the chains leave SIMDs without a wave, copies of a group share a wave and with it the
-    // draws (a wave's Philox pass then covers 64 proposals of one chain): 16 chains of 6 sites
+    // FP64: while the chains leave SIMDs without a wave, copies of a group share a wave and with it
+    // the draws (a wave's Philox pass then covers 64 proposals of one chain): 16 chains of 6 sites
     // 1.8 -> 1.2 ms per launch
-    while (a.lpc * a.rep < 64 && a.chains * a.lpc * a.rep * 2 <= kRepLanes) a.rep *= 2;
+    while (fp64 && a.lpc * a.rep < 64 && a.chains * a.lpc * a.rep * 2 <= kRepLanes) a.rep *= 2;
     // and with more than one wave per SIMD a lane takes several units instead, which shares the
     // proposal's overhead (draws, table index, acceptance) between them: 4096 chains of the 4x4 XYZ
     // network 0.95 ms at one unit per lane (2 waves per SIMD), 0.84 at two (1), 1.18 at four (1/2)
-    while (a.lpc > 8 && 4 * (a.lpc / 2) >= m && a.chains * a.lpc > kRepLanes) a.lpc /= 2;
+    while (fp64 && a.lpc > 8 && 4 * (a.lpc / 2) >= m && a.chains * a.lpc > kRepLanes) a.lpc /= 2;
     if (a.d.N > 32 || a.lpc < 1 || a.lpc > 64 || (a.lpc & (a.lpc - 1)) || m > 4 * a.lpc) return hipErrorInvalidValue;
+    if (!fp64) return m > a.lpc ? hipErrorInvalidValue : launch_f32<1>(a, st);
     switch (10 * a.lpc + (m + a.lpc - 1) / a.lpc) {
-        case 81: return launch_t<8, 1>(a, st);
-        case 82: return launch_t<8, 2>(a, st);
-        case 83: case 84: return launch_t<8, 4>(a, st);
-        case 161: return launch_t<16, 1>(a, st);
-        case 162: return launch_t<16, 2>(a, st);
-        case 163: case 164: return launch_t<16, 4>(a, st);
-        case 321: return launch_t<32, 1>(a, st);
-        case 322: return launch_t<32, 2>(a, st);
-        case 641: return launch_t<64, 1>(a, st);
+        case 81: return launch_f64<8, 1>(a, st);
+        case 82: return launch_f64<8, 2>(a, st);
+        case 83: case 84: return launch_f64<8, 4>(a, st);
+        case 161: return launch_f64<16, 1>(a, st);
+        case 162: return launch_f64<16, 2>(a, st);
+        case 163: case 164: return launch_f64<16, 4>(a, st);
+        case 321: return launch_f64<32, 1>(a, st);
+        case 322: return launch_f64<32, 2>(a, st);
+        case 641: return launch_f64<64, 1>(a, st);
         default: return hipErrorInvalidValue;
     }
 }
 
-// packed launches: groups of 8, 16 or 32 lanes, one unit per lane; variant = logcosh
-int nq_sampler_variant(const samp_args& a, int* threads, size_t* lds, int* grid) {
+// packed launches: one lane group per chain covers every unit (lanes per
+// chain >= max(nh, na), so one unit slot per lane); variant = fp64 | logcosh << 1
+int nq_sampler_variant(const samp_args& a, bool fp64, int* threads, size_t* lds, int* grid) {
     const int m = a.d.nh > a.d.na ? a.d.nh : a.d.na;
-    if (a.d.N > 32 || (a.lpc != 8 && a.lpc != 16 && a.lpc != 32) || m > a.lpc || a.rep != 1) return -1;
+    if (a.d.N > 32 || a.lpc < 1 || a.lpc > 64 || (a.lpc & (a.lpc - 1)) || m > a.lpc) return -1;
     const int64_t g = samp_grid(a);
     if (g > 0xffff) return -1;
     *threads = 64 * samp_waves(a);
-    *lds = samp_lds(a.d);
+    *lds = samp_lds(a.d, fp64);
     *grid = (int)g;
-    return a.d.act == NQ_ACT_LOGCOSH ? 1 : 0;
+    return (fp64 ? 1 : 0) | (a.d.act == NQ_ACT_LOGCOSH ? 2 : 0);
 }
 
 hipError_t nq_pk_sampler(const nq_pk_member* M, const nq_pk_launch& L, hipStream_t st) {
     if (L.nblk <= 0) return hipSuccess;
     const dim3 g((unsigned)L.nblk), b((unsigned)L.threads);
-    if (L.variant == 0) hipLaunchKernelGGL((k_metropolis_pk<NQ_ACT_SOFTPLUS>), g, b, L.lds, st, M, L.blk);
-    else if (L.variant == 1) hipLaunchKernelGGL((k_metropolis_pk<NQ_ACT_LOGCOSH>), g, b, L.lds, st, M, L.blk);
-    else return hipErrorInvalidValue;
+    switch (L.variant) {
+        case 0: hipLaunchKernelGGL((k_metropolis_pk<float, NQ_ACT_SOFTPLUS>), g, b, L.lds, st, M, L.blk); break;
+        case 1: hipLaunchKernelGGL((k_metropolis_pk<double, NQ_ACT_SOFTPLUS>), g, b, L.lds, st, M, L.blk); break;
+        case 2: hipLaunchKernelGGL((k_metropolis_pk<float, NQ_ACT_LOGCOSH>), g, b, L.lds, st, M, L.blk); break;
+        case 3: hipLaunchKernelGGL((k_metropolis_pk<double, NQ_ACT_LOGCOSH>), g, b, L.lds, st, M, L.blk); break;
+        default: return hipErrorInvalidValue;
+    }
     return hipGetLastError();
 }

@@ -1770,7 +1770,7 @@ hipError_t nq_pk_plan(const nq_pk_member& m, int kernel, int param, nq_pk_shape*
         case NQ_PK_PREP: o->gx = (int)nblk(m.chains > 0 ? m.chains : 1, 256); break;
         case NQ_PK_METROPOLIS: {
             int grid = 0;
-            o->variant = nq_sampler_variant(m.sa, &o->threads, &o->lds, &grid);
+            o->variant = nq_sampler_variant(m.sa, m.fp64 != 0, &o->threads, &o->lds, &grid);
             if (o->variant < 0) return hipErrorInvalidValue;
             o->gx = grid;
             break;

@@ -43,7 +43,7 @@ hipError_t nq_launch_estimate(const est_args& a, bool fp64, int grid, hipStream_
 // ---- Metropolis sampler (k_sampler.hip)
 struct samp_args {
     ndm_dims d;
-    const void* p;             // parameters: double for the NDM, network precision for the RBMs
+    const void* p;
     int64_t chains;
     int passes, burn, stored;  // calls = burn + stored
     uint32_t t0;               // index of this launch's first proposal within the iteration
@@ -51,8 +51,7 @@ struct samp_args {
     int diag;                  // chain on the diagonal (sigma, sigma): p ~ rho(sigma, sigma), both sides flipped
     uint32_t tag;              // random stream: counter word 3 = {0 start, 1 proposal} + 16 tag
     int lpc;                   // lanes per chain (power of two)
-    int u24;                   // 24-bit uniforms (the chains of an FP32 network)
-    int rep;                   // copies of the group in a wave (power of two, lpc rep <= 64), 1 in packed launches
+    int rep;                   // FP64: copies of the group in a wave (power of two, lpc rep <= 64), 1 in packed launches
     int restart;               // draw a fresh uniform configuration per chain
     int compat_stale_last_slice;
     uint64_t seed;
@@ -64,8 +63,8 @@ struct samp_args {
     uint32_t* chain_acc;       // chains: accepted proposals per chain, added to (nullable)
     int waves;                 // waves per workgroup, 1, 2 or 4 (0: 4)
 };
-int nq_sampler_lanes_per_chain(const ndm_dims& d);
-hipError_t nq_launch_metropolis(const samp_args& a, hipStream_t st);
+int nq_sampler_lanes_per_chain(const ndm_dims& d, bool fp64);
+hipError_t nq_launch_metropolis(const samp_args& a, bool fp64, hipStream_t st);
 
 // ---- S build (k_sbuild.hip)
 enum { NQ_GRAM_F64 = 0, NQ_GRAM_F32 = 1, NQ_GRAM_BF16 = 2 };
@@ -441,4 +440,4 @@ hipError_t nq_pk_estimate_f32(const nq_pk_member* M, const nq_pk_launch& L, hipS
 hipError_t nq_pk_sbuild(const nq_pk_member* M, const nq_pk_launch& L, hipStream_t st);
 hipError_t nq_pk_solve(const nq_pk_member* M, const nq_pk_launch& L, hipStream_t st);
 int nq_est_variant(const est_args& a, bool fp64, int* threads, size_t* lds);
-int nq_sampler_variant(const samp_args& a, int* threads, size_t* lds, int* grid);
+int nq_sampler_variant(const samp_args& a, bool fp64, int* threads, size_t* lds, int* grid);

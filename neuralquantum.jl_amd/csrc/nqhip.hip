@@ -440,7 +440,7 @@ hipError_t launch_update(nqh_ctx* c, double lr) {
 }
 
 hipError_t launch_metropolis(nqh_ctx* c, const samp_args& a) {
-    if (!is_rbm(c)) return nq_launch_metropolis(a, c->stream);
+    if (!is_rbm(c)) return nq_launch_metropolis(a, fp64_net(c), c->stream);
     rbm_samp_args r{};
     r.N = c->rbm_N;
     r.nh = c->rbm_nh;
@@ -1333,8 +1333,7 @@ static nqh_status run_sampler(nqh_ctx* c) {
     if (!c->has_sampler) return fail(c, NQH_E_STATE, "sampler not set (nqh_set_sampler)");
     samp_args a{};
     a.d = c->d;
-    a.p = (fp64_net(c) || !is_rbm(c)) ? c->p64.p : c->p32.p;
-    a.u24 = fp64_net(c) ? 0 : 1;
+    a.p = fp64_net(c) ? c->p64.p : c->p32.p;
     a.chains = c->chains;
     a.passes = c->passes;
     const bool compat = (c->flags & NQH_SAMPLER_COMPAT_STALE_LAST_SLICE) != 0;
@@ -1345,7 +1344,7 @@ static nqh_status run_sampler(nqh_ctx* c) {
     a.burn = a.restart ? c->burn : 0;
     a.stored = compat ? c->chain_len - 1 : c->chain_len;
     a.compat_stale_last_slice = compat ? 1 : 0;
-    a.lpc = is_rbm(c) ? 1 : nq_sampler_lanes_per_chain(c->d);
+    a.lpc = is_rbm(c) ? 1 : nq_sampler_lanes_per_chain(c->d, fp64_net(c));
     a.seed = c->seed;
     a.iter = c->iter;
     a.chain_state = P<uint64_t>(c->chain_state);
@@ -2430,8 +2429,7 @@ nq_pk_member pk_describe(nqh_ctx* c, double eps, int kind, double lr) {
     // the sampler (run_sampler in graph form: iteration number from iter_dev)
     samp_args& a = m.sa;
     a.d = d;
-    a.p = c->p64.p;
-    a.u24 = f64 ? 0 : 1;
+    a.p = f64 ? c->p64.p : c->p32.p;
     a.chains = c->chains;
     a.passes = c->passes;
     const bool compat = (c->flags & NQH_SAMPLER_COMPAT_STALE_LAST_SLICE) != 0;
@@ -2440,7 +2438,7 @@ nq_pk_member pk_describe(nqh_ctx* c, double eps, int kind, double lr) {
     a.burn = a.restart ? c->burn : 0;
     a.stored = compat ? c->chain_len - 1 : c->chain_len;
     a.compat_stale_last_slice = compat ? 1 : 0;
-    a.lpc = nq_sampler_lanes_per_chain(d);
+    a.lpc = nq_sampler_lanes_per_chain(d, fp64_net(c));
     a.rep = 1;
     a.seed = c->seed;
     a.iter = c->iter;
@@ -3116,8 +3114,7 @@ nqh_status nqh_observable(nqh_ctx* c, const nqh_optable* op, int64_t chains, int
     // the diagonal chain, restarted at every call (_sample_state!), its own random stream
     samp_args a{};
     a.d = c->d;
-    a.p = (fp64_net(c) || !is_rbm(c)) ? c->p64.p : c->p32.p;
-    a.u24 = fp64_net(c) ? 0 : 1;
+    a.p = fp64_net(c) ? c->p64.p : c->p32.p;
     a.chains = chains;
     a.passes = passes;
     a.burn = burn;
@@ -3125,7 +3122,7 @@ nqh_status nqh_observable(nqh_ctx* c, const nqh_optable* op, int64_t chains, int
     a.restart = 1;
     a.diag = 1;
     a.tag = 1;
-    a.lpc = is_rbm(c) ? 1 : nq_sampler_lanes_per_chain(c->d);
+    a.lpc = is_rbm(c) ? 1 : nq_sampler_lanes_per_chain(c->d, fp64_net(c));
     a.seed = c->seed;
     a.iter = c->iter;
     a.chain_state = P<uint64_t>(c->obs_state);

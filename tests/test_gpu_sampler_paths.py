@@ -39,24 +39,3 @@ def test_fp64_chains_follow_the_oracle(gpu_ok, act, N, nh, na, sigma, chains):
     assert np.array_equal(keys, keys_r)
     assert acc == acc_r
     ctx.close()
-
-
-@pytest.mark.parametrize("act", [0, 1])
-@pytest.mark.parametrize("N,nh,na,chains", [(3, 1, 2, 5), (6, 12, 7, 64), (5, 40, 33, 8)])
-def test_fp32_networks_walk_the_fp64_chains(gpu_ok, act, N, nh, na, chains):
-    """An FP32 network's chains are walked in FP64 with the upper 24 bits of
-    the uniforms: the FP64 network's trajectories, unless an acceptance lies
-    within 2^-24 of its uniform (at most 64 x 4 x 13 = 3328 proposals here,
-    expected 2e-4 of them)."""
-    flat, _, _ = ising(N)
-    keys = []
-    for net in (_lib.PREC_FP64, _lib.PREC_FP32):
-        ctx = Context(0, 71)
-        ctx.set_problem(flat)
-        ctx.set_ndm(N, nh, na, act)
-        ctx.set_params(params(ctx.np_, seed=nh, sigma=0.3))
-        ctx.set_precision(net, _lib.PREC_FP32 if net else _lib.PREC_FP64)
-        ctx.set_sampler(chains, 3, 13, 1)
-        keys.append(ctx.sample()[0])
-        ctx.close()
-    assert np.array_equal(keys[0], keys[1])
