@@ -296,6 +296,7 @@ struct rbm_samp_args {
     uint32_t t0;
     int slice0;
     int lpc;
+    int rep;                  // FP64: copies of the group in a wave (lpc rep <= 64)
     int restart;
     int compat_stale_last_slice;
     uint64_t seed;
