@@ -9,12 +9,10 @@
 // block A = columns [0, nA) (the real parts) and block B = columns [nA, R)
 // (the imaginary parts); column c belongs to parameter c (block A) or
 // offB + c - nA (block B), so Re(Oc^H Oc) v = A^T (A v_A) + B^T (B v_B).
-// One product is two passes over Y:
-//   k_yv      w_A[s] = sum_{c < nA} Yc[s, c] v[c],  w_B[s] likewise over B
-//             (one wavefront per sample row, coalesced along the row);
-//   k_ytw     per chunk of samples, part[c] = sum_s Yc[s, c] w_blk(c)[s]
-//             (threads along the columns, coalesced);
-//   k_ytw_finish  q[k] = (sum of the chunks of the columns of k) / Ns
+// One product:
+//   k_sv      per workgroup, over its samples: w_A[s] = sum_{c < nA} Yc[s, c]
+//             v[c], w_B[s] likewise over B, part[c] = sum_s Yc[s, c] w_blk(c)[s];
+//   k_ytw_finish  q[k] = (sum of the workgroups' columns of k) / Ns
 //             + shift(k) v[k].
 // Yc = Y - mu (centred on the fly, FP64 arithmetic on FP32 or FP64 rows).
 #include "nq_device.h"
@@ -22,57 +20,102 @@
 
 namespace {
 
-template <typename YT>
-__global__ __launch_bounds__(256) void k_yv(const YT* Y, int64_t Ns, int R, int nA, int offB, const double* mu,
-                                            const double* v, double* w) {
-    const int lane = threadIdx.x & 63;
-    const int64_t s = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
-    if (s >= Ns) return;
-    const YT* row = Y + s * R;
-    double a = 0.0, b = 0.0;
-    for (int c = lane; c < R; c += 64) {
-        const double y = (double)row[c] - mu[c];
-        if (c < nA) a += y * v[c];
-        else b += y * v[offB + c - nA];
+// One product, one pass over Y: a workgroup takes RB rows of its samples at a time into registers
+// (column t + 512 j in thread t), sums their products with v over the workgroup (RB rows, two blocks:
+// one transposed wave reduction, one LDS exchange and barrier), and adds w_blk Yc to its columns' sums
+// from the same registers while the next rows load.  Bound by HBM: 2 x Ns R bytes were read before, one
+// pass for w = Yc v and one for Yc^T w (4x4 XYZ, FP64, 424 MB of rows: 122 + 128 us a product; now 79 us,
+// 5.4 TB/s, and the sum over the workgroups 33 -> 12 us).
+template <typename YT, int CT, int RB>
+__global__ __launch_bounds__(512) void k_sv(const YT* Y, int64_t Ns, int R, int nA, int offB, const double* mu,
+                                            const double* v, double* part) {
+    __shared__ double red[2][8][8];
+    const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+    const int64_t per = (Ns + gridDim.x - 1) / gridDim.x;
+    const int64_t s0 = (int64_t)blockIdx.x * per, s1 = (s0 + per < Ns) ? s0 + per : Ns;
+    double vj[CT], mj[CT], acc[CT];
+#pragma unroll
+    for (int j = 0; j < CT; ++j) {
+        const int c = t + 512 * j;
+        const bool in = c < R;
+        vj[j] = in ? v[c < nA ? c : offB + c - nA] : 0.0;   // columns past R: 0 times a clamped load
+        mj[j] = in ? mu[c] : 0.0;
+        acc[j] = 0.0;
     }
-    a = wave_total(a);
-    b = wave_total(b);
-    if (lane == 0) {
-        w[2 * s] = a;
-        w[2 * s + 1] = b;
+    YT y[RB][CT], yn[RB][CT];
+    auto load = [&](int64_t s, YT (&d)[RB][CT]) {
+#pragma unroll
+        for (int r = 0; r < RB; ++r) {
+            const YT* row = Y + (s + r < s1 ? s + r : s1 - 1) * R;
+#pragma unroll
+            for (int j = 0; j < CT; ++j) d[r][j] = row[t + 512 * j < R ? t + 512 * j : R - 1];
+        }
+    };
+    int buf = 0;
+    if (s0 < s1) load(s0, y);
+    for (int64_t s = s0; s < s1; s += RB, buf ^= 1) {
+        load(s + RB < s1 ? s + RB : s, yn);
+        double p[8];
+#pragma unroll
+        for (int k = 0; k < 8; ++k) p[k] = 0.0;
+#pragma unroll
+        for (int r = 0; r < RB; ++r)
+#pragma unroll
+            for (int j = 0; j < CT; ++j) {
+                const double x = ((double)y[r][j] - mj[j]) * vj[j];
+                const bool first = t + 512 * j < nA;
+                p[r] += first ? x : 0.0;
+                p[4 + r] += first ? 0.0 : x;
+            }
+        const double tot = wave_totals<8>(p, lane);          // lane l: sum of p[l / 8]
+        if ((lane & 7) == 0) red[buf][wave][lane >> 3] = tot;
+        __syncthreads();
+        double w = red[buf][lane >> 3][lane & 7];             // lane 8 wave + k, summed over the waves
+        w += __shfl_xor(w, 8, 64);
+        w += __shfl_xor(w, 16, 64);
+        w += __shfl_xor(w, 32, 64);
+#pragma unroll
+        for (int r = 0; r < RB; ++r) {
+            const bool row = s + r < s1;
+            const double wa = row ? rl_d(w, r) : 0.0, wb = row ? rl_d(w, 4 + r) : 0.0;
+#pragma unroll
+            for (int j = 0; j < CT; ++j)
+                acc[j] += ((double)y[r][j] - mj[j]) * (t + 512 * j < nA ? wa : wb);
+        }
+#pragma unroll
+        for (int r = 0; r < RB; ++r)
+#pragma unroll
+            for (int j = 0; j < CT; ++j) y[r][j] = yn[r][j];
     }
+#pragma unroll
+    for (int j = 0; j < CT; ++j)
+        if (t + 512 * j < R) part[(int64_t)blockIdx.x * R + t + 512 * j] = acc[j];
 }
 
-template <typename YT>
-__global__ __launch_bounds__(256) void k_ytw(const YT* Y, int64_t Ns, int R, int nA, const double* mu, const double* w,
-                                             int chunks, double* part) {
-    const int c = blockIdx.x * blockDim.x + threadIdx.x;
-    if (c >= R) return;
-    const int64_t per = (Ns + chunks - 1) / chunks;
-    const int64_t s0 = (int64_t)blockIdx.y * per, s1 = (s0 + per < Ns) ? s0 + per : Ns;
-    const int blk = c < nA ? 0 : 1;
-    const double m = mu[c];
+// q[k] = scale * (column sums of parameter k) + shift(k) v[k]; a parameter owns one column of A (k < nA),
+// one of B (k >= offB, k - offB < nB) or both.  64 parameters per workgroup, the chunks over 16 thread
+// groups (coalesced along the parameters), combined in a fixed order
+__global__ __launch_bounds__(1024) void k_ytw_finish(const double* part, int chunks, int R, int nA, int offB, int np,
+                                                     double scale, double eps, int kind, const double* diag,
+                                                     const double* v, double* q) {
+    __shared__ double red[16][64];
+    const int x = threadIdx.x & 63, g = threadIdx.x >> 6;
+    const int k = blockIdx.x * 64 + x, nB = R - nA;
+    const bool inA = k < np && k < nA, inB = k < np && k >= offB && k - offB < nB;
     double acc = 0.0;
-    for (int64_t s = s0; s < s1; ++s) acc += ((double)Y[s * R + c] - m) * w[2 * s + blk];
-    part[(int64_t)blockIdx.y * R + c] = acc;
-}
-
-// q[k] = scale * (column sums of parameter k) + shift(k) v[k]; a parameter
-// owns one column of A (k < nA), one of B (k >= offB, k - offB < nB) or both
-__global__ __launch_bounds__(256) void k_ytw_finish(const double* part, int chunks, int R, int nA, int offB, int np,
-                                                    double scale, double eps, int kind, const double* diag,
-                                                    const double* v, double* q) {
-    const int k = blockIdx.x * blockDim.x + threadIdx.x;
-    if (k >= np) return;
-    const int nB = R - nA;
-    double acc = 0.0;
-    if (k < nA)
-        for (int i = 0; i < chunks; ++i) acc += part[(int64_t)i * R + k];
-    if (k >= offB && k - offB < nB)
-        for (int i = 0; i < chunks; ++i) acc += part[(int64_t)i * R + nA + (k - offB)];
+    if (inA)
+        for (int i = g; i < chunks; i += 16) acc += part[(int64_t)i * R + k];
+    if (inB)
+        for (int i = g; i < chunks; i += 16) acc += part[(int64_t)i * R + nA + (k - offB)];
+    red[g][x] = acc;
+    __syncthreads();
+    if (g != 0 || k >= np) return;
+    double sum = 0.0;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) sum += red[i][x];
     double sh = 0.0;
     if (v) sh = ((kind == 0) ? eps : eps * diag[k]) * v[k];
-    q[k] = scale * acc + sh;
+    q[k] = scale * sum + sh;
 }
 
 // diag(S)[k] = (1/Ns) sum_s (sum over the columns of k of Yc[s, c]^2)
@@ -178,17 +221,23 @@ inline int nblk(int64_t n, int b) { return (int)((n + b - 1) / b); }
 }  // namespace
 
 hipError_t nq_launch_sv(const void* Y, int y_fp64, int64_t Ns, int R, int nA, int offB, int np, const double* mu,
-                        const double* v, double eps, int kind, const double* diag, double* w, double* part,
-                        int chunks, double* q, hipStream_t st) {
-    const dim3 g1(nblk(Ns, 4)), g2(nblk(R, 256), chunks);
-    if (y_fp64) {
-        hipLaunchKernelGGL((k_yv<double>), g1, dim3(256), 0, st, (const double*)Y, Ns, R, nA, offB, mu, v, w);
-        hipLaunchKernelGGL((k_ytw<double>), g2, dim3(256), 0, st, (const double*)Y, Ns, R, nA, mu, w, chunks, part);
-    } else {
-        hipLaunchKernelGGL((k_yv<float>), g1, dim3(256), 0, st, (const float*)Y, Ns, R, nA, offB, mu, v, w);
-        hipLaunchKernelGGL((k_ytw<float>), g2, dim3(256), 0, st, (const float*)Y, Ns, R, nA, mu, w, chunks, part);
-    }
-    hipLaunchKernelGGL(k_ytw_finish, dim3(nblk(np, 256)), dim3(256), 0, st, part, chunks, R, nA, offB, np,
+                        const double* v, double eps, int kind, const double* diag, double* part, double* q,
+                        hipStream_t st) {
+    // one workgroup per CU; four rows at a time while they and the next four fit in the registers
+    const int groups = (int)(Ns < 4 * NQ_SV_GROUPS ? (Ns + 3) / 4 : NQ_SV_GROUPS);
+    const dim3 g(groups), b(512);
+#define NQ_SV(CT, RB)                                                                                              \
+    do {                                                                                                           \
+        if (y_fp64) hipLaunchKernelGGL((k_sv<double, CT, RB>), g, b, 0, st, (const double*)Y, Ns, R, nA, offB, mu, v, part); \
+        else hipLaunchKernelGGL((k_sv<float, CT, RB>), g, b, 0, st, (const float*)Y, Ns, R, nA, offB, mu, v, part);  \
+    } while (0)
+    if (R <= 1024) NQ_SV(2, 4);
+    else if (R <= 2048) NQ_SV(4, 4);
+    else if (R <= 3584) NQ_SV(7, 4);
+    else if (R <= 6656) NQ_SV(13, 2);
+    else return hipErrorInvalidValue;
+#undef NQ_SV
+    hipLaunchKernelGGL(k_ytw_finish, dim3(nblk(np, 64)), dim3(1024), 0, st, part, groups, R, nA, offB, np,
                        1.0 / (double)Ns, eps, kind, diag, v, q);
     return hipGetLastError();
 }
@@ -201,7 +250,7 @@ hipError_t nq_launch_sdiag(const void* Y, int y_fp64, int64_t Ns, int R, int nA,
     else
         hipLaunchKernelGGL((k_colsq<float>), g, dim3(256), 0, st, (const float*)Y, Ns, R, mu, chunks, part);
     // diag[k] = scale * column sums of k (the finish kernel without a shift term)
-    hipLaunchKernelGGL(k_ytw_finish, dim3(nblk(np, 256)), dim3(256), 0, st, part, chunks, R, nA, offB, np,
+    hipLaunchKernelGGL(k_ytw_finish, dim3(nblk(np, 64)), dim3(1024), 0, st, part, chunks, R, nA, offB, np,
                        1.0 / (double)Ns, 0.0, 0, (const double*)nullptr, (const double*)nullptr, diag);
     return hipGetLastError();
 }

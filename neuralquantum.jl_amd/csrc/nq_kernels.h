@@ -106,12 +106,13 @@ hipError_t nq_launch_gram2_bf16(const __bf16* Yt, int64_t nsp, int nA, int nB, i
 
 // matrix-free SR (k_cg.hip): q = S v + shift(v) with S = Re(Oc^H Oc) / Ns from
 // the compact rows Y (block A = columns [0, nA) -> parameters [0, nA), block
-// B = columns [nA, R) -> parameters [offB, offB + R - nA)); w: 2 Ns doubles,
-// part: chunks x R doubles; kind 0: eps v, 1: eps diag(S) v (diag from
+// B = columns [nA, R) -> parameters [offB, offB + R - nA));
+// part: NQ_SV_GROUPS x R doubles; kind 0: eps v, 1: eps diag(S) v (diag from
 // nq_launch_sdiag)
+constexpr int NQ_SV_GROUPS = 256;
 hipError_t nq_launch_sv(const void* Y, int y_fp64, int64_t Ns, int R, int nA, int offB, int np, const double* mu,
-                        const double* v, double eps, int kind, const double* diag, double* w, double* part,
-                        int chunks, double* q, hipStream_t st);
+                        const double* v, double eps, int kind, const double* diag, double* part, double* q,
+                        hipStream_t st);
 hipError_t nq_launch_sdiag(const void* Y, int y_fp64, int64_t Ns, int R, int nA, int offB, int np, const double* mu,
                            double* part, int chunks, double* diag, hipStream_t st);
 // *out = x . y (part: nparts doubles)

@@ -51,10 +51,9 @@ struct nqh_ctx {
     ndm_dims d{};
     int rbm_N = 0, rbm_nh = 0, rbm_npc = 0;
     dbuf p64, p32;
-    // pinned staging of the parameters: [0] number of the last transfer completed, [1] unused, then the
-    // parameters; transfers are numbered, at most one is in flight
+    // pinned staging of the parameters, behind hstat in the same allocation: [0] number of the last
+    // transfer completed, [1] unused, then the parameters; at most one transfer is in flight
     double* hpar = nullptr;
-    int hpar_cap = 0;
     double hpar_seq = 0.0;
     int net_prec = NQH_PREC_FP64;
     int s_prec = NQH_PREC_FP64;
@@ -90,7 +89,7 @@ struct nqh_ctx {
     int cg_maxiter = 0;
     int cg_iters = 0;
     double cg_resid = 0.0;
-    dbuf cg_w, cg_part, cg_p, cg_q, cg_r, cg_sc, cg_diag, cg_dpart;
+    dbuf cg_part, cg_p, cg_q, cg_r, cg_sc, cg_diag, cg_dpart;
     dbuf mr_vw;   // MINRES: three Lanczos vectors and three directions, Np doubles each
     int64_t last_ns = 0;
     bool grad_ready = false;
@@ -136,6 +135,8 @@ struct nqh_ctx {
 
 namespace {
 
+// doubles in the largest flat parameter vector (RBMSplit, N = 16, nh = 128; the NDM's is 4320)
+constexpr int kMaxParams = 2 * (2 * 16 + 128 + 2 * 128 * 16);
 constexpr int kColChunks = 256;
 constexpr int64_t kSplitSamples = 4096;   // batches from this size run the forces launch on a side stream
 constexpr int kTableLdsMax = 32 * 1024;   // connection tables up to this size are staged in LDS
@@ -710,11 +711,13 @@ nqh_status nqh_create(nqh_ctx** out, int32_t device, uint64_t seed) {
     }
     // coherent: the kernel's stores reach the host as they are made (the
     // done word is polled while the last kernel may still be running)
-    if (hipHostMalloc((void**)&c->hstat, 8 * sizeof(double), hipHostMallocCoherent) != hipSuccess) {
+    if (hipHostMalloc((void**)&c->hstat, (8 + 2 + kMaxParams) * sizeof(double), hipHostMallocCoherent) != hipSuccess) {
         (void)hipStreamDestroy(c->stream);
         delete c;
         return NQH_E_HIP;
     }
+    c->hpar = c->hstat + 8;
+    c->hpar[0] = 0.0;
     // the allocation-free entry point's scratch address on this device (a
     // failure here is reported by that entry point, which tries again)
     (void)scratch_setup(c);
@@ -729,8 +732,7 @@ void nqh_destroy(nqh_ctx* c) {
     dbuf* all[] = {&c->table_mem, &c->p64, &c->p32, &c->chain_state, &c->samples, &c->acc, &c->chain_acc, &c->keys_in, &c->lp,
                    &c->Y, &c->Lloc, &c->G, &c->Yt, &c->Fpart, &c->colpart, &c->mu, &c->stats, &c->F, &c->S, &c->S0,
                    &c->delta, &c->resid, &c->info, &c->flag, &c->fpart2, &c->winv, &c->tmp, &c->gpart, &c->A2,
-                   &c->winv2, &c->y2, &c->x2, &c->cg_w,
-                   &c->cg_part, &c->cg_p, &c->cg_q, &c->cg_r, &c->cg_sc, &c->cg_diag, &c->cg_dpart, &c->mr_vw, &c->made_th, &c->made_m, &c->made_v,
+                   &c->winv2, &c->y2, &c->x2, &c->cg_part, &c->cg_p, &c->cg_q, &c->cg_r, &c->cg_sc, &c->cg_diag, &c->cg_dpart, &c->mr_vw, &c->made_th, &c->made_m, &c->made_v,
                    &c->made_gpart, &c->made_lpart, &c->made_g, &c->made_nll, &c->made_keys, &c->made_lp,
                    &c->made_lq, &c->ring, &c->ring_posd, &c->made_tmp, &c->obs_table_mem, &c->obs_keys,
                    &c->obs_state, &c->obs_lp, &c->obs_L, &c->obs_stats, &c->crw, &c->crm, &c->cnum, &c->cwd};
@@ -748,7 +750,6 @@ void nqh_destroy(nqh_ctx* c) {
     }
     (void)hipStreamDestroy(c->stream);
     if (c->hstat) (void)hipHostFree(c->hstat);
-    if (c->hpar) (void)hipHostFree(c->hpar);
     delete c;
 }
 
@@ -991,36 +992,16 @@ static nqh_status param_wait(nqh_ctx* c) {
     return NQH_OK;
 }
 
-// the staging buffer, free of transfers in flight
-static nqh_status param_staging(nqh_ctx* c) {
-    const int n = nsys(c);
-    if (c->hpar) {
-        nqh_status s = param_wait(c);
-        if (s) return s;
-    }
-    if (c->hpar_cap >= n) return NQH_OK;
-    if (c->hpar) (void)hipHostFree(c->hpar);
-    c->hpar = nullptr;
-    c->hpar_cap = 0;
-    if (hipHostMalloc((void**)&c->hpar, sizeof(double) * (size_t)(n + 2), hipHostMallocCoherent) != hipSuccess) {
-        c->hpar = nullptr;
-        return fail(c, NQH_E_NOMEM, "hipHostMalloc of the parameter staging failed");
-    }
-    c->hpar_cap = n;
-    c->hpar[0] = c->hpar_seq;
-    return NQH_OK;
-}
-
 nqh_status nqh_set_params(nqh_ctx* c, const double* flat, int64_t np) {
     if (!c || !flat) return NQH_E_ARG;
     (void)hipSetDevice(c->device);
     nqh_status s = need_net(c);
     if (s) return s;
-    if (np != nsys(c)) return fail(c, NQH_E_ARG, "parameter count mismatch");
+    if (np != nsys(c) || np > kMaxParams) return fail(c, NQH_E_ARG, "parameter count mismatch");
     for (int64_t k = 0; k < np; ++k)
         if (!std::isfinite(flat[k])) return fail(c, NQH_E_NAN, "non-finite parameter");
     // staged, so that `flat` is free at once, and read from there by a kernel on the context's stream
-    if ((s = param_staging(c))) return s;
+    if ((s = param_wait(c))) return s;
     std::memcpy(c->hpar + 2, flat, sizeof(double) * np);
     c->hpar_seq += 1.0;
     const hipError_t e = nq_launch_params_in(c->hpar + 2, P<double>(c->p64), P<float>(c->p32), (int)np, c->hpar,
@@ -1038,8 +1019,8 @@ nqh_status nqh_get_params(const nqh_ctx* cc, double* flat, int64_t np) {
     (void)hipSetDevice(c->device);
     nqh_status s = need_net(c);
     if (s) return s;
-    if (np != nsys(c)) return fail(c, NQH_E_ARG, "parameter count mismatch");
-    if ((s = param_staging(c))) return s;
+    if (np != nsys(c) || np > kMaxParams) return fail(c, NQH_E_ARG, "parameter count mismatch");
+    if ((s = param_wait(c))) return s;
     c->hpar_seq += 1.0;
     const hipError_t e = nq_launch_params_out(P<double>(c->p64), c->hpar + 2, (int)np, c->hpar, c->hpar_seq, c->stream);
     if (e != hipSuccess) {
@@ -1464,8 +1445,7 @@ static nqh_status cg_solve(nqh_ctx* c, double eps, int kind) {
     gram_blocks(c, &nA, &nB, &offB);
     constexpr int chunks = 64, nparts = 64;
     nqh_status s;
-    if ((s = ensure(c, c->cg_w, sizeof(double) * 2 * (size_t)Ns)) ||
-        (s = ensure(c, c->cg_part, sizeof(double) * (size_t)chunks * R)) ||
+    if ((s = ensure(c, c->cg_part, sizeof(double) * (size_t)NQ_SV_GROUPS * R)) ||
         (s = ensure(c, c->cg_p, sizeof(double) * np)) || (s = ensure(c, c->cg_q, sizeof(double) * np)) ||
         (s = ensure(c, c->cg_r, sizeof(double) * np)) || (s = ensure(c, c->cg_diag, sizeof(double) * np)) ||
         (s = ensure(c, c->cg_sc, sizeof(double) * 8)) || (s = ensure(c, c->cg_dpart, sizeof(double) * nparts)))
@@ -1491,8 +1471,7 @@ static nqh_status cg_solve(nqh_ctx* c, double eps, int kind) {
     rr = f2;
     bool ok = f2 == 0.0;
     while (!ok && it < maxit) {
-        HIPCHK(c, nq_launch_sv(c->Y.p, f64, Ns, R, nA, offB, np, mu, p, eps, kind, diag, P<double>(c->cg_w),
-                               P<double>(c->cg_part), chunks, q, st));
+        HIPCHK(c, nq_launch_sv(c->Y.p, f64, Ns, R, nA, offB, np, mu, p, eps, kind, diag, P<double>(c->cg_part), q, st));
         HIPCHK(c, nq_launch_dot(p, q, np, P<double>(c->cg_dpart), nparts, sc + 1, st));
         HIPCHK(c, nq_launch_cg_xr(x, r, p, q, np, sc, st));
         HIPCHK(c, nq_launch_dot(r, r, np, P<double>(c->cg_dpart), nparts, sc + 2, st));
@@ -1672,8 +1651,7 @@ static nqh_status qlp_loop(nqh_ctx* c, double eps, int kind, double res0, int ma
     while (finite && !q.done(iteration)) {
         double betal, beta;
         q.begin(&betal, &beta);
-        HIPCHK(c, nq_launch_sv(c->Y.p, f64, Ns, R, nA, offB, np, mu, vc, eps, kind, diag, P<double>(c->cg_w),
-                               P<double>(c->cg_part), chunks, vn, st));
+        HIPCHK(c, nq_launch_sv(c->Y.p, f64, Ns, R, nA, offB, np, mu, vc, eps, kind, diag, P<double>(c->cg_part), vn, st));
         if (q.iters > 1) HIPCHK(c, nq_launch_mr_axpy(vn, vp, np, -beta, st));
         HIPCHK(c, nq_launch_dot(vc, vn, np, P<double>(c->cg_dpart), nparts, sc, st));
         HIPCHK(c, nq_launch_mr_orth(vn, vc, np, sc, st));
@@ -1730,8 +1708,7 @@ static nqh_status minres_solve(nqh_ctx* c, double eps, int kind, bool qlp) {
     gram_blocks(c, &nA, &nB, &offB);
     constexpr int chunks = 64, nparts = 64;
     nqh_status s;
-    if ((s = ensure(c, c->cg_w, sizeof(double) * 2 * (size_t)Ns)) ||
-        (s = ensure(c, c->cg_part, sizeof(double) * (size_t)chunks * R)) ||
+    if ((s = ensure(c, c->cg_part, sizeof(double) * (size_t)NQ_SV_GROUPS * R)) ||
         (s = ensure(c, c->mr_vw, sizeof(double) * 6 * (size_t)np)) ||
         (s = ensure(c, c->cg_diag, sizeof(double) * np)) || (s = ensure(c, c->cg_sc, sizeof(double) * 8)) ||
         (s = ensure(c, c->cg_dpart, sizeof(double) * nparts)))
@@ -1766,8 +1743,7 @@ static nqh_status minres_solve(nqh_ctx* c, double eps, int kind, bool qlp) {
     int it = 1;
     bool finite = std::isfinite(res0);
     while (finite && !(it > maxit || resnorm <= tolerance)) {
-        HIPCHK(c, nq_launch_sv(c->Y.p, f64, Ns, R, nA, offB, np, mu, vc, eps, kind, diag, P<double>(c->cg_w),
-                               P<double>(c->cg_part), chunks, vn, st));
+        HIPCHK(c, nq_launch_sv(c->Y.p, f64, Ns, R, nA, offB, np, mu, vc, eps, kind, diag, P<double>(c->cg_part), vn, st));
         if (it > 1) HIPCHK(c, nq_launch_mr_axpy(vn, vp, np, -h2, st));
         HIPCHK(c, nq_launch_dot(vc, vn, np, P<double>(c->cg_dpart), nparts, sc, st));
         HIPCHK(c, nq_launch_mr_orth(vn, vc, np, sc, st));
@@ -1836,8 +1812,7 @@ static nqh_status lsqr_solve(nqh_ctx* c, double eps, int kind) {
     gram_blocks(c, &nA, &nB, &offB);
     constexpr int chunks = 64, nparts = 64;
     nqh_status s;
-    if ((s = ensure(c, c->cg_w, sizeof(double) * 2 * (size_t)Ns)) ||
-        (s = ensure(c, c->cg_part, sizeof(double) * (size_t)chunks * R)) ||
+    if ((s = ensure(c, c->cg_part, sizeof(double) * (size_t)NQ_SV_GROUPS * R)) ||
         (s = ensure(c, c->mr_vw, sizeof(double) * 6 * (size_t)np)) ||
         (s = ensure(c, c->cg_diag, sizeof(double) * np)) || (s = ensure(c, c->cg_sc, sizeof(double) * 8)) ||
         (s = ensure(c, c->cg_dpart, sizeof(double) * nparts)))
@@ -1851,8 +1826,7 @@ static nqh_status lsqr_solve(nqh_ctx* c, double eps, int kind) {
     const double* F = P<double>(c->F);
     hipStream_t st = c->stream;
     auto sv = [&](const double* in, double* out) {
-        return nq_launch_sv(c->Y.p, f64, Ns, R, nA, offB, np, mu, in, eps, kind, diag, P<double>(c->cg_w),
-                            P<double>(c->cg_part), chunks, out, st);
+        return nq_launch_sv(c->Y.p, f64, Ns, R, nA, offB, np, mu, in, eps, kind, diag, P<double>(c->cg_part), out, st);
     };
     auto read = [&](double* h, int n) -> hipError_t {
         hipError_t e = hipMemcpyAsync(h, sc, sizeof(double) * n, hipMemcpyDeviceToHost, st);
