@@ -1440,8 +1440,8 @@ __global__ __launch_bounds__(512, CLS < 2 ? 4 : 2) void k_force_mma_pk(const nq_
 // from the angles themselves where the weights leave the range or the tables do not fit.  Per four
 // connections 12 products of 64 cycles against about 170 VALU instructions, on different pipes.  The
 // form it replaces, one unit per lane with the flipped site indexing a register vector and exp, sincos
-// and divides per unit, took 0.97 ms alone on the trained-chain 4x4 XYZ workload of 16384 samples and 2.2 ms beside the S
-// build; this one 0.36 both ways (12 sites: 0.6 -> 0.16).
+// and divides per unit, took 0.97 ms alone on 4x4 XYZ with 16384 samples (2.2 beside the S build);
+// this one 0.36 (12 sites, beside: 0.6 -> 0.16).
 //   LDS: HW [N + 1][SW], PU [N][SP], PD [SP] as above in double, then up, dn [N][SW], pup, pdn [N][SP]
 typedef double d4v __attribute__((ext_vector_type(4)));
 
