@@ -207,12 +207,15 @@ __device__ __forceinline__ void metropolis_body(const samp_args& a, int bx) {
 // proposals 4.49 -> 0.81 ms.
 //
 // The constants k = e^(-m / 2), m the largest |K theta| a unit can reach, centre every factor; the
-// sum of the ranges over the units bounds every partial product, and where it leaves
-// e^(+-kRatioRange), or a bias e^(+-kRatioBias), the chains run through metropolis_body instead
-// (no weight of a network near that: N = nh = na = 16, 32, 32 reaches it at weights of order 1).
+// sum of the ranges over the units bounds every product over them.  That does not bound a unit alone:
+// its kept factor goes from e^(-1.5 m) to e^(m / 2) and its table entries reach e^(+-2 m), so every
+// unit also stays within m <= kUnitRange.  Where a unit leaves that, the sum leaves e^(+-kRatioRange),
+// or a bias e^(+-kRatioBias), the chains run through metropolis_body instead, at the price of the
+// former times.  With N = 16, nh = na = 32 the sum does so at a mean |w| of about 0.65 (softplus) or
+// 0.33 (logcosh).
 // Rounding of the kept factors: one product per accepted flip, set again from the configuration
 // at least every kRatioRefresh proposals or every call, whichever is longer.
-constexpr double kRatioRange = 600.0, kRatioBias = 60.0;
+constexpr double kRatioRange = 600.0, kUnitRange = 300.0, kRatioBias = 60.0;
 constexpr int kRatioRefresh = 64;
 
 // LDS bytes of the tables: e^(+-2 K w) per (site, lambda unit), two complex factors per (site, Pi
@@ -264,7 +267,7 @@ __device__ __forceinline__ bool metropolis_ratio_body(const samp_args& a, int bx
             }
             kl[r] = exp(-0.5 * K * m);
             e0[r] = exp(K * t - 0.5 * K * m);
-            range += 0.5 * K * m + 0.7;
+            range += K * m <= kUnitRange ? 0.5 * K * m + 0.7 : HUGE_VAL;
         }
         if (au[r] >= 0) {
             double t = gp[d.dla + u], m = fabs(t);
@@ -275,7 +278,7 @@ __device__ __forceinline__ bool metropolis_ratio_body(const samp_args& a, int bx
             }
             kp[r] = exp(-0.5 * K * m);
             w0[r] = exp(K * t - 0.5 * K * m);
-            range += K * m + 1.4;
+            range += K * m <= kUnitRange ? K * m + 1.4 : HUGE_VAL;
         }
     }
     range = group_total(range, lpc);
