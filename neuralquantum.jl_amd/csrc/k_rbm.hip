@@ -435,9 +435,10 @@ __global__ __launch_bounds__(256) void k_rbm_metropolis(rbm_samp_args a) {
 // biases, w = e^theta, and a flipped site multiplies w by e^(+-2 W), a table entry (on the diagonal,
 // log p = Re log rho, the square of the ratio, compared with u^2).  Kept per lane: k w, k = e^(-m / 2)
 // with m the largest |Re theta| of the unit; per chain: the product of k^2 |1 + w|^2.  Weights whose
-// products leave e^(+-kRbmRange) run through rbm_metropolis_body.  RBMSplit of 8 sites, 16 units, 256
+// products leave e^(+-kRbmRange), or with a unit beyond m = kRbmUnit (its kept factor goes down to
+// e^(-1.5 m), its table entries to e^(+-2 m)), run through rbm_metropolis_body.  RBMSplit of 8 sites, 16 units, 256
 // chains, 1122 proposals: 1.18 -> 0.27 ms; ket RBM of 16 sites, 32 units, 1024 chains, 136: 156 -> 56 us.
-constexpr double kRbmRange = 600.0, kRbmBias = 60.0;
+constexpr double kRbmRange = 600.0, kRbmUnit = 300.0, kRbmBias = 60.0;
 constexpr int kRbmRefresh = 64;
 
 __host__ __device__ inline size_t rbm_ratio_lds(const rbm_samp_args& a) {
@@ -490,7 +491,7 @@ __device__ __forceinline__ bool rbm_ratio_body(const rbm_samp_args& a) {
             const double e = exp(t.re - 0.5 * m);
             k[r] = exp(-0.5 * m);
             w0[r] = cmk(e * cs, e * sn);
-            range += m + 1.4;
+            range += m <= kRbmUnit ? m + 1.4 : HUGE_VAL;
         }
     }
     range = group_total(range, LPC);
