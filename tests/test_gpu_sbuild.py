@@ -65,3 +65,26 @@ def test_gram_chunks_match_cpu_gram(gpu_ok, sprec, N, alpha, chains, Lc):
     assert rel_err(S, S_cpu) < (1e-12 if sprec == _lib.PREC_FP64 else 1e-5)
     assert np.array_equal(S, S.T)
     ctx.close()
+
+
+def test_fp32_rows_are_centred_in_fp64(gpu_ok):
+    """An FP32 network's rows are centred in FP64 and rounded once, as an FP64
+    network's are: with every parameter zero the rows of both are the same
+    numbers (halves, quarters and zeros), so S is the same bit for bit; six
+    and fourteen samples give means that no float holds."""
+    N, out = 4, []
+    for chains in (3, 7):
+        keys = random_keys(N, 2 * chains, seed=90 + chains)
+        for prec in (_lib.PREC_FP64, _lib.PREC_FP32):
+            ctx = Context(0, 1)
+            ctx.set_problem(ising(N)[0])
+            ctx.set_ndm(N, 2 * N, N)
+            ctx.set_params(np.zeros(ctx.np_))
+            ctx.set_precision(prec, _lib.PREC_FP32)
+            _, O = ctx.logpsi_grad(keys)
+            _, S, _, _ = ctx.grad_from_samples(keys, chains, 2)
+            out.append((O, S))
+            ctx.close()
+        (O64, S64), (O32, S32) = out[-2:]
+        assert np.array_equal(O64, O32)
+        assert np.array_equal(S64, S32)
