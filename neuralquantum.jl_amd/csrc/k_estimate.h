@@ -1651,7 +1651,6 @@ __device__ __forceinline__ void force64_samples(const est_args& a, int64_t gw, i
         // every kForceFlush samples and after the wave's last one into the exact accumulator: product
         // entry (row lane / 16 + 4 v, column lane % 16) of each tile, the bias sums over the four groups
         if (++nacc == kForceFlush || s + nw >= a.Ns) {
-            nacc = 0;
             const int PB_bla = 0, PB_hla = N, PB_wla = N + nh;
             const int PB_d = d.nlam, PB_ula = d.nlam + na, PB_umu = d.nlam + na + na * N;
             const int PB_bmu = d.nlam + d.npi, PB_hmu = PB_bmu + N, PB_wmu = PB_hmu + nh;
@@ -1662,13 +1661,13 @@ __device__ __forceinline__ void force64_samples(const est_args& a, int64_t gw, i
                     for (int v = 0; v < 4; ++v) {
                         const int u = 16 * t + kg + 4 * v;
                         if (u < 2 * nh && il < N)
-                            fx_add(sF, (u < nh ? PB_wla + u : PB_wmu + u - nh) + nh * il, Fw[t][v], poison);
+                            fx_add_sum(sF, (u < nh ? PB_wla + u : PB_wmu + u - nh) + nh * il, Fw[t][v], nacc, poison);
                     }
                     double h = hb[t];
                     h += __shfl_xor(h, 16, 64);
                     h += __shfl_xor(h, 32, 64);
                     const int u = 16 * t + il;
-                    if (kg == 0 && u < 2 * nh) fx_add(sF, u < nh ? PB_hla + u : PB_hmu + u - nh, h, poison);
+                    if (kg == 0 && u < 2 * nh) fx_add_sum(sF, u < nh ? PB_hla + u : PB_hmu + u - nh, h, nacc, poison);
                 }
                 Fw[t] = zero;
                 hb[t] = 0.0;
@@ -1680,14 +1679,14 @@ __device__ __forceinline__ void force64_samples(const est_args& a, int64_t gw, i
                     for (int v = 0; v < 4; ++v) {
                         const int au = 16 * t + kg + 4 * v;
                         if (au < na && il < N) {
-                            fx_add(sF, PB_ula + au + na * il, Fr[t][v], poison);
-                            fx_add(sF, PB_umu + au + na * il, Fi[t][v], poison);
+                            fx_add_sum(sF, PB_ula + au + na * il, Fr[t][v], nacc, poison);
+                            fx_add_sum(sF, PB_umu + au + na * il, Fi[t][v], nacc, poison);
                         }
                     }
                     double h = db[t];
                     h += __shfl_xor(h, 16, 64);
                     h += __shfl_xor(h, 32, 64);
-                    if (kg == 0 && 16 * t + il < na) fx_add(sF, PB_d + 16 * t + il, h, poison);
+                    if (kg == 0 && 16 * t + il < na) fx_add_sum(sF, PB_d + 16 * t + il, h, nacc, poison);
                 }
                 Fr[t] = Fi[t] = zero;
                 db[t] = 0.0;
@@ -1698,10 +1697,11 @@ __device__ __forceinline__ void force64_samples(const est_args& a, int64_t gw, i
             bm += __shfl_xor(bm, 16, 64);
             bm += __shfl_xor(bm, 32, 64);
             if (kg == 0 && il < N) {
-                fx_add(sF, PB_bla + il, bl, poison);
-                fx_add(sF, PB_bmu + il, bm, poison);
+                fx_add_sum(sF, PB_bla + il, bl, nacc, poison);
+                fx_add_sum(sF, PB_bmu + il, bm, nacc, poison);
             }
             vbl = vbm = 0.0;
+            nacc = 0;
         }
     }
 }

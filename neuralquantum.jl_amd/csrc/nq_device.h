@@ -243,6 +243,19 @@ __device__ __forceinline__ void fx_add(unsigned long long* acc, int k, double v,
 __device__ __forceinline__ double fx_value(const unsigned long long* acc, int k) {
     return (double)(long long)acc[2 * k] * 0x1p-20 + (double)(long long)acc[2 * k + 1] * 0x1p-64;
 }
+// the same for v a sum of n <= 8 addends of that bound, |v| < n 2^30: beyond 2^30 as eight times v / 8,
+// which is exact (a multiple of 2^-25)
+__device__ __forceinline__ void fx_add_sum(unsigned long long* acc, int k, double v, int n, int* poison) {
+    if (!(fabs(v) < 1073741824.0 * n)) {
+        atomicOr(poison, 1);
+        return;
+    }
+    const int sh = fabs(v) < 1073741824.0 ? 0 : 3;
+    long long hi, lo;
+    fx_split(sh ? 0.125 * v : v, &hi, &lo);
+    atomicAdd(acc + 2 * k, (unsigned long long)hi << sh);
+    atomicAdd(acc + 2 * k + 1, (unsigned long long)lo << sh);
+}
 // LDS bytes of an accumulator of n entries plus its poison word (16-aligned)
 __host__ __device__ inline int fx_bytes(int n) { return 16 * n + 16; }
 
