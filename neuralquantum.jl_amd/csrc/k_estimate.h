@@ -1820,9 +1820,11 @@ __global__ NQ_EST_BOUNDS void k_estimate_pk(const nq_pk_member* M, const uint2* 
 // waves per workgroup of a launch: 8 share one copy of the parameters, the
 // force accumulator and the table (two blocks per CU while that fits in half
 // the LDS: 4 waves per SIMD); otherwise 4.  The parity mode (per-sample
-// gradients) runs one wave per block.
+// gradients) runs one wave per block.  The FP64 forces go down to 2: their
+// padded tiles leave less of the LDS to the records than the parameters alone.
 inline int est_waves(const est_args& a, size_t elt) {
     if (a.G) return 1;
+    if (elt == 8 && a.rec_mode == 2 && est_lds_bytes(a, elt, 4) > 160 * 1024) return 2;
     if (a.waves == 4) return 4;
     if (elt == 8 && a.rec_mode == 2 && force_class(a.d) == 2) return 4;   // its launch bound
     if (a.waves == 8 && est_lds_bytes(a, elt, 8) <= 160 * 1024) return 8;

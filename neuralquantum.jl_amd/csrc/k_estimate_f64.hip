@@ -32,7 +32,8 @@ hipError_t nq_launch_estimate(const est_args& a0, bool fp64, int grid, hipStream
     nq_est_tables(a, fp64);
     est_args b = a;
     if (b.rec_mode == 2) b.tab_lds = 0;
-    if (est_lds_bytes(b, fp64 ? 8 : 4, b.G ? 1 : 4) > 160 * 1024) return hipErrorInvalidValue;
+    if (est_lds_bytes(b, fp64 ? 8 : 4, b.G ? 1 : (fp64 && b.rec_mode == 2 ? 2 : 4)) > 160 * 1024)
+        return hipErrorInvalidValue;
     if (fp64) return nq_est::launch_prec<double>(a, grid, st);
     return nq_launch_estimate_f32(a, grid, st);
 }

@@ -1,6 +1,9 @@
-"""The FP64 forces' exact sums at the end of their range: entries whose
-samples stay below the accumulator's bound of 2^30 although eight of them
-together do not."""
+"""The FP64 forces' exact sums and records at the ends of their range:
+entries whose samples stay below the accumulator's bound of 2^30 although
+eight of them together do not, and connection tables whose records fit in LDS
+only beside fewer waves."""
+import dataclasses
+
 import numpy as np
 import pytest
 
@@ -38,3 +41,30 @@ def test_samples_below_the_bound_whose_sum_is_not(gpu_ok, ref):
     assert rel_err(st, st_r) < 1e-10
     assert rel_err(F, F_r) < 1e-10
     ctx.close()
+
+
+def test_long_records(gpu_ok):
+    """The chain's table of 16 sites repeated until a configuration has 1280
+    connections, with nh = 1 and na = 33 (tiles of 64 units of each kind):
+    four waves' records fit beside the parameters (up to 1417 connections),
+    but not beside the tiles (1156).  L_loc grows by the number of repeats and
+    the force by its square."""
+    N, nh, na, lo, hi = 16, 1, 33, 1157, 1417
+    flat, _, _ = ising(N)
+    k = hi // flat.max_connections()
+    assert lo <= k * flat.max_connections() <= hi
+    rep = dataclasses.replace(flat, **{f: np.tile(getattr(flat, f), k) for f in ("term_kind", "term_op_l", "term_op_r")})
+    keys = random_keys(N, 40, seed=5)
+    out = []
+    for t in (flat, rep):
+        ctx = Context(0, 1)
+        ctx.set_problem(t)
+        ctx.set_ndm(N, nh, na)
+        ctx.set_params(params(ctx.np_, seed=6, sigma=0.1))
+        ctx.set_precision(_lib.PREC_FP64, _lib.PREC_FP64)
+        L = ctx.local_estimator(keys)
+        _, _, F, _ = ctx.grad_from_samples(keys, 20, 2)
+        out.append((L, F))
+        ctx.close()
+    assert rel_err(out[1][0], k * out[0][0]) < 1e-12
+    assert rel_err(out[1][1], k * k * out[0][1]) < 1e-12
