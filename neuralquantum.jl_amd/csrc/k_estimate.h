@@ -147,11 +147,14 @@ __device__ __forceinline__ bool ratio_fill(const ratio_tables& t, const double* 
         atomicMax(reinterpret_cast<unsigned long long*>(t.range) + (u < 2 * nh ? 0 : 1),
                   (unsigned long long)__double_as_longlong(K * m));
     }
+    // per site the sum over the units, 16 threads each, in a fixed order: the route must not depend on
+    // the order in which waves or workgroups run
     for (int k = threadIdx.x; k < N * 16; k += blockDim.x) {
         const int i = k >> 4;
         double m = 0.0;
         for (int u = k & 15; u < units; u += 16) m += 2.0 * K * fabs(weight(u, i));
-        atomicAdd(t.range + 2 + i, m);
+        m = group_total(m, 16);
+        if ((k & 15) == 0) t.range[2 + i] = m;
     }
     for (int i = threadIdx.x; i < N; i += blockDim.x) {
         double bl = gp[d.bla + i], bm = gp[d.bmu + i];

@@ -42,3 +42,27 @@ def test_walk_matches_the_oracle(gpu_ok, model, N, nh, na, sigma, act):
     if np.max(np.abs(F_r)) < 2.0 ** 30:   # the exact force sums take addends below 2^30 (NaN beyond, as sigma 4 is)
         assert rel_err(F, F_r) < 1e-10
     ctx.close()
+
+
+def test_route_at_the_threshold_is_one(gpu_ok):
+    """A site whose sum over the units stands at the products' bound, where the
+    order of the sum decides: every workgroup, and every call, takes the same
+    route, so equal configurations give equal L_loc bit for bit."""
+    N, nh, na = 4, 32, 32
+    ref = nqref.Ref()
+    p = np.zeros(ref.ndm_np(N, nh, na))
+    off = nqref.ndm_layout(N, nh, na)[0]
+    for block, rows in (("w_la", nh), ("w_mu", nh), ("u_la", na)):
+        first, count = off[block]
+        p[first:first + count].reshape(N, rows)[0] = 1.0e-14     # 2 w below half a unit in the last place of 300
+    p[off["w_la"][0]] = 150.0                                     # two flips of 2 |w| reach the bound of 600
+    ctx = Context(0, 1)
+    ctx.set_problem(ising(N)[0])
+    ctx.set_ndm(N, nh, na)
+    ctx.set_params(p)
+    ctx.set_precision(_lib.PREC_FP64, _lib.PREC_FP64)
+    base = random_keys(N, 16, seed=8)
+    first = ctx.local_estimator(base)
+    for _ in range(3):
+        assert np.array_equal(ctx.local_estimator(np.tile(base, 1024)), np.tile(first, 1024))
+    ctx.close()
