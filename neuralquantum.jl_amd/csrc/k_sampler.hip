@@ -512,7 +512,8 @@ __global__ __launch_bounds__(256) void k_metropolis_pk(const nq_pk_member* M, co
     if constexpr (sizeof(T) == 8) {
         if (a.lpc == 8) metropolis_f64<8, 1, ACT>(a, bx);
         else if (a.lpc == 16) metropolis_f64<16, 1, ACT>(a, bx);
-        else metropolis_f64<32, 1, ACT>(a, bx);
+        else if (a.lpc == 32) metropolis_f64<32, 1, ACT>(a, bx);
+        else metropolis_body<T, 1, ACT>(a, bx);   // fewer lanes: more chains than block records at 8
     } else {
         metropolis_body<T, 1, ACT>(a, bx);
     }

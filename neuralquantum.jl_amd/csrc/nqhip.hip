@@ -2422,6 +2422,11 @@ nq_pk_member pk_describe(nqh_ctx* c, double eps, int kind, double lr) {
     a.accepted = P<unsigned long long>(c->acc);
     a.chain_acc = P<uint32_t>(c->chain_acc);
     a.waves = c->tune_samp_waves;
+    // a block record numbers 2^16 workgroups: 2 million chains at the 8 lanes that FP64 takes at least;
+    // beyond that the chains by sums of f, on no more lanes than units
+    int samp_threads, samp_grid;
+    size_t samp_lds;
+    if (nq_sampler_variant(a, f64, &samp_threads, &samp_lds, &samp_grid) < 0) a.lpc = nq_sampler_lanes_per_chain(d, false);
     // the estimator's two launches (run_grad_pipeline)
     est_args e = make_est(c, P<uint64_t>(c->samples), Ns);
     e.do_conn = 1;

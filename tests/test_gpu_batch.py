@@ -177,3 +177,30 @@ def test_packed_batch_falls_back_for_members_it_does_not_cover(gpu_ok, ref):
         batch.close()
         for c in alone + inb:
             c.close()
+
+
+def test_packed_fp64_member_of_millions_of_chains(gpu_ok, ref):
+    """One chain per few lanes: more than 2^16 workgroups at eight lanes a
+    chain, which the packed launch's block records cannot number."""
+    def one(chains, seed):
+        ctx = Context(0, seed)
+        ctx.set_problem(ising(1, periodic=False)[0])
+        ctx.set_ndm(1, 1, 1)
+        ctx.set_params(params(ref.ndm_np(1, 1, 1), seed=seed, sigma=0.3))
+        ctx.set_precision(_lib.PREC_FP64, _lib.PREC_FP64)
+        ctx.set_sampler(chains, 2, 3, 1, 0)
+        ctx.set_iteration(0)
+        return ctx
+
+    chains = 32 * 0xffff + 5
+    alone, inb = one(chains, 3), [one(chains, 3), one(64, 4)]
+    batch = Batch(inb)
+    for _ in range(2):
+        st, sa = batch.sr_iteration(0.01, 0.01), alone.sr_iteration(0.01, 0.01)
+        assert batch.launches() > 0
+        assert rel_err(st[0][:1], sa[:1]) < 1e-12
+        assert np.array_equal(inb[0].get_samples(), alone.get_samples())
+    assert rel_err(inb[0].get_params(), alone.get_params()) < 1e-12
+    batch.close()
+    for c in inb + [alone]:
+        c.close()
