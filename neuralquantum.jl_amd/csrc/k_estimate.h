@@ -90,9 +90,10 @@ template <typename T> constexpr int est_batch() { return sizeof(T) == 8 ? 4 : 8;
 // Pi tiles of 16), then products over the 16 lanes.  Bound by FP64 issue at two waves per SIMD.
 // Before and now: 4x4 XYZ, 16384 samples 1.44 -> 0.34 ms; 12 sites, 16384 samples 0.66 -> 0.19;
 // the exact sum over 2^20 configurations of 10 sites 34.4 -> 7.7.
-// The ranges keep every partial product inside e^(+-700); a network whose weights leave them (or whose
-// tables do not fit in LDS beside the connections) takes the sums of f instead.
-constexpr double kEstRange = 600.0;
+// The ranges of the units and the bound of the visible biases, whose exponential is a factor of its
+// own, keep every partial product inside e^(+-700); a network whose weights leave them (or whose tables
+// do not fit in LDS beside the connections) takes the sums of f instead.
+constexpr double kEstRange = 600.0, kEstBias = 100.0;
 
 // doubles: e^(2 K w) and e^(-2 K w) of (site, lambda or mu, unit); complex e^(+-K (u_la + i u_mu)) of
 // (site, Pi unit); the effective biases (la, mu) of a site; scratch of the ranges
@@ -172,7 +173,8 @@ __device__ __forceinline__ bool ratio_fill(const ratio_tables& t, const double* 
     }
     __syncthreads();
     bool ok = th * (t.range[0] + 0.7) <= kEstRange && tp * (t.range[1] + 0.7) <= 0.5 * kEstRange;
-    for (int i = 0; i < N; ++i) ok = ok && fmax * t.range[2 + i] <= kEstRange;
+    for (int i = 0; i < N; ++i)
+        ok = ok && fmax * t.range[2 + i] <= kEstRange && fmax * fabs(t.bias[i].x) <= kEstBias;
     return ok;
 }
 

@@ -66,3 +66,27 @@ def test_route_at_the_threshold_is_one(gpu_ok):
     for _ in range(3):
         assert np.array_equal(ctx.local_estimator(np.tile(base, 1024)), np.tile(first, 1024))
     ctx.close()
+
+
+def test_visible_bias_against_a_unit(gpu_ok):
+    """A visible bias of 720 on one site against a Pi unit that takes 70 of it
+    back: e^650 is in range although e^720 is not.  1e-10 relative."""
+    N, nh, na = 3, 2, 2
+    ref = nqref.Ref()
+    flat, tab, _ = ising(N)
+    p = params(ref.ndm_np(N, nh, na), seed=61, sigma=0.1)
+    off = nqref.ndm_layout(N, nh, na)[0]
+    p[off["b_la"][0]] = 720.0
+    p[off["d_la"][0]] = 70.0
+    p[off["u_la"][0]] = -70.0
+    ctx = Context(0, 1)
+    ctx.set_problem(flat)
+    ctx.set_ndm(N, nh, na)
+    ctx.set_params(p)
+    ctx.set_precision(_lib.PREC_FP64, _lib.PREC_FP64)
+    keys = np.arange(1 << (2 * N), dtype=np.uint64)
+    L = ctx.local_estimator(keys)
+    L_r, _ = ref.local_estimator(tab, nh, na, p, keys)
+    assert np.all(np.isfinite(L_r)) and np.max(np.abs(L_r)) > 1e270
+    assert np.max(np.abs(L - L_r) / np.maximum(np.abs(L_r), 1.0)) < 1e-10
+    ctx.close()
