@@ -43,10 +43,13 @@ __device__ __forceinline__ void metropolis_body(const samp_args& a, int bx) {
     const int lpc = a.lpc;
     const int lane = threadIdx.x & 63;
     const int g = lane & (lpc - 1);
-    const int gbase = lane - g;
-    const int cpw = 64 / lpc;
+    // the chain's lanes: rep copies of the group (FP64), which share the random draws
+    const int width = lpc * a.rep;
+    const int gw = lane & (width - 1);
+    const int gbase = lane - gw;
+    const int cpw = 64 / width;
     const int64_t wave_glob = (int64_t)bx * (blockDim.x >> 6) + (threadIdx.x >> 6);
-    const int64_t chain = wave_glob * cpw + lane / lpc;
+    const int64_t chain = wave_glob * cpw + lane / width;
     const bool live = chain < a.chains;
     const uint32_t pmask = (N >= 32) ? 0xffffffffu : ((1u << N) - 1u);
     const uint32_t k0 = (uint32_t)a.seed, k1 = (uint32_t)(a.seed >> 32);
@@ -108,9 +111,9 @@ __device__ __forceinline__ void metropolis_body(const samp_args& a, int bx) {
             }
         }
         for (int q = 0; q < a.passes; ++q, ++t) {
-            const int slot = (int)((t - a.t0) % (uint32_t)lpc);
+            const int slot = (int)((t - a.t0) % (uint32_t)width);
             if (slot == 0) {
-                philox_out o = philox4x32_10(t + (uint32_t)g, iter, (uint32_t)chain, ctr3 + 1u, k0, k1);
+                philox_out o = philox4x32_10(t + (uint32_t)gw, iter, (uint32_t)chain, ctr3 + 1u, k0, k1);
                 rx0 = o.x[0]; rx1 = o.x[1]; rx2 = o.x[2];
             }
             const uint32_t x0 = __shfl(rx0, gbase + slot, 64);
@@ -138,17 +141,11 @@ __device__ __forceinline__ void metropolis_body(const samp_args& a, int bx) {
                     delta += nf[r] - (col ? f_e[r] : f_s[r]);
                 }
                 if (h < na) {
-                    if (diag) {
-                        nz[r].re += c * sp[d.ula + h + na * j];
-                        nfpi[r] = cact_re<ACT>(nz[r]);
-                        delta += nfpi[r] - fpi[r];
-                    } else {
-                        const T cu = c * half;
-                        nz[r].re += cu * sp[d.ula + h + na * j];
-                        nz[r].im += (col ? -cu : cu) * sp[d.umu + h + na * j];
-                        nfpi[r] = cact_re<ACT>(nz[r]);
-                        delta += T(2) * (nfpi[r] - fpi[r]);
-                    }
+                    const T cu = diag ? c : c * half;
+                    nz[r].re += cu * sp[d.ula + h + na * j];
+                    if (!diag) nz[r].im += (col ? -cu : cu) * sp[d.umu + h + na * j];
+                    nfpi[r] = cact_re<ACT>(nz[r]);
+                    delta += (diag ? T(1) : T(2)) * (nfpi[r] - fpi[r]);
                 }
             }
             delta = group_total(delta, lpc);
@@ -177,12 +174,12 @@ __device__ __forceinline__ void metropolis_body(const samp_args& a, int bx) {
                 }
             }
         }
-        if (call >= a.burn && live && g == 0 && a.samples) {
+        if (call >= a.burn && live && gw == 0 && a.samples) {
             const int slice = a.slice0 + call - a.burn;
             a.samples[chain + (int64_t)slice * a.chains] = key;
         }
     }
-    if (live && g == 0) {
+    if (live && gw == 0) {
         if (a.chain_state) a.chain_state[chain] = key;
         if (a.compat_stale_last_slice && a.samples)
             a.samples[chain + (int64_t)(a.stored) * a.chains] = 0ull;   // defect D1: slice L stays at the fill
@@ -494,9 +491,7 @@ template <int LPC, int US, int ACT>
 __device__ __forceinline__ void metropolis_f64(const samp_args& a, int bx) {
     if (a.diag ? metropolis_ratio_body<LPC, US, ACT, true>(a, bx) : metropolis_ratio_body<LPC, US, ACT, false>(a, bx)) return;
     __syncthreads();
-    samp_args w = a;
-    w.lpc = LPC * a.rep;   // the chain's lanes as one group
-    metropolis_body<double, US, ACT>(w, bx);
+    metropolis_body<double, US, ACT>(a, bx);
 }
 template <int LPC, int US, int ACT>
 __global__ __launch_bounds__(256) void k_metropolis_f64(samp_args a) {

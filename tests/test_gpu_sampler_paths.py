@@ -17,7 +17,7 @@ pytestmark = pytest.mark.gpu
 # products leave e^(+-600) (sigma 3 at nh = 64: the range is about 0.5 (N + 1) 0.8 sigma nh)
 SHAPES = [(3, 1, 1, 0.5, 2), (4, 8, 5, 0.5, 37), (4, 9, 3, 0.5, 40), (5, 16, 17, 0.4, 33), (3, 33, 20, 0.3, 21),
           (4, 64, 64, 0.2, 9), (3, 18, 32, 0.3, 2060), (3, 32, 18, 0.3, 4100), (3, 40, 12, 0.3, 2060),
-          (4, 64, 64, 3.0, 9), (3, 18, 32, 6.0, 2060)]
+          (4, 64, 64, 3.0, 9), (3, 18, 32, 6.0, 2060), (6, 6, 6, 20.0, 16)]
 
 
 @pytest.mark.parametrize("act", [0, 1])
