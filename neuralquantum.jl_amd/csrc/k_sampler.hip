@@ -46,7 +46,7 @@ __device__ __forceinline__ void metropolis_body(const samp_args& a, int bx) {
     // the chain's lanes: rep copies of the group (FP64), which share the random draws
     const int width = lpc * a.rep;
     const int gw = lane & (width - 1);
-    const int gbase = lane - gw;
+    const int gbase = lane - g;
     const int cpw = 64 / width;
     const int64_t wave_glob = (int64_t)bx * (blockDim.x >> 6) + (threadIdx.x >> 6);
     const int64_t chain = wave_glob * cpw + lane / width;
@@ -111,9 +111,9 @@ __device__ __forceinline__ void metropolis_body(const samp_args& a, int bx) {
             }
         }
         for (int q = 0; q < a.passes; ++q, ++t) {
-            const int slot = (int)((t - a.t0) % (uint32_t)width);
+            const int slot = (int)((t - a.t0) % (uint32_t)lpc);
             if (slot == 0) {
-                philox_out o = philox4x32_10(t + (uint32_t)gw, iter, (uint32_t)chain, ctr3 + 1u, k0, k1);
+                philox_out o = philox4x32_10(t + (uint32_t)g, iter, (uint32_t)chain, ctr3 + 1u, k0, k1);
                 rx0 = o.x[0]; rx1 = o.x[1]; rx2 = o.x[2];
             }
             const uint32_t x0 = __shfl(rx0, gbase + slot, 64);
