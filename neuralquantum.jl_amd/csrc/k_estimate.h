@@ -19,7 +19,7 @@
 //
 // Three kinds of launch (template parameter KIND, and the forces):
 //   EK_WALK   log rho, O rows, and pass 1 over the connections: FP64 by
-//             products of the units' factors, FP32 (and FP64 weights outside
+//             products over the units, FP32 (and FP64 weights outside
 //             their range) by softplus (or logcosh) of the changed angles +
 //             one wave reduction -> W_c
 //             = mel_c exp(log rho_c - log rho_s), L_loc = sum_c W_c; with
@@ -76,67 +76,80 @@ __device__ __forceinline__ int p2ref(int k, const ndm_dims& d) {
 template <typename T> constexpr int est_batch() { return sizeof(T) == 8 ? 4 : 8; }
 
 // ---- FP64 connections by products (the walk; the forces below)
-// e^(dlog rho) of a connection is a product over the units, as in the sampler: with E = e^(K theta),
-// w = e^(K z) (K = 1 softplus, 2 logcosh, whose linear parts join the visible biases)
-//   |.|   = sqrt(prod over lambda units of (1 + E') / (1 + E)) |prod over Pi units of (1 + w') / (1 + w)|
-//   phase = (1/2) log(prod over mu units of (1 + E') / (1 + E)) (row side; minus, column side) + the
-//           phase of the complex Pi product
-// and E' = E e^(+-2 K w_i) per flipped site, from tables in LDS.  Per unit and connection that is one
-// product per flipped site, an addition and a product, in place of exp + log1p (real units) and exp +
-// sincos + log1p + atan2 (Pi units), about 360 instructions of the wave per connection; the square
-// root, logarithm, exponential and sincos that finish a connection are taken by one lane per
-// connection, 64 connections at a time.
+// e^(dlog rho) of a connection is a product over the units, as in the sampler.  Two forms, chosen by the
+// weights' size, each where its error is the smaller:
+//   differences  1 + d, d the relative change of cosh(K x / 2) (K = 1 softplus, 2 logcosh; softplus has a
+//       linear part that joins the visible biases): with t = tanh(K x / 2) of the sample's angle (2 f' - 1
+//       or f'), a flip that moves K x / 2 by +-v gives d = (cosh v - 1) +- t sinh v from tables; products
+//       are kept less one, p + q + p q, so that what is rounded is the change, not the value.
+//   factors      (1 + E') / (1 + E), E = e^(K x), E' = E e^(+-2 K w) per flipped site.
+//   |.|   = sqrt(product over lambda units) |product over Pi units|
+//   phase = (1/2) log(product over mu units) (row side; minus, column side) + the phase of the complex Pi
+//           product
+// Per unit and connection that is one FMA or product per flipped site and one combination, in place of
+// exp + log1p (real units) and exp + sincos + log1p + atan2 (Pi units), about 360 instructions of the
+// wave per connection; the square root, logarithm, exponential and sincos that finish a connection are
+// taken by one lane per connection, 64 connections at a time.
 // Four connections per round, lane i + 16 k taking connection k and its units 16 t + i (lambda, mu and
 // Pi tiles of 16), then products over the 16 lanes.  Bound by FP64 issue at two waves per SIMD.
-// Before and now: 4x4 XYZ, 16384 samples 1.44 -> 0.34 ms; 12 sites, 16384 samples 0.66 -> 0.19;
-// the exact sum over 2^20 configurations of 10 sites 34.4 -> 7.7.
+// By sums of f, by factors alone, and now: 4x4 XYZ, 16384 samples 1.44, 0.34, 0.39 ms; 12 sites, 16384
+// samples 0.66, 0.20, 0.22; the exact sum over 2^20 configurations of 10 sites 34.4, 7.7, 7.9.
+// Distance of L_loc from an 80-bit evaluation, 1e-16 (2-norm over 2-norm), in the same order: 6 sites,
+// weights of 0.1: 2.1, 3.7, 1.4; 12 sites, 0.05: 4.1, 8.1, 1.4; 3x3 XYZ, log cosh, 0.05: 14, 24, 4.6;
+// weights too large for the differences (8 sites, log cosh, 0.5): 600, 13 by factors.
 // The ranges of the units and the bound of the visible biases, whose exponential is a factor of its
 // own, keep every partial product inside e^(+-700); a network whose weights leave them (or whose tables
 // do not fit in LDS beside the connections) takes the sums of f instead.
 constexpr double kEstRange = 600.0, kEstBias = 100.0;
+// the differences' bound: the sum over the units of |K w|^2 at a site, times the sites a connection flips
+constexpr double kEstSmall = 24.5;
+enum { EST_SUMS = 0, EST_FACTORS = 1, EST_DIFFERENCES = 2 };
 
-// doubles: e^(2 K w) and e^(-2 K w) of (site, lambda or mu, unit); complex e^(+-K (u_la + i u_mu)) of
-// (site, Pi unit); the effective biases (la, mu) of a site; scratch of the ranges
+// units of a kind in the tables, padded to whole tiles of the walk, whose template takes as many for
+// both kinds
+__host__ __device__ inline int ratio_units(const ndm_dims& d) { return 32 * ((2 * max(d.nh, d.na) + 63) / 64); }
+// bytes: two doubles per (site, lambda or mu, unit), two complex per (site, Pi unit), the effective
+// biases (la, mu) of a site; the ranges
 __host__ __device__ inline int ratio_bytes(const ndm_dims& d) {
-    return (8 * (4 * d.N * d.nh + 4 * d.N * d.na + 2 * d.N + d.N + 4) + 15) & ~15;
+    return (8 * (8 * d.N * ratio_units(d) + 2 * d.N + 2 * d.N + 2) + 15) & ~15;
 }
 struct ratio_tables {
-    double *up, *dn;      // [(2 i + s) nh + h], s = 0 lambda, 1 mu
-    double2 *pup, *pdn;   // [i na + a]
-    double2* bias;        // [i]
-    double* range;        // max range of a real unit, of a Pi unit, then per site the sum over the units
+    double2* real;    // [(2 i + s) SH + h], s = 0 lambda, 1 mu: (cosh v - 1, sinh v) or factors of (up, down)
+    double2* pi;      // [2 (i SP + a)], two entries: the same for a Pi unit
+    double2* bias;    // [i]
+    double* range;    // max range of a real unit, of a Pi unit, then per site two sums over the units
 };
 __device__ __forceinline__ ratio_tables ratio_at(unsigned char* mem, const ndm_dims& d) {
     ratio_tables t;
-    t.pup = reinterpret_cast<double2*>(mem);
-    t.pdn = t.pup + d.N * d.na;
-    t.bias = t.pdn + d.N * d.na;
-    t.up = reinterpret_cast<double*>(t.bias + d.N);
-    t.dn = t.up + 2 * d.N * d.nh;
-    t.range = t.dn + 2 * d.N * d.nh;
+    t.real = reinterpret_cast<double2*>(mem);
+    t.pi = t.real + 2 * d.N * ratio_units(d);
+    t.bias = t.pi + 2 * d.N * ratio_units(d);
+    t.range = reinterpret_cast<double*>(t.bias + d.N);
     return t;
 }
-// fills the tables from the parameters gp (all threads; synchronises) and says whether the ranges hold:
+// sum of y^n / (2 n + 1)! and of y^n / (2 n)!: sinh x / x and cosh x at y = x^2, sin x / x and cos x at
+// y = -x^2; the tables' arguments stay within |y| <= kEstSmall / 4 (the terms left out are below 2e-18)
+__device__ __forceinline__ double odd_series(double y) {
+    double p = 1.0;
+#pragma unroll
+    for (int n = 14; n >= 1; --n) p = fma(p, y * (1.0 / (2.0 * n * (2.0 * n + 1.0))), 1.0);
+    return p;
+}
+__device__ __forceinline__ double even_series(double y) {
+    double p = 1.0;
+#pragma unroll
+    for (int n = 14; n >= 1; --n) p = fma(p, y * (1.0 / (2.0 * n * (2.0 * n - 1.0))), 1.0);
+    return p;
+}
+// fills the tables from the parameters gp (all threads; synchronises) and returns the form;
 // th, tp: real and Pi units a lane multiplies, fmax: sites a connection flips
 template <int ACT>
-__device__ __forceinline__ bool ratio_fill(const ratio_tables& t, const double* gp, const ndm_dims& d, int th, int tp,
-                                           int fmax) {
+__device__ __forceinline__ int ratio_fill(const ratio_tables& t, const double* gp, const ndm_dims& d, int th, int tp,
+                                          int fmax) {
     constexpr double K = ACT == NQ_ACT_LOGCOSH ? 2.0 : 1.0;
     const int N = d.N, nh = d.nh, na = d.na, units = 2 * nh + na;
-    for (int k = threadIdx.x; k < N + 4; k += blockDim.x) t.range[k] = 0.0;
-    for (int k = threadIdx.x; k < 2 * N * nh; k += blockDim.x) {
-        const int h = k % nh, is = k / nh, i = is >> 1;
-        const double e = exp(2.0 * K * gp[((is & 1) ? d.wmu : d.wla) + h + nh * i]);
-        t.up[k] = e;
-        t.dn[k] = 1.0 / e;
-    }
-    for (int k = threadIdx.x; k < N * na; k += blockDim.x) {
-        double s, c;
-        sincos(K * gp[d.umu + k], &s, &c);
-        const double e = exp(K * gp[d.ula + k]), r = 1.0 / e;
-        t.pup[k] = make_double2(e * c, e * s);
-        t.pdn[k] = make_double2(r * c, -r * s);
-    }
+    const int SH = 16 * th, SP = 16 * tp;
+    for (int k = threadIdx.x; k < 2; k += blockDim.x) t.range[k] = 0.0;
     __syncthreads();
     // unit u's weight at site i: lambda, mu, then the Pi units' real parts
     auto weight = [&](int u, int i) {
@@ -148,34 +161,94 @@ __device__ __forceinline__ bool ratio_fill(const ratio_tables& t, const double* 
         atomicMax(reinterpret_cast<unsigned long long*>(t.range) + (u < 2 * nh ? 0 : 1),
                   (unsigned long long)__double_as_longlong(K * m));
     }
-    // per site the sum over the units, 16 threads each, in a fixed order: the route must not depend on
+    // per site the sums over the units, 16 threads each, in a fixed order: the form must not depend on
     // the order in which waves or workgroups run
     for (int k = threadIdx.x; k < N * 16; k += blockDim.x) {
         const int i = k >> 4;
-        double m = 0.0;
-        for (int u = k & 15; u < units; u += 16) m += 2.0 * K * fabs(weight(u, i));
-        m = group_total(m, 16);
-        if ((k & 15) == 0) t.range[2 + i] = m;
-    }
-    for (int i = threadIdx.x; i < N; i += blockDim.x) {
-        double bl = gp[d.bla + i], bm = gp[d.bmu + i];
-        if constexpr (ACT == NQ_ACT_LOGCOSH) {
-            for (int h = 0; h < nh; ++h) {
-                bl -= gp[d.wla + h + nh * i];
-                bm -= gp[d.wmu + h + nh * i];
-            }
-            for (int q = 0; q < na; ++q) {
-                bl -= gp[d.ula + q + na * i];
-                bm -= gp[d.umu + q + na * i];
+        double m = 0.0, q = 0.0, bl = 0.0, bm = 0.0;
+        for (int u = k & 15; u < units; u += 16) {
+            const double w = weight(u, i);
+            m += 2.0 * K * fabs(w);
+            q += K * K * w * w;
+            bl += u < nh || u >= 2 * nh ? w : 0.0;
+            bm += u >= nh && u < 2 * nh ? w : 0.0;
+            if (u >= 2 * nh) {
+                const double v = gp[d.umu + u - 2 * nh + na * i];
+                q += K * K * v * v;
+                bm += v;
             }
         }
-        t.bias[i] = make_double2(bl, bm);
+        m = group_total(m, 16);
+        q = group_total(q, 16);
+        bl = group_total(bl, 16);
+        bm = group_total(bm, 16);
+        if ((k & 15) == 0) {
+            t.range[2 + 2 * i] = m;
+            t.range[3 + 2 * i] = q;
+            t.bias[i] = make_double2(bl, bm);
+        }
     }
     __syncthreads();
-    bool ok = th * (t.range[0] + 0.7) <= kEstRange && tp * (t.range[1] + 0.7) <= 0.5 * kEstRange;
-    for (int i = 0; i < N; ++i)
-        ok = ok && fmax * t.range[2 + i] <= kEstRange && fmax * fabs(t.bias[i].x) <= kEstBias;
-    return ok;
+    bool ok = th * (t.range[0] + 0.7) <= kEstRange && tp * (t.range[1] + 0.7) <= 0.5 * kEstRange, small = true;
+    for (int i = 0; i < N; ++i) {
+        ok = ok && fmax * t.range[2 + 2 * i] <= kEstRange;
+        small = small && fmax * t.range[3 + 2 * i] <= kEstSmall;
+    }
+    // the linear parts of f: x / 2 beside the differences of softplus, -x beside the factors of logcosh
+    const double lin = small ? (ACT == NQ_ACT_LOGCOSH ? 0.0 : 0.5) : (ACT == NQ_ACT_LOGCOSH ? -1.0 : 0.0);
+    for (int i = 0; i < N; ++i) ok = ok && fmax * fabs(gp[d.bla + i] + lin * t.bias[i].x) <= kEstBias;
+    __syncthreads();
+    for (int i = threadIdx.x; i < N; i += blockDim.x) {
+        const double2 b = t.bias[i];
+        t.bias[i] = make_double2(gp[d.bla + i] + lin * b.x, gp[d.bmu + i] + lin * b.y);
+    }
+    for (int k = threadIdx.x; k < 2 * N * SH; k += blockDim.x) {
+        const int h = k % SH, is = k / SH, i = is >> 1;
+        const double v = h < nh ? K * gp[((is & 1) ? d.wmu : d.wla) + h + nh * i] : 0.0;   // absent units: no change
+        if (small) {
+            const double h = 0.5 * v * odd_series(0.25 * v * v);   // sinh(v / 2)
+            t.real[k] = make_double2(2.0 * h * h, 2.0 * h * sqrt(fma(h, h, 1.0)));
+        } else {
+            t.real[k] = make_double2(exp(2.0 * v), exp(-2.0 * v));
+        }
+    }
+    for (int k = threadIdx.x; k < N * SP; k += blockDim.x) {
+        const int u = k % SP, i = k / SP;
+        const double vr = u < na ? K * gp[d.ula + u + na * i] : 0.0, vi = u < na ? K * gp[d.umu + u + na * i] : 0.0;
+        if (small) {
+            // v = (vr + i vi) / 2, h = sinh(v / 2), g = cosh(v / 2): cosh v - 1 = 2 h^2, sinh v = 2 h g
+            const double x = 0.25 * vr, y = 0.25 * vi;
+            const double s = y * odd_series(-y * y), c = even_series(-y * y);
+            const double sh = x * odd_series(x * x), ch = sqrt(fma(sh, sh, 1.0));
+            const double hr = sh * c, hi = ch * s, gr = ch * c, gi = sh * s;
+            t.pi[2 * k] = make_double2(2.0 * (hr * hr - hi * hi), 4.0 * hr * hi);
+            t.pi[2 * k + 1] = make_double2(2.0 * (hr * gr - hi * gi), 2.0 * (hr * gi + hi * gr));
+        } else {
+            double s, c;
+            sincos(vi, &s, &c);
+            const double e = exp(vr), r = exp(-vr);
+            t.pi[2 * k] = make_double2(e * c, e * s);
+            t.pi[2 * k + 1] = make_double2(r * c, -r * s);
+        }
+    }
+    __syncthreads();
+    return ok ? (small ? EST_DIFFERENCES : EST_FACTORS) : EST_SUMS;
+}
+// 1 / x for normal x of moderate size: v_rcp_f64 and two Newton steps (1 ulp)
+__device__ __forceinline__ double rcp_newton(double x) {
+    double r = __builtin_amdgcn_rcp(x);
+    r = fma(fma(-x, r, 1.0), r, r);
+    return fma(fma(-x, r, 1.0), r, r);
+}
+
+// (1 + p)(1 + q) - 1
+__device__ __forceinline__ double less_one(double p, double q) { return fma(p, q, p + q); }
+__device__ __forceinline__ cplx<double> less_one(cplx<double> p, cplx<double> q) {
+    return cmk(fma(p.re, q.re, fma(-p.im, q.im, p.re + q.re)), fma(p.re, q.im, fma(p.im, q.re, p.im + q.im)));
+}
+// c + a b
+__device__ __forceinline__ cplx<double> cfma(cplx<double> a, cplx<double> b, cplx<double> c) {
+    return cmk(fma(a.re, b.re, fma(-a.im, b.im, c.re)), fma(a.re, b.im, fma(a.im, b.re, c.im)));
 }
 
 // TAB_LDS: the connection table is staged in LDS (a compile-time choice, so
@@ -207,12 +280,12 @@ __device__ __forceinline__ void estimate_body(const est_args& a, int bx, int gx)
         if (threadIdx.x == 0) *poison = 0;
     }
     __syncthreads();
-    bool products = false;   // the connections by products of the units' factors
+    int form = EST_SUMS;     // of the connections
     const ratio_tables rt = ratio_at(smem + a.lds_param_bytes + fbytes, d);
     if constexpr (RATIO) {
         if (a.ratio) {
-            products = __builtin_amdgcn_readfirstlane(
-                           (int)ratio_fill<ACT>(rt, reinterpret_cast<const double*>(sp), d, 2 * RS, 2 * PS, tab.fmax)) != 0;
+            form = __builtin_amdgcn_readfirstlane(
+                ratio_fill<ACT>(rt, reinterpret_cast<const double*>(sp), d, 2 * RS, 2 * PS, tab.fmax));
         }
     }
 
@@ -520,21 +593,27 @@ __device__ __forceinline__ void estimate_body(const est_args& a, int bx, int gx)
                         Lacc = cadd(Lacc, W);
                     }
                 }
-            } else if (RATIO && products) {
+            } else if (RATIO && form != EST_SUMS) {
               if constexpr (RATIO) {
                 constexpr double K = ACT == NQ_ACT_LOGCOSH ? 2.0 : 1.0;
                 constexpr int TH = 2 * RS, TP = 2 * PS;   // tiles of 16 lambda (mu) and Pi units
+                constexpr int SH = 16 * TH, SP = 16 * TP;
                 const int il = lane & 15, kg = lane >> 4;
+                const bool diff = form == EST_DIFFERENCES;
+                // the sample's t or factors, one unit per lane, then in the tile layout (0: no such unit)
                 double es[RS], ee[RS];
 #pragma unroll
                 for (int r = 0; r < RS; ++r) {
-                    es[r] = exp(K * th_s[r]);
-                    ee[r] = exp(K * th_e[r]);
+                    if (diff) {
+                        es[r] = ACT == NQ_ACT_LOGCOSH ? a_s[r] : fma(2.0, a_s[r], -1.0);
+                        ee[r] = ACT == NQ_ACT_LOGCOSH ? a_e[r] : fma(2.0, a_e[r], -1.0);
+                    } else {
+                        es[r] = exp(K * th_s[r]);
+                        ee[r] = exp(K * th_e[r]);
+                    }
                 }
-                // the sample's factors in the tile layout (0: no such unit) and the lane's products
                 double ls[TH], le[TH], ms_[TH], me_[TH];
                 cplx<double> w[TP];
-                double qls = 1.0, qle = 1.0, qms = 1.0, qme = 1.0;
 #pragma unroll
                 for (int t = 0; t < TH; ++t) {
                     const int h = 16 * t + il, u = nh + h;
@@ -552,128 +631,242 @@ __device__ __forceinline__ void estimate_body(const est_args& a, int bx, int gx)
                     le[t] = in ? le[t] : 0.0;
                     ms_[t] = in ? ms_[t] : 0.0;
                     me_[t] = in ? me_[t] : 0.0;
-                    qls *= 1.0 + ls[t];
-                    qle *= 1.0 + le[t];
-                    qms *= 1.0 + ms_[t];
-                    qme *= 1.0 + me_[t];
                 }
-                const double ils = 1.0 / qls, ile = 1.0 / qle, ims = 1.0 / qms;
-                cplx<double> qp = cmk(1.0, 0.0);
                 {
-                    double sn, cs;
-                    sincos(K * pi_z[0].im, &sn, &cs);
-                    const double ex = exp(K * pi_z[0].re);
+                    cplx<double> w0 = pi_p[0];
+                    if (!diff) {
+                        double sn, cs;
+                        sincos(K * pi_z[0].im, &sn, &cs);
+                        const double ex = exp(K * pi_z[0].re);
+                        w0 = cmk(ex * cs, ex * sn);
+                    } else if constexpr (ACT == NQ_ACT_SOFTPLUS) {
+                        w0 = cmk(fma(2.0, w0.re, -1.0), 2.0 * w0.im);
+                    }
 #pragma unroll
                     for (int t = 0; t < TP; ++t) {
                         const int q = 16 * t + il;
-                        w[t] = cmk(__shfl(ex * cs, q & 63, 64), __shfl(ex * sn, q & 63, 64));
+                        w[t] = cmk(__shfl(w0.re, q & 63, 64), __shfl(w0.im, q & 63, 64));
                         if (q >= na) w[t] = cmk(0.0, 0.0);
-                        qp = cmul(qp, cmk(1.0 + w[t].re, w[t].im));
                     }
                 }
-                const double ipn = 1.0 / (qp.re * qp.re + qp.im * qp.im);
-                const cplx<double> ipc = cmk(qp.re * ipn, -qp.im * ipn);
-                const int hb = il < nh ? il : 0, ab = il < na ? il : 0;   // tables of absent units: any entry (0 times it)
+                // 64 connections' products, one per lane: lane i + 16 k takes round i's connection k
                 double kl = 1.0, km = 1.0;
                 cplx<double> kc = cmk(1.0, 0.0);
-                for (int c0 = 0, r = 0; c0 < ncc; c0 += 4, ++r) {
-                    uint32_t ms = 0u, me = 0u;
-                    if (c0 + kg < ncc) {
-                        const uint2 mm = mbuf[c0 + kg];
-                        ms = mm.x;
-                        me = mm.y;
-                    }
-                    double pl = 1.0, pm = 1.0;
-                    cplx<double> z[TP];
-#pragma unroll
-                    for (int t = 0; t < TP; ++t) z[t] = w[t];
-                    // one side's flips: the lambda and mu factors into fl, fm, the Pi units' into z
-                    auto side = [&](uint32_t m, uint32_t kk, double (&fl)[TH], double (&fm)[TH], double sgn) {
-                        for (; m; m &= m - 1) {
+                // finishes them from the moduli (squared, real units), mu product and Pi product
+                auto finish = [&](int r, double el, double lm, cplx<double> ec) {
+                    const int c = 4 * ((r & ~15) + il) + kg;
+                    if (c < ncc) {
+                        const uint2 mm = mbuf[c];
+                        double dre = 0.0, dim = 0.5 * lm;
+                        for (uint32_t m = mm.x; m; m &= m - 1) {
                             const int i = __builtin_ctz(m);
-                            const bool down = ((kk >> i) & 1u) != 0;
-                            const double* tb = (down ? rt.dn : rt.up) + 2 * i * nh + hb;
-                            const double2* tc = (down ? rt.pdn : rt.pup) + i * na + ab;
+                            const double cc = 0.5 * cflip<double>(ks, i);
+                            const double2 b = rt.bias[i];
+                            dre += cc * b.x;
+                            dim += cc * b.y;
+                        }
+                        for (uint32_t m = mm.y; m; m &= m - 1) {
+                            const int i = __builtin_ctz(m);
+                            const double cc = 0.5 * cflip<double>(ke, i);
+                            const double2 b = rt.bias[i];
+                            dre += cc * b.x;
+                            dim -= cc * b.y;
+                        }
+                        double sn, cs;
+                        sincos(dim, &sn, &cs);
+                        const double er = sqrt(el) * exp(dre);
+                        const cplx<double> W = cmul(cmul(wbuf[c], cmk(er * cs, er * sn)), ec);
+                        wbuf[c] = W;
+                        Lacc = cadd(Lacc, W);
+                    }
+                };
+                if (diff) {
+                    for (int c0 = 0, r = 0; c0 < ncc; c0 += 4, ++r) {
+                        uint32_t ms = 0u, me = 0u;
+                        if (c0 + kg < ncc) {
+                            const uint2 mm = mbuf[c0 + kg];
+                            ms = mm.x;
+                            me = mm.y;
+                        }
+                        double pl = 0.0, pm = 0.0;
+                        cplx<double> z[TP], sz[TP], pc = cmk(0.0, 0.0);
+#pragma unroll
+                        for (int t = 0; t < TP; ++t) z[t] = sz[t] = cmk(0.0, 0.0);
+                        bool zfirst = true;
+                        // one side's flips: (cosh - 1, sinh) of the angles' change relative to the sample's
+                        // cosh, (z, sz) for the Pi units, combined over this lane's units into ql, qm
+                        auto side = [&](uint32_t m, uint32_t kk, bool more, const double (&tl)[TH],
+                                        const double (&tm)[TH], double sgn, double& ql, double& qm) {
+                            double dl[TH], dm[TH], sl[TH], sm[TH];
+                            bool first = true;
+                            while (m) {
+                                const int i = __builtin_ctz(m);
+                                m &= m - 1;
+                                const double up = ((kk >> i) & 1u) ? -1.0 : 1.0;
+                                const double2* tb = rt.real + 2 * SH * i + il;
+                                const double2* tc = rt.pi + 2 * (SP * i + il);
+#pragma unroll
+                                for (int t = 0; t < TH; ++t)
+                                    if (16 * t < nh) {
+                                        const double2 a = tb[16 * t], b = tb[SH + 16 * t];
+                                        const double ay = up * a.y, by = up * b.y;
+                                        if (first) {
+                                            dl[t] = fma(tl[t], ay, a.x);
+                                            dm[t] = fma(tm[t], by, b.x);
+                                            if (m) {
+                                                sl[t] = fma(tl[t], a.x, tl[t] + ay);
+                                                sm[t] = fma(tm[t], b.x, tm[t] + by);
+                                            }
+                                        } else {
+                                            const double p = dl[t], q = dm[t];
+                                            dl[t] = fma(sl[t], ay, fma(p, a.x, p + a.x));
+                                            dm[t] = fma(sm[t], by, fma(q, b.x, q + b.x));
+                                            if (m) {
+                                                sl[t] = fma(p, ay, fma(sl[t], a.x, sl[t] + ay));
+                                                sm[t] = fma(q, by, fma(sm[t], b.x, sm[t] + by));
+                                            }
+                                        }
+                                    }
+#pragma unroll
+                                for (int t = 0; t < TP; ++t)
+                                    if (16 * t < na) {
+                                        const double2 a = tc[32 * t], b = tc[32 * t + 1];
+                                        const cplx<double> C = cmk(a.x, sgn * a.y), S = cmk(up * b.x, sgn * up * b.y);
+                                        if (zfirst) {
+                                            z[t] = cfma(w[t], S, C);
+                                            if (m || more) sz[t] = cfma(w[t], C, cadd(w[t], S));
+                                        } else {
+                                            const cplx<double> p = z[t];
+                                            z[t] = cfma(sz[t], S, less_one(p, C));
+                                            if (m || more) sz[t] = cfma(p, S, cfma(sz[t], C, cadd(sz[t], S)));
+                                        }
+                                    }
+                                first = zfirst = false;
+                            }
+                            ql = dl[0];
+                            qm = dm[0];
+#pragma unroll
+                            for (int t = 1; t < TH; ++t)
+                                if (16 * t < nh) {
+                                    ql = less_one(ql, dl[t]);
+                                    qm = less_one(qm, dm[t]);
+                                }
+                        };
+                        if (ms) side(ms, ks, me != 0u, ls, ms_, 1.0, pl, pm);
+                        if (me) {
+                            double ql, qm;
+                            side(me, ke, false, le, me_, -1.0, ql, qm);
+                            pl = less_one(pl, ql);
+                            pm = less_one(pm, -qm * rcp_newton(1.0 + qm));   // 1 / (1 + qm) - 1
+                        }
+#pragma unroll
+                        for (int t = 0; t < TP; ++t)
+                            if (16 * t < na) pc = t == 0 ? z[0] : less_one(pc, z[t]);
+                        // products over the connection's 16 lanes
+                        pl = less_one(pl, dpp_d<0xB1>(pl));
+                        pl = less_one(pl, dpp_d<0x4E>(pl));
+                        pl = less_one(pl, dpp_d<0x141>(pl));
+                        pl = less_one(pl, dpp_d<0x140>(pl));
+                        pm = less_one(pm, dpp_d<0xB1>(pm));
+                        pm = less_one(pm, dpp_d<0x4E>(pm));
+                        pm = less_one(pm, dpp_d<0x141>(pm));
+                        pm = less_one(pm, dpp_d<0x140>(pm));
+                        pc = less_one(pc, cmk(dpp_d<0xB1>(pc.re), dpp_d<0xB1>(pc.im)));
+                        pc = less_one(pc, cmk(dpp_d<0x4E>(pc.re), dpp_d<0x4E>(pc.im)));
+                        pc = less_one(pc, cmk(dpp_d<0x141>(pc.re), dpp_d<0x141>(pc.im)));
+                        pc = less_one(pc, cmk(dpp_d<0x140>(pc.re), dpp_d<0x140>(pc.im)));
+                        const bool mine = il == (r & 15);
+                        kl = mine ? pl : kl;
+                        km = mine ? pm : km;
+                        kc.re = mine ? pc.re : kc.re;
+                        kc.im = mine ? pc.im : kc.im;
+                        if ((r & 15) == 15 || c0 + 4 >= ncc) finish(r, 1.0 + kl, log1p(km), cmk(1.0 + kc.re, kc.im));
+                    }
+                } else {
+                    double qls = 1.0, qle = 1.0, qms = 1.0, qme = 1.0;
+#pragma unroll
+                    for (int t = 0; t < TH; ++t) {
+                        qls *= 1.0 + ls[t];
+                        qle *= 1.0 + le[t];
+                        qms *= 1.0 + ms_[t];
+                        qme *= 1.0 + me_[t];
+                    }
+                    const double ils = 1.0 / qls, ile = 1.0 / qle, ims = 1.0 / qms;
+                    cplx<double> qp = cmk(1.0, 0.0);
+#pragma unroll
+                    for (int t = 0; t < TP; ++t) qp = cmul(qp, cmk(1.0 + w[t].re, w[t].im));
+                    const double ipn = 1.0 / (qp.re * qp.re + qp.im * qp.im);
+                    const cplx<double> ipc = cmk(qp.re * ipn, -qp.im * ipn);
+                    for (int c0 = 0, r = 0; c0 < ncc; c0 += 4, ++r) {
+                        uint32_t ms = 0u, me = 0u;
+                        if (c0 + kg < ncc) {
+                            const uint2 mm = mbuf[c0 + kg];
+                            ms = mm.x;
+                            me = mm.y;
+                        }
+                        double pl = 1.0, pm = 1.0;
+                        cplx<double> z[TP];
+#pragma unroll
+                        for (int t = 0; t < TP; ++t) z[t] = w[t];
+                        // one side's flips: the lambda and mu factors into fl, fm, the Pi units' into z
+                        auto side = [&](uint32_t m, uint32_t kk, double (&fl)[TH], double (&fm)[TH], double sgn) {
+                            for (; m; m &= m - 1) {
+                                const int i = __builtin_ctz(m);
+                                const int down = (kk >> i) & 1u;
+                                const double* tb = reinterpret_cast<const double*>(rt.real + 2 * SH * i + il) + down;
+                                const double2* tc = rt.pi + 2 * (SP * i + il) + down;
+#pragma unroll
+                                for (int t = 0; t < TH; ++t)
+                                    if (16 * t < nh) {
+                                        fl[t] *= tb[32 * t];
+                                        fm[t] *= tb[2 * SH + 32 * t];
+                                    }
+#pragma unroll
+                                for (int t = 0; t < TP; ++t)
+                                    if (16 * t < na) {
+                                        const double2 f = tc[32 * t];
+                                        z[t] = cmul(z[t], cmk(f.x, sgn * f.y));
+                                    }
+                            }
+                        };
+                        if (ms) {
+                            double fl[TH], fm[TH], ql = ils, qm = ims;
+#pragma unroll
+                            for (int t = 0; t < TH; ++t) { fl[t] = ls[t]; fm[t] = ms_[t]; }
+                            side(ms, ks, fl, fm, 1.0);
 #pragma unroll
                             for (int t = 0; t < TH; ++t)
-                                if (16 * t < nh) {
-                                    const int o = 16 * t + hb < nh ? 16 * t : 0;
-                                    fl[t] *= tb[o];
-                                    fm[t] *= tb[o + nh];
-                                }
-#pragma unroll
-                            for (int t = 0; t < TP; ++t)
-                                if (16 * t < na) {
-                                    const double2 f = tc[16 * t + ab < na ? 16 * t : 0];
-                                    z[t] = cmul(z[t], cmk(f.x, sgn * f.y));
-                                }
+                                if (16 * t < nh) { ql *= 1.0 + fl[t]; qm *= 1.0 + fm[t]; }
+                            pl = ql;
+                            pm = qm;
                         }
-                    };
-                    if (ms) {
-                        double fl[TH], fm[TH], ql = ils, qm = ims;
+                        if (me) {
+                            double fl[TH], fm[TH], ql = ile, qm = 1.0;
 #pragma unroll
-                        for (int t = 0; t < TH; ++t) { fl[t] = ls[t]; fm[t] = ms_[t]; }
-                        side(ms, ks, fl, fm, 1.0);
+                            for (int t = 0; t < TH; ++t) { fl[t] = le[t]; fm[t] = me_[t]; }
+                            side(me, ke, fl, fm, -1.0);
 #pragma unroll
-                        for (int t = 0; t < TH; ++t)
-                            if (16 * t < nh) { ql *= 1.0 + fl[t]; qm *= 1.0 + fm[t]; }
-                        pl = ql;
-                        pm = qm;
-                    }
-                    if (me) {
-                        double fl[TH], fm[TH], ql = ile, qm = 1.0;
-#pragma unroll
-                        for (int t = 0; t < TH; ++t) { fl[t] = le[t]; fm[t] = me_[t]; }
-                        side(me, ke, fl, fm, -1.0);
-#pragma unroll
-                        for (int t = 0; t < TH; ++t)
-                            if (16 * t < nh) { ql *= 1.0 + fl[t]; qm *= 1.0 + fm[t]; }
-                        pl *= ql;
-                        pm *= qme / qm;
-                    }
-                    cplx<double> pc = ipc;
-#pragma unroll
-                    for (int t = 0; t < TP; ++t)
-                        if (16 * t < na) pc = cmul(pc, cmk(1.0 + z[t].re, z[t].im));
-                    // products over the connection's 16 lanes
-                    pl = group_product<16>(pl);
-                    pm = group_product<16>(pm);
-                    pc = cmul(pc, cmk(dpp_d<0xB1>(pc.re), dpp_d<0xB1>(pc.im)));
-                    pc = cmul(pc, cmk(dpp_d<0x4E>(pc.re), dpp_d<0x4E>(pc.im)));
-                    pc = cmul(pc, cmk(dpp_d<0x141>(pc.re), dpp_d<0x141>(pc.im)));
-                    pc = cmul(pc, cmk(dpp_d<0x140>(pc.re), dpp_d<0x140>(pc.im)));
-                    // lane i + 16 k keeps round i's connection k; after 16 rounds every lane finishes its own
-                    const bool mine = il == (r & 15);
-                    kl = mine ? pl : kl;
-                    km = mine ? pm : km;
-                    kc.re = mine ? pc.re : kc.re;
-                    kc.im = mine ? pc.im : kc.im;
-                    if ((r & 15) == 15 || c0 + 4 >= ncc) {
-                        const int c = 4 * ((r & ~15) + il) + kg;
-                        if (c < ncc) {
-                            const uint2 mm = mbuf[c];
-                            double dre = 0.0, dim = 0.5 * log(km);
-                            for (uint32_t m = mm.x; m; m &= m - 1) {
-                                const int i = __builtin_ctz(m);
-                                const double cc = 0.5 * cflip<double>(ks, i);
-                                const double2 b = rt.bias[i];
-                                dre += cc * b.x;
-                                dim += cc * b.y;
-                            }
-                            for (uint32_t m = mm.y; m; m &= m - 1) {
-                                const int i = __builtin_ctz(m);
-                                const double cc = 0.5 * cflip<double>(ke, i);
-                                const double2 b = rt.bias[i];
-                                dre += cc * b.x;
-                                dim -= cc * b.y;
-                            }
-                            double sn, cs;
-                            sincos(dim, &sn, &cs);
-                            const double er = sqrt(kl) * exp(dre);
-                            const cplx<double> W = cmul(cmul(wbuf[c], cmk(er * cs, er * sn)), kc);
-                            wbuf[c] = W;
-                            Lacc = cadd(Lacc, W);
+                            for (int t = 0; t < TH; ++t)
+                                if (16 * t < nh) { ql *= 1.0 + fl[t]; qm *= 1.0 + fm[t]; }
+                            pl *= ql;
+                            pm *= qme / qm;
                         }
+                        cplx<double> pc = ipc;
+#pragma unroll
+                        for (int t = 0; t < TP; ++t)
+                            if (16 * t < na) pc = cmul(pc, cmk(1.0 + z[t].re, z[t].im));
+                        pl = group_product<16>(pl);
+                        pm = group_product<16>(pm);
+                        pc = cmul(pc, cmk(dpp_d<0xB1>(pc.re), dpp_d<0xB1>(pc.im)));
+                        pc = cmul(pc, cmk(dpp_d<0x4E>(pc.re), dpp_d<0x4E>(pc.im)));
+                        pc = cmul(pc, cmk(dpp_d<0x141>(pc.re), dpp_d<0x141>(pc.im)));
+                        pc = cmul(pc, cmk(dpp_d<0x140>(pc.re), dpp_d<0x140>(pc.im)));
+                        const bool mine = il == (r & 15);
+                        kl = mine ? pl : kl;
+                        km = mine ? pm : km;
+                        kc.re = mine ? pc.re : kc.re;
+                        kc.im = mine ? pc.im : kc.im;
+                        if ((r & 15) == 15 || c0 + 4 >= ncc) finish(r, kl, log(km), kc);
                     }
                 }
               }
@@ -1446,7 +1639,9 @@ __global__ __launch_bounds__(512, CLS < 2 ? 4 : 2) void k_force_mma_pk(const nq_
 // connections 12 products of 64 cycles against about 170 VALU instructions, on different pipes.  The
 // form it replaces, one unit per lane with the flipped site indexing a register vector and exp, sincos
 // and divides per unit, took 0.97 ms alone on 4x4 XYZ with 16384 samples (2.2 beside the S build);
-// this one 0.36 (12 sites, beside: 0.6 -> 0.16).
+// this one 0.36 (12 sites, beside: 0.6 -> 0.16).  The force is as far from an 80-bit evaluation as it
+// was by that form (4096 samples, 1e-16: 6 sites 4.9 -> 4.1, 12 sites 5.7 -> 6.9, 3x3 XYZ 5.1 -> 4.5; up
+// to eight samples summed before the exact accumulator change that by less than one in ten).
 //   LDS: HW [N + 1][SW], PU [N][SP], PD [SP] as above in double, then up, dn [N][SW], pup, pdn [N][SP]
 typedef double d4v __attribute__((ext_vector_type(4)));
 
@@ -1455,13 +1650,6 @@ __host__ __device__ inline int force64_stage_doubles(const ndm_dims& d, bool rat
     const int c = force_class(d) < 0 ? 2 : force_class(d);
     const int sw = 32 << c, sp = 16 << c;
     return sw * (d.N + 1) + sp * (2 * d.N + 1) + (ratio ? 2 * d.N * (sw + 2 * sp) : 0);
-}
-
-// 1 / x for normal x of moderate size: v_rcp_f64 and two Newton steps (1 ulp)
-__device__ __forceinline__ double rcp_newton(double x) {
-    double r = __builtin_amdgcn_rcp(x);
-    r = fma(fma(-x, r, 1.0), r, r);
-    return fma(fma(-x, r, 1.0), r, r);
 }
 
 template <int NMAX, int CLS, int ACT, bool RATIO>
@@ -1742,9 +1930,8 @@ __device__ __forceinline__ void force64_body(const est_args& a, int bx, int gx) 
         const double w = u < 2 * nh ? gp[src] : 0.0;
         HW[k] = w;
         if (a.ratio && r > 0) {
-            const double e = exp(2.0 * K * w);
-            up[k - SW] = e;
-            dn[k - SW] = 1.0 / e;
+            up[k - SW] = exp(2.0 * K * w);
+            dn[k - SW] = exp(-2.0 * K * w);
         }
     }
     for (int k = threadIdx.x; k < SP * N; k += blockDim.x) {
@@ -1755,7 +1942,7 @@ __device__ __forceinline__ void force64_body(const est_args& a, int bx, int gx) 
         if (a.ratio) {
             double sn, cs;
             sincos(K * um, &sn, &cs);
-            const double e = exp(K * ul), r = 1.0 / e;
+            const double e = exp(K * ul), r = exp(-K * ul);
             pup[k] = make_double2(e * cs, e * sn);
             pdn[k] = make_double2(r * cs, -r * sn);
         }
