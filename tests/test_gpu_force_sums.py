@@ -1,7 +1,8 @@
-"""The FP64 forces' exact sums and records at the ends of their range:
-entries whose samples stay below the accumulator's bound of 2^30 although
-eight of them together do not, and connection tables whose records fit in LDS
-only beside fewer waves."""
+"""The FP64 forces at the ends of their range: entries whose samples stay
+below the accumulator's bound of 2^30 although eight of them together do not,
+connection tables whose records fit in LDS only beside fewer waves, and f' at
+the angles themselves, where the factor tables do not fit in LDS or a unit
+leaves their range."""
 import dataclasses
 
 import numpy as np
@@ -68,3 +69,21 @@ def test_long_records(gpu_ok):
         ctx.close()
     assert rel_err(out[1][0], k * out[0][0]) < 1e-12
     assert rel_err(out[1][1], k * k * out[0][1]) < 1e-12
+
+
+# 16 sites with 64 units of each kind: the tables alone take 98 KB beside an accumulator of 68; and a
+# hidden bias of 320 (softplus) on a unit of small weights
+@pytest.mark.parametrize("N,nh,na,sigma,bias", [(16, 64, 64, 0.03, 0.0), (3, 5, 4, 0.1, 320.0)])
+def test_forces_at_the_angles(gpu_ok, ref, N, nh, na, sigma, bias):
+    flat, tab, _ = ising(N)
+    p = params(ref.ndm_np(N, nh, na), seed=7, sigma=sigma)
+    p[nqref.ndm_layout(N, nh, na)[0]["h_la"][0] + 1] += bias
+    keys = random_keys(N, 24, seed=8)
+    ctx = context(flat, N, nh, na, p)
+    st, _, F, _ = ctx.grad_from_samples(keys, 12, 2)
+    L_r, dL_r = ref.local_estimator(tab, nh, na, p, keys)
+    _, O_r = ref.logpsi_grad(N, nh, na, p, keys)
+    _, F_r, _, st_r = ref.grad_step(12, 2, O_r, L_r, dL_r)
+    assert rel_err(st, st_r) < 1e-10
+    assert rel_err(F, F_r) < 1e-10
+    ctx.close()

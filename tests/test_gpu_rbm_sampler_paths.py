@@ -1,5 +1,5 @@
 """The complex RBMs' FP64 sampler: chains by products of the units' factors
-(groups of 8, 16, 32 and 64 lanes, one and two units per lane, few chains with
+(groups of 8, 16, 32 and 64 lanes, one to four units per lane, few chains with
 copies of a group, many chains) and, where the weights leave their range, by
 sums of f, against the oracle's trajectories bit for bit."""
 import numpy as np
@@ -13,7 +13,9 @@ pytestmark = pytest.mark.gpu
 
 # sigma 2 at 70 units leaves the range (sum over the units of (2 N + 1) 0.8 sigma + 1.4 > 600)
 SHAPES = [(2, 1, 0.3, 3), (3, 9, 0.3, 5), (2, 17, 0.3, 4), (2, 33, 0.2, 4), (2, 70, 0.1, 3), (2, 128, 0.05, 2),
-          (2, 18, 0.3, 2060), (2, 70, 2.0, 3)]
+          (2, 18, 0.3, 2060), (2, 70, 2.0, 3),
+          # four units per lane, full and ragged (groups of 8, 16 and 32), and the largest tables (132 KB of LDS)
+          (2, 32, 0.2, 4100), (2, 40, 0.2, 2060), (2, 70, 0.1, 1100), (16, 128, 0.02, 3)]
 
 
 @pytest.mark.parametrize("ket", [False, True])
