@@ -208,8 +208,8 @@ nqh_status nqh_precondition(nqh_ctx* ctx, double eps, int32_t shift_kind, int32_
  *   NQH_SOLVER_CG        sr_cg through SRIterative.jl:71-152 with the
  *                        matrix-free S of SrMatrixR (SR_notfull.jl:84-148):
  *                        S is never formed (no Np^2 memory); conjugate
- *                        gradients on S v = Re(Oc^H Oc v)/Ns + shift, two
- *                        passes over the O rows per product, until
+ *                        gradients on S v = Re(Oc^H Oc v)/Ns + shift, one
+ *                        pass over the O rows per product, until
  *                        ||r|| <= tol ||F|| or maxiter products (0: 10 Np,
  *                        the reference's limit); without convergence the
  *                        step is zero (SRIterative.jl:134-150).  NDM networks

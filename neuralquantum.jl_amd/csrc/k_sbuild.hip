@@ -564,11 +564,12 @@ hipError_t nq_launch_center_t(const void* Y, int y_fp64, int64_t Ns, int ldy, in
 // shape), otherwise about three tiles in flight per CU.  FP64 / FP32 (64 x 64 tiles): a multiple of
 // eight chunks, one XCD each, at least three workgroups per CU.  The partial sums stay within twice
 // the input, so that small problems (many of them sharing the device) do not turn into partial-sum
-// traffic; at least 64 samples per chunk, at most 64 chunks.
+// traffic (0.7 GB at the most, FP64 with 16 sites and 64 units of each kind); at least 64 samples per
+// chunk, at most 64 chunks.
 // One workgroup per tile over all samples, one launch per block -> chunks (time of both blocks):
 // FP64 4x4 XYZ (702 tiles, 16384 samples) 3.3 -> 2.4 ms beside the forces launch; 12 sites (240 tiles)
 // 4.1 -> 0.75 ms beside it; ket RBM of 16 sites (171 tiles, 8192 samples) alone 0.59 -> 0.24 ms, 49
-// TFLOP/s; FP32 12 sites 2.26 -> 0.41 ms; 6 sites (6 tiles, 2000 samples) 294 -> 12 us.  Twice and four
+// TFLOP/s; FP32 12 sites 2.26 -> 0.42 ms; 6 sites (6 tiles, 2000 samples) 294 -> 12 us.  Twice and four
 // times the chunks changed none of these by more than 5 % and made the sum over them longer.
 nq_gram_plan nq_plan_gram(int mode, int nA, int nB, int64_t Ns, int max_splits) {
     nq_gram_plan g{};

@@ -221,8 +221,7 @@ hipError_t nq_launch_update(double* p64, float* p32, const double* delta, ndm_di
 hipError_t nq_split_tail(int nl, int npi, const double* x2, double* delta, int* flag, double* p64, float* p32,
                          const ndm_dims& d, double lr, const int* info, const double* stats, double* out,
                          hipStream_t st);
-// FP32 copy of the parameters
-// parameters from / into pinned host memory; *done = seq when the transfer is complete
+// parameters from / into pinned host memory (from: with their FP32 copy); *done = seq when the transfer is complete
 hipError_t nq_launch_params_in(const double* host, double* p64, float* p32, int n, double* done, double seq,
                                hipStream_t st);
 hipError_t nq_launch_params_out(const double* p64, double* host, int n, double* done, double seq, hipStream_t st);
